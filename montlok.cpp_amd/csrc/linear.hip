@@ -28,7 +28,10 @@
 //
 // Shapes with fewer 128-row blocks x 64-column chunks than CUs (a few
 // thousand rows) take linear_small_kernel instead: one wave per 16 x 16
-// output tile, operands straight from L2, no LDS.
+// output tile, operands straight from L2, no LDS; with few tiles and K beyond
+// 256, linear_small_split_kernel, four waves per tile. fp32 weights with K
+// above 128 otherwise take linear_split.hip's three-plane bf16 form; the fp32
+// forms here then serve K up to 128 and operands that are not 16-byte aligned.
 //
 // K is reduced in an order of its own (the 8 k of a lane, then the four lane
 // groups inside the MFMA); for fp32 weights the result differs from a
@@ -38,6 +41,7 @@
 #include <type_traits>
 #include <cstring>
 
+#include "linear_args.h"
 #include "mlk_common.h"
 #include "tile_f32.h"
 
@@ -71,24 +75,6 @@ struct WTraits<false> {
     using T = float;
     static constexpr int kKChunk = 128;
     static constexpr int kPitch = kKChunk + 4;
-};
-
-struct LinearArgs {
-    const float* x;
-    int64_t rows, K, x_stride;
-    const void* w;
-    const float* bias;
-    int64_t N;
-    float* out;
-    int64_t out_stride;
-    // Optional residual added to the result (out = residual + (x W^T + b),
-    // the add as a separate fp32 rounding), rows res_stride apart.
-    const float* residual;
-    int64_t res_stride;
-    // Optional grouped RMSNorm of x before the product (linear_small_kernel
-    // only): weight and eps as the rms_norm operator takes them.
-    const float* norm_w;
-    double norm_eps;
 };
 
 // Loads 8 consecutive floats x[row, k .. k+7] (zero past K or past the last
@@ -637,6 +623,86 @@ void launch_small_norm(const LinearArgs& p, int64_t tiles, hipStream_t stream) {
         launch_small<BF16W, 4, GS>(p, tiles, stream);
     } else {
         launch_small<BF16W, 8, GS>(p, tiles, stream);
+    }
+}
+
+// The one-tile form for 256 < K <= 128 KS: four waves share a 16 x 16 output
+// tile, each the products of a quarter of K (whole 32-wide steps), whose sums
+// meet in LDS. A few hundred rows leave the tiled forms a handful of blocks
+// that walk K alone; here the longest chain is a quarter of K.
+template <bool BF16W, int KS>
+__global__ __launch_bounds__(256) void linear_small_split_kernel(LinearArgs p) {
+    __shared__ f32x4 part[3][64];
+    const int lane = threadIdx.x & 63, li = lane & 15, group = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t n_tiles = (p.N + 15) / 16;
+    unsigned lin = blockIdx.x;  // (tile order as in linear_small_kernel)
+    if (gridDim.x % 8 == 0) lin = (lin % 8) * (gridDim.x / 8) + lin / 8;
+    const int64_t row0 = static_cast<int64_t>(lin / n_tiles) * 16;
+    const int64_t n0 = static_cast<int64_t>(lin % n_tiles) * 16;
+    const int64_t xr = row0 + li < p.rows ? row0 + li : p.rows - 1;
+    const int64_t wr = n0 + li < p.N ? n0 + li : p.N - 1;
+    const int K = static_cast<int>(p.K);
+    const int quarter = (K + 127) / 128 * 32;
+    const int k0 = wave * quarter < K ? wave * quarter : 0;
+    const int span = wave * quarter < K ? (K - k0 < quarter ? K - k0 : quarter) : 0;
+    float xv[KS][8];
+    bool live[KS];
+    tile_load8<KS>(p.x + xr * p.x_stride + k0, span, group, xv, live);
+    f32x4 y;
+    if constexpr (BF16W) {
+        const u16* wrow = static_cast<const u16*>(p.w) + wr * p.K + k0;
+        uint4 wv[KS];
+#pragma unroll
+        for (int s = 0; s < KS; ++s) wv[s] = *reinterpret_cast<const uint4*>(wrow + (live[s] ? 32 * s + 8 * group : 0));
+        y = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int s = 0; s < KS; ++s) {
+            bf16x8 a;
+            const bf16x8 b = __builtin_bit_cast(bf16x8, live[s] ? wv[s] : uint4{0u, 0u, 0u, 0u});
+#pragma unroll
+            for (int j = 0; j < 8; ++j) a[j] = static_cast<__bf16>(live[s] ? xv[s][j] : 0.0f);
+            y = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b, a, y, 0, 0, 0);
+        }
+    } else {
+        float wv[KS][8];
+        bool wlive[KS];
+        tile_load8<KS>(static_cast<const float*>(p.w) + wr * p.K + k0, span, group, wv, wlive);
+        y = tile_mfma_f32<KS>(wv, xv, live);
+    }
+    if (wave > 0) part[wave - 1][lane] = y;
+    __syncthreads();
+    if (wave > 0) return;
+    y = (y + part[0][lane]) + (part[1][lane] + part[2][lane]);
+    const int64_t row = row0 + li;
+    if (row >= p.rows) return;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+        const int64_t col = n0 + 4 * group + v;
+        if (p.bias != nullptr) y[v] += p.bias[col < p.N ? col : p.N - 1];
+    }
+    float* dst = p.out + row * p.out_stride + n0 + 4 * group;
+    const float* res = p.residual != nullptr ? p.residual + row * p.res_stride + n0 + 4 * group : nullptr;
+    const bool vec_out = (reinterpret_cast<uintptr_t>(p.out) & 15) == 0 && p.out_stride % 4 == 0 && n0 + 16 <= p.N &&
+                         (res == nullptr ||
+                          ((reinterpret_cast<uintptr_t>(p.residual) & 15) == 0 && p.res_stride % 4 == 0));
+    if (vec_out) {
+        if (res != nullptr) y = *reinterpret_cast<const f32x4*>(res) + y;
+        *reinterpret_cast<f32x4*>(dst) = y;
+    } else {
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            if (n0 + 4 * group + v < p.N) dst[v] = res != nullptr ? res[v] + y[v] : y[v];
+        }
+    }
+}
+
+template <bool BF16W>
+void launch_small_split(const LinearArgs& p, int64_t tiles, hipStream_t stream) {
+    if (p.K <= 512) {
+        hipLaunchKernelGGL((linear_small_split_kernel<BF16W, 4>), dim3(static_cast<unsigned>(tiles)), dim3(256), 0, stream, p);
+    } else {
+        hipLaunchKernelGGL((linear_small_split_kernel<BF16W, 8>), dim3(static_cast<unsigned>(tiles)), dim3(256), 0, stream, p);
     }
 }
 
@@ -1296,6 +1362,23 @@ bool small_shape(int64_t rows, int64_t K, int64_t N) {
            ceil_div(rows, 16) * ceil_div(N, 16) <= 0x7fffffff;
 }
 
+int64_t tiles16(int64_t rows, int64_t N) { return ceil_div(rows, 16) * ceil_div(N, 16); }
+
+// fp32 weights with K above 128 go to the three-plane form (linear_split.hip) unless so few 16 x 16 tiles are
+// asked for that one wave per tile ends sooner: its blocks walk K alone, 8 us at K = 256 however few they are,
+// and the one-wave form takes 4.0 us for 300 tiles, 7.6 for 1320 and 9.4 for 1920 (12.1 for 2640). Up to K = 128
+// the forms here are kept (the row-layout form has rms_norm_linear's prologue there).
+bool split_shape(const LinearArgs& p) {
+    return p.K > 128 && !(small_shape(p.rows, p.K, p.N) && tiles16(p.rows, p.N) <= 1536) && linear_split_fits(p);
+}
+
+// Four waves a tile for K in (256, 1024] (linear_small_split_kernel): 31 us -> 6.2 at 480 x 512 -> 256 in fp32
+// and 12.8 -> 5.3 with bf16 weights, 59 -> 9.8 at 480 x 1024 -> 256. Its time grows with the tiles and passes
+// the three-plane form's 14 us at 1450 of them (K = 512; 1250 at K = 264, bf16 against the tiled form 1750).
+bool small_split_shape(const LinearArgs& p) {
+    return p.K > 256 && p.K <= 1024 && p.K % 8 == 0 && tiles16(p.rows, p.N) <= 1280;
+}
+
 // MLK_LINEAR_FORM=t32 keeps linear_t32_kernel for the shapes the streaming form takes (read at each
 // call, so a caller can compare the two forms).
 bool stream_form() {
@@ -1334,7 +1417,15 @@ void launch(const LinearArgs& p, int64_t rows, int64_t n_chunks, hipStream_t str
     // Shapes too small to give the 128-row blocks one per CU (256 CUs) take
     // one wave per 16 x 16 tile (2048 x 128 -> 64: 16 blocks of the tiled
     // form, 512 waves here).
-    const int64_t tiles = ceil_div(rows, 16) * ceil_div(p.N, 16);
+    const int64_t tiles = tiles16(rows, p.N);
+    if (VEC && small_split_shape(p)) {
+        launch_small_split<BF16W>(p, tiles, stream);
+        return;
+    }
+    if (VEC && !BF16W && split_shape(p)) {
+        launch_linear_split(p, stream);
+        return;
+    }
     if (VEC && small_shape(rows, p.K, p.N)) {
         if (p.K <= 64) {
             launch_small<BF16W, 2>(p, tiles, stream);
@@ -1540,7 +1631,12 @@ extern "C" mlk_status mlk_rms_norm_linear(const float* x, int64_t rows, int64_t 
 #undef MLK_ROWS_GS
         return launch_status("rms_norm_linear");
     }
-    const int64_t tiles = ceil_div(rows, 16) * ceil_div(out_features, 16);
+    // Where linear takes the three-plane form, so does this (at most 256 of K: a small shape).
+    if (weight_dtype == MLK_DTYPE_F32 && split_shape(p)) {
+        launch_linear_split_norm(p, gs, s);
+        return launch_status("rms_norm_linear");
+    }
+    const int64_t tiles = tiles16(rows, out_features);
 #define MLK_NORM_GS(G)                                                                             \
     (weight_dtype == MLK_DTYPE_BF16 ? launch_small_norm<true, G>(p, tiles, s) : launch_small_norm<false, G>(p, tiles, s))
     switch (gs) {

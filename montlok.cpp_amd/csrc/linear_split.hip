@@ -1,0 +1,296 @@
+// Dense linear y = x W^T (+ bias, + residual) with fp32 weights on the bf16
+// matrix cores, to fp32 accuracy.
+//
+// An fp32 value is the exact sum of three bf16 values (8 + 8 + 8 bits of its
+// 24-bit significand; each part is the rounding of what the ones before it
+// left, so their magnitudes fall by 2^-9 a step), so
+//
+//   x w = x1 w1 + (x1 w2 + x2 w1) + (x1 w3 + x2 w2 + x3 w1) + O(2^-26 x w)
+//
+// and six v_mfma_f32_32x32x16_bf16 form, with every product exact and fp32
+// accumulation, what the fp32 form needs sixteen v_mfma_f32_32x32x2_f32 for,
+// at a sixth of the matrix-core time (2.2 PFLOP/s bf16 and 155 TFLOP/s fp32
+// measured on this chip). The first term and the other five are summed apart
+// and added at the end: the large sum then takes one rounding per 16 k, and
+// the error against float64 is 8.5e-8 (2-norm, N(0, 1) x, K = 256; 1.2e-7 at
+// K = 512) where the fp32 forms it replaces have 2.9e-7 (4.1e-7).
+//
+//   block  = 64 rows x 64 columns of y, 4 waves of 32 x 32; K in steps of 32.
+//   stage  = 16-row pieces of x and W, whole 128-byte lines per load (the
+//            MFMA operand order straight from memory takes every line in four
+//            separate instructions: 20-25% slower), split in registers and
+//            written as three bf16 planes in LDS, in the operand order.
+//   D      = transposed products (W as the A operand): lane (g, l) of a wave
+//            holds row l, columns 8 j + 4 g .. + 3 (j = 0..3), 16-byte stores.
+//
+// What bounds it: per step and SIMD the matrix cores take 220 cycles and the
+// splits about 200 issue cycles; both run at 48% of the time with five blocks
+// a CU (27 KiB of LDS, 68 registers) in different phases. One LDS buffer and
+// two barriers: a second buffer, or 64 x 128 and 128 x 128 blocks, which split
+// less often, leave fewer waves to overlap and were not faster below 65,536
+// rows (7680 x 256 -> 1192: 36 us against 38 and 48; 65536 x 512 -> 256: 115
+// against 107 and 101). Measured against the fp32 forms: 7680 x 256 -> 1192
+// 69 -> 36 us, 7680 x 512 -> 256 34 -> 18, 15360 x 256 -> 1192 112 -> 68.
+//
+// Parts of an infinity or of a value that rounds to bf16 infinity are
+// inf and -inf (or NaN), so a result that involves one is NaN; such results
+// (and any other NaN) are formed again as a plain fp32 sum, which is infinite
+// or NaN where the fp32 product is.
+
+#include "linear_args.h"
+#include "mlk_common.h"
+
+namespace mlk {
+namespace {
+
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+
+constexpr int kPlanes = 3, kStep = 32, kBlock = 64;
+constexpr int kMaxNormGroups = 32;  // RMSNorm groups of a row (K = 256 in groups of 8)
+
+// 16-byte units of the LDS image of a 32-row x 32-k tile: [k half][plane][lane group][32 rows]. The groups are
+// 576 bytes apart, so that the eight lanes that write one row's two halves and groups hit different banks.
+constexpr int kGroupUnits = 36, kTileUnits = 2 * kPlanes * 2 * kGroupUnits;
+__device__ __forceinline__ unsigned unit(int tile, int half, int plane, int group) {
+    return tile * kTileUnits + ((half * kPlanes + plane) * 2 + group) * kGroupUnits;
+}
+
+// Two floats to one plane's packed bf16 pair; v keeps what the pair leaves.
+__device__ __forceinline__ uint32_t take_bf16(f32x2& v) {
+    const uint32_t u = __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2));
+    v[0] -= __builtin_bit_cast(float, u << 16);
+    v[1] -= __builtin_bit_cast(float, u & 0xffff0000u);
+    return u;
+}
+
+// rms_norm's scale of each (row, group) of the block's 64 rows: per 4 floats (a^2 + b^2) + (c^2 + d^2) in fp64,
+// the chunks of a group combined highest index bit first, as tile_rms_norm and rms_norm_vec_kernel do.
+template <int GS>
+__device__ __forceinline__ void norm_scales(const LinearArgs& p, int64_t row0, int groups, double* scale) {
+    for (int u = threadIdx.x; u < kBlock * groups; u += 256) {
+        const int64_t row = row0 + u / groups;
+        const float* x = p.x + (row < p.rows ? row : p.rows - 1) * p.x_stride + (u % groups) * GS;
+        double part[GS / 4];
+#pragma unroll
+        for (int c = 0; c < GS / 4; ++c) {
+            const float4 f = *reinterpret_cast<const float4*>(x + 4 * c);
+            const double a = f.x, b = f.y, e = f.z, d = f.w;
+            part[c] = (a * a + b * b) + (e * e + d * d);
+        }
+#pragma unroll
+        for (int n = GS / 8; n >= 1; n /= 2)
+#pragma unroll
+            for (int c = 0; c < n; ++c) part[c] += part[c + n];
+        scale[u] = 1.0 / sqrt(part[0] / static_cast<double>(GS) + p.norm_eps);
+    }
+}
+
+// FULL: K a multiple of the step. GS > 0: the grouped RMSNorm of x (groups of GS floats, at most kMaxNormGroups
+// of them) applied to the staged values, bit for bit rms_norm then this kernel. SWIGLU: W holds 2 N rows, gate
+// then up; a wave's W tile is 16 gate rows and the 16 up rows of the same columns, so that a lane holds both
+// of its outputs' factors, and out = silu(gate) * up in fp64, rounded once (p.N = hidden columns of out).
+template <bool FULL, int GS, bool SWIGLU>
+__global__ __launch_bounds__(256) void linear_split_kernel(LinearArgs p, unsigned n_blocks) {
+    constexpr int kCols = SWIGLU ? kBlock / 2 : kBlock;  // output columns of the block
+    __shared__ uint4 frag[4 * kTileUnits];               // x tiles 0, 1, W tiles 2, 3
+    __shared__ double scale[GS > 0 ? kBlock * kMaxNormGroups : 1];
+    const int lane = threadIdx.x & 63, li = lane & 31, g = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    // XCD x takes the x-th eighth of the blocks, column blocks of one row block side by side: a row block's x
+    // is fetched into one L2.
+    unsigned lin = blockIdx.x;
+    if (gridDim.x % 8 == 0) lin = (lin % 8) * (gridDim.x / 8) + lin / 8;
+    const int64_t row0 = static_cast<int64_t>(lin / n_blocks) * kBlock;
+    const int64_t n0 = static_cast<int64_t>(lin % n_blocks) * kCols;
+    const int K = static_cast<int>(p.K);
+    const int groups = GS > 0 ? K / GS : 0;
+    const float* w = static_cast<const float*>(p.w);
+
+    // Wave w stages rows 16 w .. + 15 of x and of W: lane 8 r + c of a load holds k = 4 c .. + 3 of row r (of
+    // 8), whole lines; byte offsets in 32 bits from the block's first row (strides checked at launch).
+    const int sr = lane >> 3, sc = lane & 7;
+    const char* base[2] = {reinterpret_cast<const char*>(p.x + row0 * p.x_stride), reinterpret_cast<const char*>(w + n0 * p.K)};
+    unsigned off[2][2];
+#pragma unroll
+    for (int m = 0; m < 2; ++m) {
+        const int r = 16 * wave + 8 * m + sr;
+        off[0][m] = static_cast<unsigned>((row0 + r < p.rows ? r : p.rows - 1 - row0) * p.x_stride * 4) + 16 * sc;
+        int64_t n = r;
+        if constexpr (SWIGLU) {
+            const int64_t col = 16 * (wave >> 1) + 8 * m + sr;
+            n = (n0 + col < p.N ? col : p.N - 1 - n0) + (wave & 1 ? p.N : 0);
+        } else {
+            n = n0 + n < p.N ? n : p.N - 1 - n0;
+        }
+        off[1][m] = static_cast<unsigned>(n * p.K * 4) + 16 * sc;
+    }
+    float4 v[2][2], nw;
+    bool live = true;  // of the fetched step (K a multiple of 4: a lane's 4 k are on one side of it)
+    auto fetch = [&](int k0) {
+        live = k0 + 4 * sc < K;
+        const unsigned ko = FULL ? (k0 < K ? 4 * k0 : 0u) : (live ? 4 * k0 : 0u - 16 * sc);
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int m = 0; m < 2; ++m) v[i][m] = *reinterpret_cast<const float4*>(base[i] + static_cast<unsigned>(off[i][m] + ko));
+        if constexpr (GS > 0) nw = *reinterpret_cast<const float4*>(p.norm_w + (live ? k0 + 4 * sc : 0));
+    };
+    // Values past K become zeros here and not at the load, whose wait would then stand in front of the products.
+    auto stage = [&](int k0) {
+        uint2* dst = reinterpret_cast<uint2*>(frag);
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int m = 0; m < 2; ++m) {
+                float4 f = v[i][m];
+                if (GS > 0 && i == 0) {
+                    const int k = live ? k0 + 4 * sc : 0;
+                    const double s = scale[(16 * wave + 8 * m + sr) * groups + k / (GS > 0 ? GS : 1)];
+                    f.x = static_cast<float>((static_cast<double>(f.x) * s) * static_cast<double>(nw.x));
+                    f.y = static_cast<float>((static_cast<double>(f.y) * s) * static_cast<double>(nw.y));
+                    f.z = static_cast<float>((static_cast<double>(f.z) * s) * static_cast<double>(nw.z));
+                    f.w = static_cast<float>((static_cast<double>(f.w) * s) * static_cast<double>(nw.w));
+                }
+                if (!FULL && !live) f = float4{0.0f, 0.0f, 0.0f, 0.0f};
+                f32x2 lo = {f.x, f.y}, hi = {f.z, f.w};
+                const unsigned slot = unit(2 * i + (wave >> 1), sc >> 2, 0, (sc >> 1) & 1) + 16 * (wave & 1) + 8 * m + sr;
+#pragma unroll
+                for (int q = 0; q < kPlanes; ++q) dst[2 * (slot + q * 2 * kGroupUnits) + (sc & 1)] = uint2{take_bf16(lo), take_bf16(hi)};
+            }
+    };
+
+    const int wm = wave & 1, wn = wave >> 1;
+    f32x16 acc, low;
+#pragma unroll
+    for (int c = 0; c < 16; ++c) acc[c] = low[c] = 0.0f;
+
+    fetch(0);
+    if constexpr (GS > 0) {
+        norm_scales<(GS > 0 ? GS : 8)>(p, row0, groups, scale);
+        __syncthreads();
+    }
+    for (int k0 = 0; k0 < K; k0 += kStep) {
+        if (k0 > 0) __syncthreads();
+        stage(k0);
+        __syncthreads();
+        fetch(k0 + kStep);
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            bf16x8 xf[kPlanes], wf[kPlanes];
+#pragma unroll
+            for (int q = 0; q < kPlanes; ++q) {
+                xf[q] = __builtin_bit_cast(bf16x8, frag[unit(wm, h, q, g) + li]);
+                wf[q] = __builtin_bit_cast(bf16x8, frag[unit(2 + wn, h, q, g) + li]);
+            }
+            acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[0], xf[0], acc, 0, 0, 0);
+#pragma unroll
+            for (int order = 1; order < kPlanes; ++order)
+#pragma unroll
+                for (int q = 0; q <= order; ++q) low = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[q], xf[order - q], low, 0, 0, 0);
+        }
+    }
+#pragma unroll
+    for (int c = 0; c < 16; ++c) acc[c] += low[c];
+
+    const int64_t row = row0 + 32 * wm + li;
+    if (row >= p.rows) return;
+    // W row of accumulator element c (0 .. 15), and its column of out.
+    auto w_row = [&](int c) -> int64_t {
+        const int r = 8 * (c >> 2) + 4 * g + (c & 3);
+        if constexpr (SWIGLU) return n0 + 16 * wn + (r & 15) + (r & 16 ? p.N : 0);
+        return n0 + 32 * wn + r;
+    };
+    auto in_range = [&](int c) {
+        if constexpr (SWIGLU) return w_row(c & 7) < p.N;
+        return w_row(c) < p.N;
+    };
+    bool finite = true;
+#pragma unroll
+    for (int c = 0; c < 16; ++c) finite = finite && acc[c] == acc[c];
+    if (!finite) {
+#pragma unroll 1
+        for (int c = 0; c < 16; ++c) {
+            if (!in_range(c)) continue;
+            const float* xr = p.x + row * p.x_stride;
+            const float* wr = w + w_row(c) * p.K;
+            float sum = 0.0f;
+#pragma unroll 1
+            for (int k = 0; k < K; ++k) {
+                float x = xr[k];
+                if constexpr (GS > 0)
+                    x = static_cast<float>((static_cast<double>(x) * scale[(32 * wm + li) * groups + k / GS]) *
+                                           static_cast<double>(p.norm_w[k]));
+                sum = fmaf(x, wr[k], sum);
+            }
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[e] = e == c && acc[e] != acc[e] ? sum : acc[e];
+        }
+    }
+    if (p.bias != nullptr) {
+#pragma unroll
+        for (int c = 0; c < 16; ++c) acc[c] += p.bias[in_range(c) ? w_row(c) : 0];
+    }
+
+    const bool vec_out = (reinterpret_cast<uintptr_t>(p.out) & 15) == 0 && p.out_stride % 4 == 0 &&
+                         (p.residual == nullptr ||
+                          ((reinterpret_cast<uintptr_t>(p.residual) & 15) == 0 && p.res_stride % 4 == 0));
+#pragma unroll
+    for (int j = 0; j < (SWIGLU ? 2 : 4); ++j) {
+        const int64_t col = w_row(4 * j);
+        if (col >= p.N) continue;
+        f32x4 y = {acc[4 * j], acc[4 * j + 1], acc[4 * j + 2], acc[4 * j + 3]};
+        if constexpr (SWIGLU) {
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+                y[c] = static_cast<float>(silu_d(static_cast<double>(y[c])) * static_cast<double>(acc[8 + 4 * j + c]));
+        }
+        float* dst = p.out + row * p.out_stride + col;
+        const float* res = p.residual != nullptr ? p.residual + row * p.res_stride + col : nullptr;
+        if (vec_out && col + 4 <= p.N) {
+            if (res != nullptr) y = *reinterpret_cast<const f32x4*>(res) + y;
+            *reinterpret_cast<f32x4*>(dst) = y;
+        } else {
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+                if (col + c < p.N) dst[c] = res != nullptr ? res[c] + y[c] : y[c];
+        }
+    }
+}
+
+template <int GS, bool SWIGLU>
+void launch(const LinearArgs& p, hipStream_t stream) {
+    const int64_t nb = ceil_div(p.N, SWIGLU ? kBlock / 2 : kBlock);
+    const dim3 grid(static_cast<unsigned>(ceil_div(p.rows, kBlock) * nb));
+    if (p.K % kStep == 0) {
+        hipLaunchKernelGGL((linear_split_kernel<true, GS, SWIGLU>), grid, dim3(256), 0, stream, p, static_cast<unsigned>(nb));
+    } else {
+        hipLaunchKernelGGL((linear_split_kernel<false, GS, SWIGLU>), grid, dim3(256), 0, stream, p, static_cast<unsigned>(nb));
+    }
+}
+
+// 32-bit byte offsets from a block's first rows, and the grid.
+bool fits(const LinearArgs& p, int64_t w_rows) {
+    return p.K % 4 == 0 && p.x_stride < (int64_t{1} << 23) && p.K * w_rows < (int64_t{1} << 30) &&
+           ceil_div(p.rows, kBlock) * ceil_div(p.N, kBlock / 2) < (int64_t{1} << 31);
+}
+
+}  // namespace
+
+bool linear_split_fits(const LinearArgs& p) { return fits(p, kBlock); }
+
+void launch_linear_split(const LinearArgs& p, hipStream_t stream) { launch<0, false>(p, stream); }
+
+void launch_linear_split_norm(const LinearArgs& p, int64_t group_size, hipStream_t stream) {
+    switch (group_size) {
+        case 8: launch<8, false>(p, stream); break;
+        case 16: launch<16, false>(p, stream); break;
+        case 32: launch<32, false>(p, stream); break;
+        default: launch<64, false>(p, stream); break;
+    }
+}
+
+}  // namespace mlk

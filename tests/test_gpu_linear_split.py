@@ -1,0 +1,91 @@
+"""The fp32-weight linear on three bf16 planes (linear_split.hip) and the four-waves-per-tile form for few tiles
+(linear_small_split_kernel): edges of their tiles and of the rules that choose them, against float64."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _operands(dev, M, K, N, seed, wdt="f32", pad=0):
+    g = torch.Generator(device="cpu").manual_seed(seed)
+    x = torch.randn(M, K + pad, generator=g).to(dev)[:, :K]
+    w = (torch.randn(N, K, generator=g) / K ** 0.5).to(dev)
+    b, r = torch.randn(N, generator=g).to(dev), torch.randn(M, N, generator=g).to(dev)
+    return x, w.bfloat16() if wdt == "bf16" else w, b, r
+
+
+def _assert_bound(got, x, w, terms, extra=0.0):
+    """|y - x W^T| <= c 2^-24 sum |x| |w|: c counts the fp32 roundings a sum meets (one per `terms` products and
+    the few that join partial sums, bias and residual) and, for the three planes, the dropped 2^-26 terms."""
+    xd, wd = x.double(), w.double()
+    K = x.shape[1]
+    slack = (K / terms + 8) * 2.0 ** -24 * (xd.abs() @ wd.abs().t() + extra)
+    off = (got.double() - xd @ wd.t()).abs() - slack
+    assert bool((off <= 0).all()), f"{off.max().item():.3e} over the bound"
+
+
+# (rows, K, N, x row padding): one past a block, K not a multiple of the 32-wide step or of 8, ragged and tiny N, the
+# first shapes past the one-wave rule's 1536 tiles, K just above 128, one row against many columns.
+SPLIT = [(1921, 256, 352, 0), (2049, 136, 200, 4), (1600, 132, 257, 0), (30000, 256, 1, 8), (64, 2048, 5200, 0),
+         (1, 256, 24592, 0), (12304, 160, 30, 0), (1537, 256, 256, 12)]
+
+
+@pytest.mark.parametrize("M,K,N,pad", SPLIT)
+def test_split_linear_vs_float64(dev, M, K, N, pad):
+    from montlok import _C
+
+    x, w, b, r = _operands(dev, M, K, N, M + K + N, pad=pad)
+    y = _C.linear(x, w)
+    _assert_bound(y, x, w, 16)
+    assert torch.equal(_C.linear(x, w, b), y + b)
+    assert torch.equal(_C.linear_residual(x, w, b, r), r + (y + b))
+
+
+@pytest.mark.parametrize("M,K,N", [(1, 264, 16), (480, 512, 256), (77, 1000, 33), (1280 * 16, 520, 9), (17, 1024, 300)])
+@pytest.mark.parametrize("wdt", ["f32", "bf16"])
+def test_four_waves_per_tile_vs_float64(dev, M, K, N, wdt):
+    from montlok import _C
+
+    x, w, b, r = _operands(dev, M, K, N, M + K + N, wdt)
+    y = _C.linear(x, w)
+    _assert_bound(y, x.bfloat16() if wdt == "bf16" else x, w, 2)
+    assert torch.equal(_C.linear(x, w, b), y + b)
+    assert torch.equal(_C.linear_residual(x, w, b, r), r + (y + b))
+
+
+@pytest.mark.parametrize("M,K,N,groups", [(1921, 256, 352, 32), (1921, 256, 352, 16), (2500, 256, 300, 8),
+                                          (3001, 256, 270, 4), (2100, 160, 260, 20), (1930, 192, 350, 3)])
+def test_rms_norm_split_linear_equals_the_two_operators(dev, M, K, N, groups):
+    """Still one launch where the one-wave form used to serve these shapes, and the two operators bit for bit."""
+    from montlok import _C
+    from montlok._C import _load
+
+    x, w, b, _ = _operands(dev, M, K, N, M + groups)
+    x = 3 * x
+    nw = torch.rand(K, generator=torch.Generator().manual_seed(1)).to(dev) + 0.5
+    out = torch.empty(M, N, device=dev)
+    status = _load().mlk_rms_norm_linear(x.data_ptr(), M, K, K, nw.data_ptr(), 1e-5, groups, w.data_ptr(), 0,
+                                         b.data_ptr(), N, out.data_ptr(), N, torch.cuda.current_stream().cuda_stream)
+    assert status == 0
+    assert torch.equal(out, _C.linear(_C.rms_norm(x, nw, 1e-5, groups), w, b))
+
+
+def test_split_linear_special_values(dev):
+    """Infinities, NaN, values whose bf16 rounding is infinite, subnormals: as the fp32 sum has them."""
+    from montlok import _C
+
+    x, w, _, _ = _operands(dev, 2000, 256, 300, 7)
+    x[3, 5], x[64, 9], x[70, 11], x[200, 200] = float("inf"), float("nan"), 3.4e38, float("-inf")
+    x[300] = 1e-39
+    w[7, 200], w[9, 3], w[11] = float("inf"), 0.0, 0.0
+    w[11, 11] = 0.5
+    y, ref = _C.linear(x, w), (x.double() @ w.double().t()).float()
+    assert torch.equal(torch.isnan(y), torch.isnan(ref)) and torch.equal(torch.isinf(y), torch.isinf(ref))
+    assert torch.equal(y[torch.isinf(y)], ref[torch.isinf(ref)])
+    assert abs(y[70, 11].item() / 1.7e38 - 1) < 1e-6
+    plain = [i for i in range(2000) if i not in (3, 64, 70, 200, 300)]
+    cols = [j for j in range(300) if j != 7]
+    _assert_bound(y[plain][:, cols], x[plain], w[cols], 16)
