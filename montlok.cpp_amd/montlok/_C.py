@@ -88,6 +88,29 @@ def _load():
     return lib
 
 
+_native = None
+
+
+def _ops():
+    """The operators that make one launch each, from tensors to the C ABI (csrc/torch_ops.cpp), bound to the
+    library that ``_load`` opened."""
+    global _native
+    if _native is None:
+        import importlib.machinery
+        import importlib.util
+
+        _load()
+        path = LIB_PATH.with_name("_torch_ops.so")
+        if not path.exists():
+            raise RuntimeError(f"{path} is not built: run __graft_entry__.build() (make -C montlok.cpp_amd)")
+        loader = importlib.machinery.ExtensionFileLoader("_torch_ops", str(path))
+        module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_torch_ops", loader))
+        loader.exec_module(module)
+        module.bind(os.environ.get("MLK_HIP_LIB", str(LIB_PATH)))
+        _native = module
+    return _native
+
+
 def library():
     """The loaded ``libmlk_hip.so`` (ctypes.CDLL)."""
     return _load()
@@ -101,7 +124,7 @@ def _call(name: str, *args) -> None:
 
 
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    return (_native or _ops()).current_stream()
 
 
 def _ptr(t: torch.Tensor | None) -> int | None:
@@ -140,60 +163,23 @@ def _rows(x: torch.Tensor, dim: int) -> tuple[torch.Tensor, int, int]:
 
 def rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float, groups: int) -> torch.Tensor:
     """montlok.cpp:915-938."""
-    _require_f32_gpu(x, "x")
-    _check(x.dim() >= 1, "x must have at least one dimension")
-    dim = x.size(-1)
-    _check(groups > 0 and dim % groups == 0, "groups must divide the normalised dimension")
-    w = _dense_parameter(weight, dim, "weight")
-    rows, count, stride = _rows(x, dim)
-    out = torch.empty((count, dim), dtype=torch.float32, device=x.device)
-    _call("mlk_rms_norm", _ptr(rows), count, dim, stride, _ptr(w), float(eps), int(groups), _ptr(out), _stream())
-    return out.view(x.shape)
+    return (_native or _ops()).rms_norm(x, weight, eps, groups)
 
 
 def add_rms_norm(left: torch.Tensor, right: torch.Tensor, weight: torch.Tensor, eps: float,
                  groups: int) -> tuple[torch.Tensor, torch.Tensor]:
     """montlok.cpp:978-1007: (left + right, rms_norm(left + right))."""
-    _require_f32_gpu(left, "left")
-    _require_f32_gpu(right, "right")
-    _check(left.shape == right.shape and left.dim() >= 1, "residual operands must have the same shape")
-    dim = left.size(-1)
-    _check(groups > 0 and dim % groups == 0, "groups must divide the normalized dimension")
-    lr = left.reshape(-1, dim).contiguous()
-    rr = right.reshape(-1, dim).contiguous()
-    w = _dense_parameter(weight, dim, "weight")
-    residual = torch.empty_like(lr)
-    normalized = torch.empty_like(lr)
-    _call("mlk_add_rms_norm", _ptr(lr), _ptr(rr), lr.size(0), dim, _ptr(w), float(eps), int(groups), _ptr(residual),
-          _ptr(normalized), _stream())
-    return residual.view(left.shape), normalized.view(left.shape)
+    return (_native or _ops()).add_rms_norm(left, right, weight, eps, groups)
 
 
 def layer_norm(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None, eps: float) -> torch.Tensor:
     """montlok.cpp:1057-1082 (bias may be None or empty)."""
-    _require_f32_gpu(x, "x")
-    _check(x.dim() >= 1, "x must have at least one dimension")
-    dim = x.size(-1)
-    w = _dense_parameter(weight, dim, "weight")
-    b = None
-    if bias is not None and bias.numel() > 0:
-        b = _dense_parameter(bias, dim, "bias")
-    rows, count, stride = _rows(x, dim)
-    out = torch.empty((count, dim), dtype=torch.float32, device=x.device)
-    _call("mlk_layer_norm", _ptr(rows), count, dim, stride, _ptr(w), _ptr(b), float(eps), _ptr(out), _stream())
-    return out.view(x.shape)
+    return (_native or _ops()).layer_norm(x, weight, bias, eps)
 
 
 def swiglu(x: torch.Tensor) -> torch.Tensor:
     """montlok.cpp:942-963: x [..., 2*hidden] = [gate | up] -> silu(gate) * up."""
-    _require_f32_gpu(x, "x")
-    _check(x.dim() >= 1 and x.size(-1) % 2 == 0, "x must end in an even dimension [gate | up]")
-    width = x.size(-1)
-    hidden = width // 2
-    rows, count, stride = _rows(x, width)
-    out = torch.empty((count, hidden), dtype=torch.float32, device=x.device)
-    _call("mlk_swiglu", _ptr(rows), count, hidden, stride, _ptr(out), _stream())
-    return out.view(*x.shape[:-1], hidden)
+    return (_native or _ops()).swiglu(x)
 
 
 # ------------------------------------------------------------------ linear
@@ -220,65 +206,24 @@ def linear(input: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None 
     """linear_dispatch (montlok.cpp:67-91): input [..., K] @ weight[N, K]^T + bias -> [..., N].
 
     weight may be float32 or bfloat16 (bf16 matrix cores, fp32 accumulate)."""
-    _require_f32_gpu(input, "input")
-    w = _weight(weight)
-    n, k = w.shape
-    _check(input.dim() >= 1 and input.size(-1) == k, f"input must end in in_features={k}")
-    b = None
-    if bias is not None and bias.numel() > 0:
-        b = _dense_parameter(bias, n, "bias")
-    rows, count, stride = _rows(input, k)
-    out = torch.empty((count, n), dtype=torch.float32, device=input.device)
-    _linear_into(rows, count, stride, w, b, out, n)
-    return out.view(*input.shape[:-1], n)
+    return (_native or _ops()).linear(input, weight, bias)
 
 
 def linear_residual(input: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None,
                     residual: torch.Tensor) -> torch.Tensor:
     """residual + linear(input, weight, bias) in one launch, bit-identical to the two steps (the
     x = x + f(x) update of python/montlok/rdt/reference/Model/blocks.py:66-75)."""
-    _require_f32_gpu(input, "input")
-    _require_f32_gpu(residual, "residual")
-    w = _weight(weight)
-    n, k = w.shape
-    _check(input.dim() >= 1 and input.size(-1) == k, f"input must end in in_features={k}")
-    _check(tuple(residual.shape) == tuple(input.shape[:-1]) + (n,), "residual must have the output's shape")
-    b = None
-    if bias is not None and bias.numel() > 0:
-        b = _dense_parameter(bias, n, "bias")
-    rows, count, stride = _rows(input, k)
-    res = residual.reshape(count, n).contiguous()
-    out = torch.empty((count, n), dtype=torch.float32, device=input.device)
-    _call("mlk_linear_residual", _ptr(rows), count, k, stride, _ptr(w), _WEIGHT_DTYPES[w.dtype], _ptr(b), n,
-          _ptr(res), n, _ptr(out), n, _stream())
-    return out.view(*input.shape[:-1], n)
+    return (_native or _ops()).linear_residual(input, weight, bias, residual)
 
 
 def rms_norm_linear(x: torch.Tensor, norm_weight: torch.Tensor, eps: float, groups: int, weight: torch.Tensor,
                     bias: torch.Tensor | None = None) -> torch.Tensor:
     """linear(rms_norm(x, norm_weight, eps, groups), weight, bias), one launch where the fused form is
     built (small row counts), else the two operators; the results are identical either way."""
-    _require_f32_gpu(x, "x")
-    _check(x.dim() >= 1, "x must have at least one dimension")
-    dim = x.size(-1)
-    _check(groups > 0 and dim % groups == 0, "groups must divide the normalised dimension")
-    nw = _dense_parameter(norm_weight, dim, "weight")
-    w = _weight(weight)
-    n, k = w.shape
-    _check(k == dim, f"input must end in in_features={k}")
-    b = None
-    if bias is not None and bias.numel() > 0:
-        b = _dense_parameter(bias, n, "bias")
-    rows, count, stride = _rows(x, dim)
-    out = torch.empty((count, n), dtype=torch.float32, device=x.device)
-    lib = _load()
-    status = lib.mlk_rms_norm_linear(_ptr(rows), count, k, stride, _ptr(nw), float(eps), int(groups), _ptr(w),
-                                     _WEIGHT_DTYPES[w.dtype], _ptr(b), n, _ptr(out), n, _stream())
-    if status == 3:  # MLK_ERR_UNSUPPORTED: no fused form for this shape
+    out = (_native or _ops()).rms_norm_linear(x, norm_weight, eps, groups, weight, bias)
+    if out is None:  # no fused form for this shape
         return linear(rms_norm(x, norm_weight, eps, groups), weight, bias)
-    if status != 0:
-        raise RuntimeError(lib.mlk_last_error().decode())
-    return out.view(*x.shape[:-1], n)
+    return out
 
 
 def swiglu_mlp(input, in_weight, in_bias=None, out_weight=None, out_bias=None):
@@ -289,97 +234,21 @@ def swiglu_mlp(input, in_weight, in_bias=None, out_weight=None, out_bias=None):
 # ------------------------------------------------------------------ mHC
 
 
-def _streams_view(streams: torch.Tensor, n_streams: int, name: str):
-    """montlok.cpp:535-557 (StreamsView): [B,L,n,d] or the broadcast [B,L,d] backbone."""
-    _require_f32_gpu(streams, name)
-    _check(streams.is_contiguous(), f"{name} must be contiguous")
-    if streams.dim() == 4:
-        n, d = streams.size(2), streams.size(3)
-        sd = d
-        _check(n_streams <= 0 or n_streams == n, f"{name} has {n} streams, expected {n_streams}")
-    else:
-        _check(streams.dim() == 3, f"{name} must be [B,L,n,d] or a broadcast [B,L,d]")
-        _check(n_streams > 0, f"n_streams is required for a broadcast [B,L,d] {name}")
-        n, d = n_streams, streams.size(2)
-        sd = 0
-    B, L = streams.size(0), streams.size(1)
-    ts = d if sd == 0 else n * d
-    _check(n > 0 and d > 0, f"{name} must be non-empty")
-    return B, L, n, d, sd, ts
-
-
-def _scalar(t: torch.Tensor, name: str) -> torch.Tensor:
-    _require_f32_gpu(t, name)
-    _check(t.numel() == 1, f"{name} must be a scalar")
-    return t.reshape(1).contiguous()
-
-
-def _prepare_params(n, d, norm_w, proj_w, pre_bias, post_bias, res_bias, pre_alpha, post_alpha, res_alpha,
-                    sinkhorn_iters, agg_norm_w):
-    """montlok.cpp:568-649 (mhc_prepare_plan)."""
-    _check(sinkhorn_iters >= 0, "sinkhorn_iters must be non-negative")
-    params = [
-        _dense_parameter(norm_w, d, "dyn_norm.weight"),
-        _dense_parameter(pre_bias, n, "pre_bias"),
-        _dense_parameter(post_bias, n, "post_bias"),
-        _dense_parameter(res_bias, n * n, "res_bias"),
-    ]
-    _check(proj_w.device.type == "cuda" and proj_w.dtype == torch.float64 and proj_w.is_contiguous(),
-           "proj_w must be a contiguous float64 GPU tensor")
-    _check(proj_w.dim() == 2 and proj_w.size(0) == 2 * n + n * n and proj_w.size(1) == d,
-           "proj_w must be [2n + n*n, d]")
-    alphas = [_scalar(pre_alpha, "pre_alpha"), _scalar(post_alpha, "post_alpha"), _scalar(res_alpha, "res_alpha")]
-    anw = None
-    if agg_norm_w is not None and agg_norm_w.numel() > 0:
-        anw = _dense_parameter(agg_norm_w, d, "agg_norm_w")
-    return params, alphas, anw
-
-
 def mhc_prepare(streams, norm_w, eps, proj_w, pre_bias, post_bias, res_bias, pre_alpha, post_alpha, res_alpha,
                 sinkhorn_iters, n_streams=0, agg_norm_w=None, agg_norm_eps=0.0):
     """montlok.cpp:659-691 -> (agg [B,L,d], pre [B,L,n], post [B,L,n], res [B,L,n,n])."""
-    B, L, n, d, sd, ts = _streams_view(streams, n_streams, "streams")
-    (nw, pb, qb, rb), (pa, qa, ra), anw = _prepare_params(n, d, norm_w, proj_w, pre_bias, post_bias, res_bias,
-                                                          pre_alpha, post_alpha, res_alpha, sinkhorn_iters,
-                                                          agg_norm_w)
-    dev = streams.device
-    agg = torch.empty((B, L, d), dtype=torch.float32, device=dev)
-    pre = torch.empty((B, L, n), dtype=torch.float32, device=dev)
-    post = torch.empty((B, L, n), dtype=torch.float32, device=dev)
-    res = torch.empty((B, L, n, n), dtype=torch.float32, device=dev)
-    _call("mlk_mhc_prepare", _ptr(streams), B * L, n, d, sd, ts, _ptr(nw), float(eps), _ptr(proj_w), _ptr(pb),
-          _ptr(qb), _ptr(rb), _ptr(pa), _ptr(qa), _ptr(ra), int(sinkhorn_iters), _ptr(anw), float(agg_norm_eps),
-          _ptr(agg), _ptr(pre), _ptr(post), _ptr(res), _stream())
-    return agg, pre, post, res
-
-
-def _combine_inputs(streams, res, post, out):
-    B, L, n, d, sd, ts = _streams_view(streams, res.size(-1) if res.dim() == 4 else 0, "streams")
-    _require_f32_gpu(res, "res")
-    _require_f32_gpu(post, "post")
-    _require_f32_gpu(out, "out")
-    _check(tuple(res.shape) == (B, L, n, n) and res.is_contiguous(), "res must be contiguous [B,L,n,n]")
-    _check(tuple(post.shape) == (B, L, n) and post.is_contiguous(), "post must be contiguous [B,L,n]")
-    _check(tuple(out.shape) == (B, L, d) and out.is_contiguous(), "out must be contiguous [B,L,d]")
-    return B, L, n, d, sd, ts
+    return (_native or _ops()).mhc_prepare(streams, norm_w, eps, proj_w, pre_bias, post_bias, res_bias, pre_alpha, post_alpha,
+                                           res_alpha, sinkhorn_iters, n_streams, agg_norm_w, agg_norm_eps)
 
 
 def mhc_combine(streams, res, post, out):
     """montlok.cpp:726-739 -> new streams [B,L,n,d]."""
-    B, L, n, d, sd, ts = _combine_inputs(streams, res, post, out)
-    new = torch.empty((B, L, n, d), dtype=torch.float32, device=streams.device)
-    _call("mlk_mhc_combine", _ptr(streams), B * L, n, d, sd, ts, _ptr(res), _ptr(post), _ptr(out), _ptr(new), None,
-          _stream())
-    return new
+    return (_native or _ops()).mhc_combine(streams, res, post, out, False)
 
 
 def mhc_combine_collapse(streams, res, post, out):
     """montlok.cpp:743-758 -> mean over the new streams [B,L,d]; streams never materialised."""
-    B, L, n, d, sd, ts = _combine_inputs(streams, res, post, out)
-    hidden = torch.empty((B, L, d), dtype=torch.float32, device=streams.device)
-    _call("mlk_mhc_combine", _ptr(streams), B * L, n, d, sd, ts, _ptr(res), _ptr(post), _ptr(out), None,
-          _ptr(hidden), _stream())
-    return hidden
+    return (_native or _ops()).mhc_combine(streams, res, post, out, True)
 
 
 def mhc_combine_prepare(streams, res, post, out, norm_w, eps, proj_w, pre_bias, post_bias, res_bias, pre_alpha,
@@ -396,32 +265,9 @@ def _mhc_combine_prepare(streams, res, post, out, norm_w, eps, proj_w, pre_bias,
     mhc_combine_prepare_reuse): reuse_streams writes the new streams over `streams` (contiguous
     [B, L, n, d], n <= 8); `into` = (agg, pre, post, res) buffers the next residual's coefficients are
     written into (they may be the `res` and `post` this call reads). Values are those of the plain call."""
-    B, L, n, d, sd, ts = _combine_inputs(streams, res, post, out)
-    (nw, pb, qb, rb), (pa, qa, ra), anw = _prepare_params(n, d, norm_w, proj_w, pre_bias, post_bias, res_bias,
-                                                          pre_alpha, post_alpha, res_alpha, sinkhorn_iters,
-                                                          agg_norm_w)
-    dev = streams.device
-    if reuse_streams:
-        _check(streams.dim() == 4 and sd == d and ts == n * d and n <= 8,
-               "in-place mHC requires contiguous materialised streams with at most eight lanes")
-        new = streams
-    else:
-        new = torch.empty((B, L, n, d), dtype=torch.float32, device=dev)
-    if into is not None:
-        agg, pre_o, post_o, res_o = into
-        for t, shape, name in ((agg, (B, L, d), "agg"), (pre_o, (B, L, n), "pre"), (post_o, (B, L, n), "post"),
-                               (res_o, (B, L, n, n), "res")):
-            _check(t.dtype == torch.float32 and t.is_contiguous() and tuple(t.shape) == shape,
-                   f"{name} workspace must be contiguous float32 {list(shape)}")
-    else:
-        agg = torch.empty((B, L, d), dtype=torch.float32, device=dev)
-        pre_o = torch.empty((B, L, n), dtype=torch.float32, device=dev)
-        post_o = torch.empty((B, L, n), dtype=torch.float32, device=dev)
-        res_o = torch.empty((B, L, n, n), dtype=torch.float32, device=dev)
-    _call("mlk_mhc_combine_prepare", _ptr(streams), B * L, n, d, sd, ts, _ptr(res), _ptr(post), _ptr(out), _ptr(nw),
-          float(eps), _ptr(proj_w), _ptr(pb), _ptr(qb), _ptr(rb), _ptr(pa), _ptr(qa), _ptr(ra), int(sinkhorn_iters),
-          _ptr(anw), float(agg_norm_eps), _ptr(new), _ptr(agg), _ptr(pre_o), _ptr(post_o), _ptr(res_o), _stream())
-    return new, agg, pre_o, post_o, res_o
+    return (_native or _ops()).mhc_combine_prepare(streams, res, post, out, norm_w, eps, proj_w, pre_bias, post_bias, res_bias,
+                                                   pre_alpha, post_alpha, res_alpha, sinkhorn_iters, agg_norm_w,
+                                                   agg_norm_eps, reuse_streams, into)
 
 
 # ------------------------------------------------------------------ Mamba-3
@@ -481,42 +327,13 @@ def _siso_recurrent(q, k, v, gate, adt, dt, trap_logit, skip, noalloc: bool):
     return out
 
 
-def _mamba_params(b_bias, c_bias, b_norm_w, c_norm_w, dt_bias, skip, d_state, nheads):
-    return (_dense_parameter(b_bias, nheads * d_state, "B_bias"), _dense_parameter(c_bias, nheads * d_state, "C_bias"),
-            _dense_parameter(b_norm_w, d_state, "B_norm.weight"), _dense_parameter(c_norm_w, d_state, "C_norm.weight"),
-            _dense_parameter(dt_bias, nheads, "dt_bias"), _dense_parameter(skip, nheads, "D"))
-
-
 def mamba3_siso_forward(projected, gate, b_bias, c_bias, b_norm_w, c_norm_w, dt_bias, skip, d_state, ngroups,
                         nheads, headdim, num_rope_angles, b_eps, c_eps, a_floor):
     """montlok.cpp:333-492: in_proj output [B, L, W] -> out_proj input [B, L, d_inner].
 
     An empty ``gate`` evaluates silu of the z lanes of ``projected`` in the kernel."""
-    _require_f32_gpu(projected, "projected")
-    gate_logits = gate is None or gate.numel() == 0
-    if not gate_logits:
-        _require_f32_gpu(gate, "gate")
-    _check(projected.dim() == 3, "projected must be [B,L,W]")
-    _check(d_state > 0 and ngroups > 0 and nheads > 0 and headdim > 0, "invalid Mamba-3 geometry")
-    _check(nheads % ngroups == 0, "nheads must be divisible by ngroups")
-    _check(num_rope_angles >= 0 and 2 * num_rope_angles <= d_state, "num_rope_angles must fit in d_state")
-    _require_inner_dense(projected, "projected")
-    B, L, W = projected.shape
-    d_inner = nheads * headdim
-    if not gate_logits:
-        _require_inner_dense(gate, "gate")
-        _check(gate.dim() == 3 and tuple(gate.shape) == (B, L, d_inner), "gate must be [B,L,d_inner]")
-    expected = 2 * d_inner + 2 * ngroups * d_state + 3 * nheads + num_rope_angles
-    _check(W == expected, f"projected width {W} does not match the Mamba-3 layout width {expected}")
-    params = _mamba_params(b_bias, c_bias, b_norm_w, c_norm_w, dt_bias, skip, d_state, nheads)
-    out = torch.empty((B, L, d_inner), dtype=torch.float32, device=projected.device)
-    lib = _load()
-    ws = _workspace(lib.mlk_mamba3_workspace_bytes(B, L, nheads, d_state, num_rope_angles), projected.device)
-    gsb, gst = (0, 0) if gate_logits else (gate.stride(0), gate.stride(1))
-    _call("mlk_mamba3_siso_forward", _ptr(projected), B, L, W, projected.stride(0), projected.stride(1),
-          None if gate_logits else _ptr(gate), gsb, gst, *(_ptr(t) for t in params), d_state, ngroups, nheads, headdim,
-          num_rope_angles, float(b_eps), float(c_eps), float(a_floor), _ptr(out), _ptr(ws), ws.numel(), _stream())
-    return out
+    return (_native or _ops()).mamba3_siso_forward(projected, gate, b_bias, c_bias, b_norm_w, c_norm_w, dt_bias, skip, d_state,
+                                                   ngroups, nheads, headdim, num_rope_angles, b_eps, c_eps, a_floor)
 
 
 def mamba3_siso_step(projected, state, b_bias, c_bias, b_norm_w, c_norm_w, dt_bias, skip, d_state, ngroups,
@@ -527,27 +344,9 @@ def mamba3_siso_step(projected, state, b_bias, c_bias, b_norm_w, c_norm_w, dt_bi
     (float32), angle [S,H,max(R,1)] (float64) updated in place, and
     ``started`` (False before the first token of a zero state; set True here).
     Returns [S, H*D]."""
-    _require_f32_gpu(projected, "projected")
-    _check(projected.dim() == 2, "projected must be [S,W]")
-    _require_inner_dense(projected, "projected")
-    S, W = projected.shape
-    d_inner = nheads * headdim
-    expected = 2 * d_inner + 2 * ngroups * d_state + 3 * nheads + num_rope_angles
-    _check(W == expected, f"projected width {W} does not match the Mamba-3 layout width {expected}")
-    rw = max(num_rope_angles, 1)
-    shapes = {"ssm": (S, nheads, d_state, headdim), "k": (S, nheads, d_state), "v": (S, nheads, headdim),
-              "angle": (S, nheads, rw)}
-    for key, shape in shapes.items():
-        t = state[key]
-        _check(tuple(t.shape) == shape and t.is_contiguous() and t.device.type == "cuda",
-               f"state['{key}'] must be a contiguous GPU tensor of shape {shape}")
-        _check(t.dtype == (torch.float64 if key == "angle" else torch.float32), f"state['{key}'] has the wrong dtype")
-    params = _mamba_params(b_bias, c_bias, b_norm_w, c_norm_w, dt_bias, skip, d_state, nheads)
-    out = torch.empty((S, d_inner), dtype=torch.float32, device=projected.device)
-    _call("mlk_mamba3_siso_step", _ptr(projected), S, projected.stride(0), *(_ptr(t) for t in params), d_state,
-          ngroups, nheads, headdim, num_rope_angles, float(b_eps), float(c_eps), float(a_floor), _ptr(state["ssm"]),
-          _ptr(state["k"]), _ptr(state["v"]), _ptr(state["angle"]), int(bool(state.get("started", False))), _ptr(out),
-          _stream())
+    out = (_native or _ops()).mamba3_siso_step(projected, state["ssm"], state["k"], state["v"], state["angle"],
+                                               bool(state.get("started", False)), b_bias, c_bias, b_norm_w, c_norm_w, dt_bias,
+                                               skip, d_state, ngroups, nheads, headdim, num_rope_angles, b_eps, c_eps, a_floor)
     state["started"] = True
     return out
 
@@ -572,29 +371,12 @@ def rms_norm_mamba3_forward(inputs, norm_weight, norm_eps, norm_groups, in_weigh
     geometry (the in_proj rows stay in LDS), else rms_norm_linear then mamba3_siso_forward; the same result
     bit for bit where rms_norm_linear takes its one-wave-per-tile form. No single counterpart in the
     reference's op table (montlok.cpp:915-938, 333-492)."""
-    _require_f32_gpu(inputs, "inputs")
-    _check(inputs.dim() == 3, "inputs must be [B,L,d_model]")
-    B, L, dm = inputs.shape
-    _check(norm_groups > 0 and dm % norm_groups == 0, "groups must divide the normalised dimension")
-    nw = _dense_parameter(norm_weight, dm, "weight")
-    w_in = _weight(in_weight)
-    d_inner = nheads * headdim
-    width = 2 * d_inner + 2 * ngroups * d_state + 3 * nheads + num_rope_angles
-    _check(tuple(w_in.shape) == (width, dm), f"in_proj weight must be [{width}, {dm}]")
-    params = _mamba_params(b_bias, c_bias, b_norm_w, c_norm_w, dt_bias, skip, d_state, nheads)
-    if inputs.stride(-1) == 1:
-        out = torch.empty((B, L, d_inner), dtype=torch.float32, device=inputs.device)
-        lib = _load()
-        status = lib.mlk_rms_norm_mamba3_forward(_ptr(inputs), B, L, dm, inputs.stride(0), inputs.stride(1),
-                                                 _ptr(nw), float(norm_eps), int(norm_groups), _ptr(w_in),
-                                                 _WEIGHT_DTYPES[w_in.dtype], *(_ptr(t) for t in params), d_state,
-                                                 ngroups, nheads, headdim, num_rope_angles, float(b_eps),
-                                                 float(c_eps), float(a_floor), _ptr(out), _stream())
-        if status == 0:
-            _BLOCK_PATH["mixer"] = ["rms_norm_mamba3_forward"]
-            return out
-        if status != 3:  # anything but MLK_ERR_UNSUPPORTED
-            raise RuntimeError(lib.mlk_last_error().decode())
+    out = (_native or _ops()).rms_norm_mamba3_forward(inputs, norm_weight, norm_eps, norm_groups, in_weight, b_bias, c_bias,
+                                                      b_norm_w, c_norm_w, dt_bias, skip, d_state, ngroups, nheads, headdim,
+                                                      num_rope_angles, b_eps, c_eps, a_floor)
+    if out is not None:
+        _BLOCK_PATH["mixer"] = ["rms_norm_mamba3_forward"]
+        return out
     projected = rms_norm_linear(inputs, norm_weight, norm_eps, norm_groups, in_weight)
     _BLOCK_PATH["mixer"] = ["rms_norm_linear", "mamba3_siso_forward"]
     return mamba3_siso_forward(projected, None, b_bias, c_bias, b_norm_w, c_norm_w, dt_bias, skip, d_state, ngroups,
@@ -776,39 +558,7 @@ MASK_NONE, MASK_CAUSAL_TOP_LEFT, MASK_CAUSAL_BOTTOM_RIGHT = 0, 1, 2
 def mla_rope_qk(q: torch.Tensor, kv: torch.Tensor, k_rope: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor,
                 nope_dim: int) -> torch.Tensor:
     """montlok.cpp:1093-1154: rotates q's rope lanes IN PLACE and returns k = cat(k_nope, rope(k_rope))."""
-    for t, name in ((q, "q"), (kv, "kv"), (k_rope, "k_rope"), (cos, "cos"), (sin, "sin")):
-        _require_f32_gpu(t, name)
-    _check(q.dim() == 4, "q must be [B,Lq,H,head_dim]")
-    _check(kv.dim() == 4 and kv.is_contiguous(), "kv must be contiguous [B,L,H,nope_dim+head_dim]")
-    batch, q_length, heads, head_dim = q.shape
-    length = kv.size(1)
-    rope_dim = head_dim - nope_dim
-    _check(nope_dim >= 0 and rope_dim > 0 and rope_dim % 2 == 0, "head_dim - nope_dim must be a positive even rope_dim")
-    _check(1 <= q_length <= length, "q must cover between 1 and L trailing positions")
-    _check((q.stride(3) == 1 or head_dim == 1) and (q.stride(2) == head_dim or heads == 1) and
-           (q.stride(0) == q_length * q.stride(1) or batch == 1),
-           "q must be dense within a token with a uniform token stride")
-    _check(tuple(kv.shape) == (batch, length, heads, nope_dim + head_dim), "kv must be [B,L,H,nope_dim+head_dim]")
-    _check(tuple(k_rope.shape) == (batch, length, rope_dim), "k_rope must be [B,L,rope_dim]")
-    _check((k_rope.stride(2) == 1 or rope_dim == 1) and (k_rope.stride(0) == length * k_rope.stride(1) or batch == 1),
-           "k_rope must be dense within a token with a uniform token stride")
-    _check(tuple(cos.shape) == (length, rope_dim) and cos.is_contiguous(), "cos must be contiguous [L,rope_dim]")
-    _check(sin.shape == cos.shape and sin.is_contiguous(), "sin must be contiguous [L,rope_dim]")
-    k = torch.empty((batch, length, heads, head_dim), dtype=torch.float32, device=q.device)
-    q_ts = q.stride(1) if q_length > 1 or batch == 1 else q.stride(0)
-    kr_ts = k_rope.stride(1) if length > 1 else k_rope.stride(0)
-    _call("mlk_mla_rope_qk", _ptr(q), max(q_ts, heads * head_dim), q_length, _ptr(kv), _ptr(k_rope),
-          max(kr_ts, rope_dim), _ptr(cos), _ptr(sin), batch, length, heads, head_dim, nope_dim, _ptr(k), _stream())
-    return k
-
-
-def _token_strides(t: torch.Tensor, name: str) -> tuple[int, int]:
-    """(token stride, head stride) of a [B, L, H, hd] view whose sequences are L tokens apart."""
-    B, L, H, hd = t.shape
-    _check(t.stride(3) == 1 or hd == 1, f"{name} must be dense in head_dim")
-    ts = t.stride(1) if L > 1 else (t.stride(0) if B > 1 else H * t.stride(2))
-    _check(B == 1 or t.stride(0) == L * ts, f"{name} must have a uniform token stride")
-    return ts, (t.stride(2) if H > 1 else hd)
+    return (_native or _ops()).mla_rope_qk(q, kv, k_rope, cos, sin, nope_dim)
 
 
 def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, mask: int, scale: float,
@@ -817,18 +567,8 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, mask: int, scal
 
     mask: MASK_NONE, MASK_CAUSAL_TOP_LEFT (is_causal) or MASK_CAUSAL_BOTTOM_RIGHT (trailing queries).
     precision: torch.bfloat16 runs QK^T and PV on bf16 matrix cores, torch.float32 stays fp32."""
-    for t, name in ((q, "q"), (k, "k"), (v, "v")):
-        _require_f32_gpu(t, name)
-        _check(t.dim() == 4, f"{name} must be [B,L,H,head_dim]")
-    B, Lq, H, hd = q.shape
-    Lk = k.size(1)
-    _check(tuple(k.shape) == (B, Lk, H, hd) and tuple(v.shape) == (B, Lk, H, hd), "k and v must be [B,L,H,head_dim]")
     _check(precision in (torch.float32, torch.bfloat16), "precision must be float32 or bfloat16")
-    qs, ks, vs = _token_strides(q, "q"), _token_strides(k, "k"), _token_strides(v, "v")
-    out = torch.empty((B, Lq, H, hd), dtype=torch.float32, device=q.device)
-    _call("mlk_attention", _ptr(q), *qs, _ptr(k), *ks, _ptr(v), *vs, B, H, Lq, Lk, hd, int(mask), float(scale),
-          _WEIGHT_DTYPES[precision], _ptr(out), _stream())
-    return out
+    return (_native or _ops()).attention(q, k, v, mask, scale, precision == torch.bfloat16)
 
 
 def mla_forward(x, in_proj_weight, q_weight, kv_norm_weight, kv_norm_bias, kv_norm_eps, kv_up_weight, out_weight,
