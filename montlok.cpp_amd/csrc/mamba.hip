@@ -1573,6 +1573,462 @@ bool launch_scan_fused(const ScanArgs& s, int64_t N, int64_t D, hipStream_t stre
 }
 
 // ---------------------------------------------------------------------------
+// The scan with its chunks in parallel, for few (window, head) pairs
+// ---------------------------------------------------------------------------
+//
+// scan_fused_kernel walks a (window, head)'s chunks on one block: 8.3 us a
+// chunk however few pairs there are (480 tokens: 125 us for 8 pairs and for
+// 256), nearly all of it the preparation of q, k and the weights, which no
+// chunk needs another one for. With few pairs the same arithmetic runs in four
+// launches, three of them over every chunk at once:
+//   token  (window, chunk)        step coefficients of every head, tanh(angle)
+//                                 pi once for all heads, and each head's sum
+//                                 of the chunk's angle terms
+//   chunk  (window, head, chunk)  steps a to e of scan_head: norm scales, decay
+//                                 weights, q and k, their rotation (from the
+//                                 angle sums of the chunks before), the masked
+//                                 G^T tiles; q, k and the tiles to the workspace
+//   state  (window, head)         step g alone, chunk after chunk: the state
+//                                 before every chunk to the workspace
+//   out    (window, head, chunk)  step f: outputs and gates
+// Every product and sum is scan_head's, in its order, so the result is the
+// fused kernel's bit for bit, but for the running angle sum, which adds fp64
+// sums of whole chunks (the last bits of an fp64 sum that is then rounded to
+// fp32).
+// 8 pairs x 480 tokens (d_state and headdim 64): 123 -> 34 us, 32 pairs 124 -> 43, 128 pairs 124 -> 75;
+// 8 pairs x 200 tokens 58 -> 25. What is left with few pairs is the state pass, 1.0 us a chunk (the instructions
+// of one or two waves a SIMD), and four launches of 4 to 5 us.
+
+// The workspace in floats: per (window, head, chunk) an item of
+//   k    [token tile][v][lane][NT]: k[16 st + 4 g + v][16 nt + li], the state pass's A operands
+//   q    [C][N]
+//   P    [tile pair][lane][4]
+//   w    [3][C]: the last token's decay weights, Din and Wp of every token
+//   last [N]: k of the chunk's last token
+//   S    [column tile][NT][lane][4]: the state before the chunk (not written for the first)
+// then the tokens' (alpha, beta, gamma, dt) [B, H, chunks C][4], tanh(angle) pi [B, chunks C][R] and, as
+// doubles, the chunks' angle sums [B, H, chunks][R].
+struct SplitScan {
+    int64_t chunks, item, coef, ang, csum, total;  // floats
+    int64_t k = 0, q, P, w, last, S;
+};
+__host__ __device__ inline SplitScan split_layout(int64_t B, int64_t L, int64_t H, int64_t N, int64_t D, int64_t R) {
+    constexpr int C = 32;
+    SplitScan s;
+    s.chunks = (L + C - 1) / C;
+    s.q = C * N;
+    s.P = s.q + C * N;
+    s.w = s.P + 3 * 64 * 4;
+    s.last = s.w + 3 * C;
+    s.S = s.last + N;
+    s.item = s.S + N * D;
+    s.coef = B * H * s.chunks * s.item;
+    s.ang = s.coef + B * H * s.chunks * C * 4;
+    s.csum = (s.ang + B * s.chunks * C * R + 3) / 4 * 4;
+    s.total = s.csum + 2 * B * H * s.chunks * R;
+    return s;
+}
+
+struct SplitScanArgs {
+    ScanArgs a;
+    float* ws;
+    SplitScan s;
+    int64_t N, D;
+};
+
+__global__ __launch_bounds__(256) void split_token_kernel(SplitScanArgs p) {
+    constexpr int C = 32;
+    extern __shared__ float token_s[];  // [C][R] tanh(angle) pi, [H][C] dt
+    const int H = static_cast<int>(p.a.H), R = static_cast<int>(p.a.R), L = static_cast<int>(p.a.L);
+    const int chunks = static_cast<int>(p.s.chunks);
+    const int64_t b = blockIdx.x / chunks;
+    const int c = static_cast<int>(blockIdx.x % chunks), c0 = C * c, Lc = L - c0 < C ? L - c0 : C;
+    const float* row = p.a.proj + b * p.a.sb + static_cast<int64_t>(c0) * p.a.st + 2 * H * p.D + 2 * p.a.G * p.N;
+    float* ang_s = token_s;
+    float* dt_s = token_s + C * R;
+    for (int i = threadIdx.x; i < C * H; i += 256) {
+        const int t = i % C, h = i / C;
+        const float* m = row + static_cast<int64_t>(t < Lc ? t : Lc - 1) * p.a.st + h;
+        const float dt = softplus_f(m[0] + p.a.dt_bias[h]);
+        const float am = -fmaxf(heavy_tail_f(m[H]), p.a.a_floor);
+        float al, be, ga;
+        step_coefficients(am * dt, dt, m[2 * H], &al, &be, &ga);
+        const bool valid = t < Lc;
+        dt_s[h * C + t] = dt;
+        float4* coef = reinterpret_cast<float4*>(p.ws + p.s.coef);
+        coef[((b * H + h) * chunks + c) * C + t] = valid ? make_float4(al, be, ga, dt) : make_float4(0.0f, 0.0f, 0.0f, dt);
+    }
+    for (int i = threadIdx.x; i < C * R; i += 256) {
+        const int t = i / R, r = i - t * R;
+        const float v = tanhf_cr(row[static_cast<int64_t>(t < Lc ? t : Lc - 1) * p.a.st + 3 * H + r]) * kPiF;
+        ang_s[i] = v;
+        p.ws[p.s.ang + (b * chunks + c) * C * R + i] = v;
+    }
+    __syncthreads();
+    double* csum = reinterpret_cast<double*>(p.ws + p.s.csum);
+    for (int i = threadIdx.x; i < H * R; i += 256) {
+        const int h = i / R, r = i - h * R;
+        double running = 0.0;
+#pragma unroll 8
+        for (int t = 0; t < C; ++t) running += static_cast<double>(ang_s[t * R + r] * dt_s[h * C + t]);
+        csum[((b * H + h) * chunks + c) * R + r] = running;
+    }
+}
+
+// (window, head, chunk) of a block; as in scan_fused_kernel the heads of one window run on one XCD.
+__device__ __forceinline__ void split_item(const SplitScanArgs& p, int64_t& b, int& h, int& c) {
+    unsigned lin = blockIdx.x;
+    if (gridDim.x % 8 == 0) lin = (lin % 8) * (gridDim.x / 8) + lin / 8;
+    const unsigned chunks = static_cast<unsigned>(p.s.chunks), H = static_cast<unsigned>(p.a.H);
+    c = static_cast<int>(lin % chunks);
+    h = static_cast<int>((lin / chunks) % H);
+    b = lin / chunks / H;
+}
+
+template <int NT>
+__global__ __launch_bounds__(256) void split_chunk_kernel(SplitScanArgs p) {
+    constexpr int C = 32, CT = 2, N = 16 * NT, NTH = 256, NP = N + 4, WP = C + 4, RM = N / 2;
+    __shared__ __attribute__((aligned(16))) float q_sh[C * NP];
+    __shared__ __attribute__((aligned(16))) float k_sh[C * NP];
+    __shared__ __attribute__((aligned(16))) float w_s[(C + 1) * WP];
+    __shared__ float cum_s[C * RM];
+    __shared__ float coef[4][C];
+    __shared__ float sc_s[2][C];
+    int64_t b;
+    int h, c;
+    split_item(p, b, h, c);
+    const ScanArgs& a = p.a;
+    const int R = static_cast<int>(a.R), H = static_cast<int>(a.H), L = static_cast<int>(a.L), st32 = static_cast<int>(a.st);
+    const int c0 = C * c, Lc = L - c0 < C ? L - c0 : C;
+    const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, g = lane >> 4, n_own = tid % N;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int64_t GN = a.G * N;
+    const float* brow = a.proj + b * a.sb + static_cast<int64_t>(c0) * a.st + 2 * H * p.D + (h / (H / static_cast<int>(a.G))) * N;
+    const int64_t bh = b * H + h;
+    float* item = p.ws + (bh * p.s.chunks + c) * p.s.item;
+
+    constexpr int BU = C * N / NTH;
+    float bx[BU], cx[BU];
+#pragma unroll
+    for (int j = 0; j < BU; ++j) {
+        const int t = (tid + NTH * j) / N;
+        const unsigned off = static_cast<unsigned>((t < Lc ? t : Lc - 1) * st32 + n_own);
+        bx[j] = load_off32(brow, off);
+        cx[j] = load_off32(brow + GN, off);
+    }
+    const float bw = a.b_norm_w[n_own], cw = a.c_norm_w[n_own], bb = a.b_bias[h * N + n_own], cb = a.c_bias[h * N + n_own];
+    if (tid < C) {
+        const float4 v = reinterpret_cast<const float4*>(p.ws + p.s.coef)[(bh * p.s.chunks + c) * C + tid];
+        coef[0][tid] = v.x;
+        coef[1][tid] = v.y;
+        coef[2][tid] = v.z;
+        coef[3][tid] = v.w;
+    }
+    for (int i = tid; i < C * R; i += NTH) cum_s[(i / R) * RM + i % R] = p.ws[p.s.ang + (b * p.s.chunks + c) * C * R + i];
+#pragma unroll
+    for (int j = 0; j < BU; ++j) {
+        const int t = (tid + NTH * j) / N;
+        k_sh[t * NP + n_own] = bx[j];
+        q_sh[t * NP + n_own] = cx[j];
+    }
+    __syncthreads();
+    // Norm scales on wave 0, decay weights on wave 1, the running angles on wave 2 (and 3).
+    if (wave == 0) {
+        const bool isb = lane < C;
+        sc_s[isb ? 0 : 1][lane % C] = bc_norm_scale_rows<N>((isb ? k_sh : q_sh) + (lane % C) * NP, isb ? a.b_eps : a.c_eps);
+    }
+    if (wave == 1) decay_walk<C, true>(lane, c == 0, coef, w_s);
+    if (tid >= 128 && tid - 128 < R) {
+        const int r = tid - 128;
+        const double* csum = reinterpret_cast<const double*>(p.ws + p.s.csum) + bh * p.s.chunks * R + r;
+        double running = 0.0;
+#pragma unroll 4
+        for (int i = 0; i < c; ++i) running += csum[i * R];
+#pragma unroll
+        for (int t0 = 0; t0 < C; t0 += 16) {
+            float term[16];
+#pragma unroll
+            for (int i = 0; i < 16; ++i) term[i] = cum_s[(t0 + i) * RM + r] * coef[3][t0 + i];
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                running += static_cast<double>(term[i]);
+                cum_s[(t0 + i) * RM + r] = static_cast<float>(running);
+            }
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < BU; ++j) {
+        const int t = (tid + NTH * j) / N, i = t * NP + n_own;
+        k_sh[i] = (bx[j] * sc_s[0][t]) * bw + bb;
+        q_sh[i] = (cx[j] * sc_s[1][t]) * cw + cb;
+    }
+    __syncthreads();
+    for (int i = tid; i < C * R; i += NTH) {
+        const int t = i / R, r = i - t * R;
+        float sine, cosine;
+        rotation_of(cum_s[t * RM + r], &sine, &cosine);
+        float* qp = q_sh + t * NP + 2 * r;
+        float* kq = k_sh + t * NP + 2 * r;
+        const float ql = qp[0], qr = qp[1], kl = kq[0], kr = kq[1];
+        qp[0] = fmaf(ql, cosine, -(qr * sine));
+        qp[1] = fmaf(ql, sine, qr * cosine);
+        kq[0] = fmaf(kl, cosine, -(kr * sine));
+        kq[1] = fmaf(kl, sine, kr * cosine);
+    }
+    __syncthreads();
+    if (wave < 3) {  // tile pairs (0, 0), (1, 0), (1, 1)
+        const int tt = wave > 0 ? 1 : 0, st = wave > 1 ? 1 : 0;
+        f32x4_t acc = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) {
+            const float4 k4 = *reinterpret_cast<const float4*>(k_sh + (16 * st + li) * NP + 16 * nt + 4 * g);
+            const float4 q4 = *reinterpret_cast<const float4*>(q_sh + (16 * tt + li) * NP + 16 * nt + 4 * g);
+            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(k4.x, q4.x, acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(k4.y, q4.y, acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(k4.z, q4.z, acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(k4.w, q4.w, acc, 0, 0, 0);
+        }
+        const float4 w4 = *reinterpret_cast<const float4*>(w_s + (16 * tt + li) * WP + 16 * st + 4 * g);
+        f32x4_t pv = f32x4_t{w4.x * acc[0], w4.y * acc[1], w4.z * acc[2], w4.w * acc[3]};
+        if (st == tt) {  // W[t][s] is defined for s <= t only
+#pragma unroll
+            for (int v = 0; v < 4; ++v) pv[v] = 4 * g + v <= li ? pv[v] : 0.0f;
+        }
+        reinterpret_cast<f32x4_t*>(item + p.s.P)[wave * 64 + lane] = pv;
+    } else {
+        for (int i = lane; i < 3 * C; i += 64)
+            item[p.s.w + i] = i < C ? w_s[(C - 1) * WP + i] : w_s[(i % C) * WP + (i < 2 * C ? C : C + 1)];
+        for (int i = lane; i < N; i += 64) item[p.s.last + i] = k_sh[(C - 1) * NP + i];
+    }
+    for (int i = tid; i < C * N / 4; i += NTH) {
+        const int t = 4 * i / N, n = 4 * i % N;
+        *reinterpret_cast<float4*>(item + p.s.q + 4 * i) = *reinterpret_cast<const float4*>(q_sh + t * NP + n);
+    }
+    if (c + 1 < p.s.chunks) {
+        for (int i = tid; i < CT * 4 * 64; i += NTH) {
+            const int ln = i & 63, v = (i >> 6) & 3, st = i >> 8;
+            const float* src = k_sh + (16 * st + 4 * (ln >> 4) + v) * NP + (ln & 15);
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt) item[i * NT + nt] = src[16 * nt];
+        }
+    }
+}
+
+// One wave per 16 state columns and NT / NS of their row tiles.
+template <int NT, int NS>
+struct StateChunk {
+    static constexpr int W = NT / NS;
+    typedef float kvec __attribute__((ext_vector_type(W)));
+    kvec k[2][4];
+    f32x4_t kp[W];
+    float4 w[2];
+    float v[2][4], vp, dl, wl;
+};
+
+template <int NT, int DT>
+__global__ __launch_bounds__(64 * DT * (NT > 1 ? 2 : 1)) void split_state_kernel(SplitScanArgs p) {
+    constexpr int C = 32, NS = NT > 1 ? 2 : 1, W = NT / NS;
+    using kvec = typename StateChunk<NT, NS>::kvec;
+    const int lane = threadIdx.x & 63, li = lane & 15, g = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), dt = wave / NS, ns = wave % NS;
+    unsigned bh = blockIdx.x;
+    if (gridDim.x % 8 == 0) bh = (bh % 8) * (gridDim.x / 8) + bh / 8;
+    const ScanArgs& a = p.a;
+    const int64_t b = bh / static_cast<unsigned>(a.H), h = bh % static_cast<unsigned>(a.H);
+    const int chunks = static_cast<int>(p.s.chunks);
+    float* item0 = p.ws + static_cast<int64_t>(bh) * chunks * p.s.item;
+    // Scalar bases per chunk and 32-bit lane offsets: one wave a SIMD issues an instruction every eight cycles, so
+    // address arithmetic is what a step would spend its time on.
+    const float* x0 = a.proj + b * a.sb + a.H * p.D + h * p.D + 16 * dt;
+    const unsigned st32 = static_cast<unsigned>(a.st);
+    unsigned xoff[2][4];
+#pragma unroll
+    for (int st = 0; st < 2; ++st)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) xoff[st][v] = static_cast<unsigned>(16 * st + 4 * g + v) * st32 + li;
+    auto load = [&](int c, StateChunk<NT, NS>& r) {
+        const float* item = item0 + c * p.s.item;
+        const float* x = x0 + static_cast<int64_t>(C) * c * a.st;
+        const float* before = item - (c > 0 ? p.s.item : 0) + p.s.last;  // (the first chunk's are zeros)
+#pragma unroll
+        for (int st = 0; st < 2; ++st) {
+            r.w[st] = *reinterpret_cast<const float4*>(item + p.s.w + 16 * st + 4 * g);
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                r.k[st][v] = *reinterpret_cast<const kvec*>(item + ((st * 4 + v) * 64 + lane) * NT + ns * W);
+                r.v[st][v] = load_off32(x, xoff[st][v]);
+            }
+        }
+        r.dl = item[p.s.w + 2 * C - 1];
+        r.wl = item[p.s.w + 3 * C - 1];
+        r.vp = load_off32(c > 0 ? x - a.st : x, li);
+#pragma unroll
+        for (int nt = 0; nt < W; ++nt) r.kp[nt] = *reinterpret_cast<const f32x4_t*>(before + 16 * (ns * W + nt) + 4 * g);
+        if (c == 0) {
+            r.vp = 0.0f;
+#pragma unroll
+            for (int nt = 0; nt < W; ++nt) r.kp[nt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        }
+    };
+    f32x4_t S[W];
+#pragma unroll
+    for (int nt = 0; nt < W; ++nt) S[nt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    auto step = [&](int c, const StateChunk<NT, NS>& r) {
+#pragma unroll
+        for (int nt = 0; nt < W; ++nt)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) S[nt][v] = fmaf(r.wl * r.kp[nt][v], r.vp, S[nt][v] * r.dl);
+#pragma unroll
+        for (int st = 0; st < 2; ++st) {
+            const float w[4] = {r.w[st].x, r.w[st].y, r.w[st].z, r.w[st].w};
+#pragma unroll
+            for (int v = 0; v < 4; ++v)
+#pragma unroll
+                for (int nt = 0; nt < W; ++nt)
+                    S[nt] = __builtin_amdgcn_mfma_f32_16x16x4f32(r.k[st][v][nt], w[v] * r.v[st][v], S[nt], 0, 0, 0);
+        }
+#pragma unroll
+        for (int nt = 0; nt < W; ++nt)
+            reinterpret_cast<f32x4_t*>(item0 + (c + 1) * p.s.item + p.s.S)[(dt * NT + ns * W + nt) * 64 + lane] = S[nt];
+    };
+    // The next chunk's loads in flight, in buffers that the unrolled steps name at compile time (chunks past the end
+    // load the last one again and are not used); three chunks ahead was no faster.
+    constexpr int kAhead = 1;
+    StateChunk<NT, NS> buf[kAhead + 1];
+    const int n = chunks - 1;
+#pragma unroll
+    for (int i = 0; i < kAhead; ++i) load(i < n ? i : n - 1, buf[i]);
+    for (int c = 0; c < n; c += kAhead + 1) {
+#pragma unroll
+        for (int i = 0; i <= kAhead; ++i) {
+            load(c + i + kAhead < n ? c + i + kAhead : n - 1, buf[(i + kAhead) % (kAhead + 1)]);
+            if (c + i < n) step(c + i, buf[i]);
+        }
+    }
+}
+
+template <int NT, int DT>
+__global__ __launch_bounds__(64 * DT) void split_out_kernel(SplitScanArgs p) {
+    constexpr int C = 32, CT = 2, N = 16 * NT, D = 16 * DT;
+    __shared__ float ck_s[C];
+    int64_t b;
+    int h, c;
+    split_item(p, b, h, c);
+    const ScanArgs& a = p.a;
+    const int lane = threadIdx.x & 63, li = lane & 15, g = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), col = 16 * wave + li;
+    const int c0 = C * c, L = static_cast<int>(a.L), Lc = L - c0 < C ? L - c0 : C;
+    const bool first = c == 0;
+    const int64_t d_inner = a.H * D;
+    const float* item = p.ws + ((b * a.H + h) * p.s.chunks + c) * p.s.item;
+    const float* xc = a.proj + b * a.sb + static_cast<int64_t>(c0) * a.st + d_inner + h * D + col;
+    const float* zc = a.gate + b * a.gsb + static_cast<int64_t>(c0) * a.gst + h * D + col;
+    const int st32 = static_cast<int>(a.st), gst32 = static_cast<int>(a.gst);
+    float vx[CT][4], zx[CT][4];
+#pragma unroll
+    for (int st = 0; st < CT; ++st)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const int t = 16 * st + 4 * g + v, tc = t < Lc ? t : Lc - 1;
+            vx[st][v] = load_off32(xc, static_cast<unsigned>(tc * st32));
+            zx[st][v] = load_off32(zc, static_cast<unsigned>(tc * gst32));
+        }
+    const float vp = first ? 0.0f : xc[-a.st];
+    f32x4_t P[3], S[NT], qf[CT][NT];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) P[i] = reinterpret_cast<const f32x4_t*>(item + p.s.P)[i * 64 + lane];
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) {
+        // (the first chunk has no state before it: its slot is not written, and not read)
+        S[nt] = first ? f32x4_t{0.f, 0.f, 0.f, 0.f} : reinterpret_cast<const f32x4_t*>(item + p.s.S)[(wave * NT + nt) * 64 + lane];
+#pragma unroll
+        for (int tt = 0; tt < CT; ++tt)
+            qf[tt][nt] = *reinterpret_cast<const f32x4_t*>(item + p.s.q + (16 * tt + li) * N + 16 * nt + 4 * g);
+    }
+    float din[CT][4];
+#pragma unroll
+    for (int tt = 0; tt < CT; ++tt)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) din[tt][v] = item[p.s.w + C + 16 * tt + 4 * g + v];
+    if (!first && wave == DT - 1 && lane < C) {
+        const float* q = item + p.s.q + lane * N;
+        const float* kp = item - p.s.item + p.s.last;
+        float dot = 0.0f;
+#pragma unroll
+        for (int n = 0; n < N; ++n) dot = fmaf(q[n], kp[n], dot);
+        ck_s[lane] = dot * item[p.s.w + 2 * C + lane];
+    }
+    double gz[CT][4];
+#pragma unroll
+    for (int tt = 0; tt < CT; ++tt)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const double z = static_cast<double>(zx[tt][v]);
+            const double sz = silu_d(z);
+            gz[tt][v] = a.gate_logits ? sz : z;
+        }
+    const float skip = a.skip[h];
+    __syncthreads();
+    float* ochunk = a.out + (b * a.L + c0) * d_inner + h * D + col;
+#pragma unroll
+    for (int tt = 0; tt < CT; ++tt) {
+        if (16 * tt >= Lc) continue;
+        f32x4_t Y = f32x4_t{0.f, 0.f, 0.f, 0.f}, Yi = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int st = 0; st <= tt; ++st)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) Y = __builtin_amdgcn_mfma_f32_16x16x4f32(P[tt + st][v], vx[st][v], Y, 0, 0, 0);
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) Yi = __builtin_amdgcn_mfma_f32_16x16x4f32(qf[tt][nt][v], S[nt][v], Yi, 0, 0, 0);
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const int t = 16 * tt + 4 * g + v;
+            const float yc = first ? 0.0f : fmaf(ck_s[t], vp, fmaf(din[tt][v], Yi[v], Y[v]));
+            float y = first ? Y[v] : yc;
+            y = fmaf(skip, vx[tt][v], y);
+            const float o = static_cast<float>(static_cast<double>(y) * gz[tt][v]);
+            if (t < Lc) store_off32(ochunk, static_cast<unsigned>(t) * static_cast<unsigned>(d_inner), o);
+        }
+    }
+}
+
+// Whether the chunk-parallel form takes the call. With at most 128 pairs (half of the CUs one block each) it wins
+// from four chunks on; at three the launches it adds eat the gain (8 pairs x 96 tokens: 20 against 26 us on the
+// device, and 4 us more on the host). Up to 256 pairs the fused blocks still have a CU each and its extra traffic
+// (73 KB an item at d_state and headdim 64) only pays over many chunks: 192 pairs x 480 tokens 95 against 124 us,
+// 256 pairs x 480 116 against 124, but 256 x 256 70 against 69 and 192 x 96 30 against 27.
+bool split_scan_shape(int64_t B, int64_t L, int64_t H) {
+    const int64_t pairs = B * H, chunks = (L + 31) / 32;
+    return (pairs <= 128 && chunks >= 4) || (pairs <= 256 && chunks >= 12);
+}
+
+bool launch_scan_split(const ScanArgs& s, int64_t N, int64_t D, void* workspace, size_t bytes, hipStream_t stream) {
+    const SplitScan layout = split_layout(s.B, s.L, s.H, N, D, s.R);
+    if (!split_scan_shape(s.B, s.L, s.H) || bytes < sizeof(float) * static_cast<size_t>(layout.total) || !aligned16(workspace))
+        return false;
+    const SplitScanArgs p{s, static_cast<float*>(workspace), layout, N, D};
+    const unsigned pairs = static_cast<unsigned>(s.B * s.H), items = pairs * static_cast<unsigned>(layout.chunks);
+    const size_t token_lds = sizeof(float) * 32 * static_cast<size_t>(s.H + s.R);
+    if (token_lds > 64 * 1024) return false;
+    const int NT = static_cast<int>(N / 16), DT = static_cast<int>(D / 16);
+#define MLK_SPLIT(NTV, DTV)                                                                                                  \
+    if (NT == NTV && DT == DTV) {                                                                                            \
+        hipLaunchKernelGGL(split_token_kernel, dim3(static_cast<unsigned>(s.B * layout.chunks)), dim3(256), token_lds, stream, p); \
+        hipLaunchKernelGGL((split_chunk_kernel<NTV>), dim3(items), dim3(256), 0, stream, p);                                 \
+        hipLaunchKernelGGL((split_state_kernel<NTV, DTV>), dim3(pairs), dim3(64 * DTV * (NTV > 1 ? 2 : 1)), 0, stream, p);   \
+        hipLaunchKernelGGL((split_out_kernel<NTV, DTV>), dim3(items), dim3(64 * DTV), 0, stream, p);                         \
+        return true;                                                                                                         \
+    }
+    MLK_SPLIT(1, 1) MLK_SPLIT(1, 2) MLK_SPLIT(1, 4) MLK_SPLIT(2, 1) MLK_SPLIT(2, 2) MLK_SPLIT(2, 4)
+    MLK_SPLIT(4, 1) MLK_SPLIT(4, 2) MLK_SPLIT(4, 4)
+#undef MLK_SPLIT
+    return false;
+}
+
+// ---------------------------------------------------------------------------
 // The RMSNorm -> Mamba-3 block: GroupedRMSNorm + in_proj + scan in one kernel
 // ---------------------------------------------------------------------------
 //
@@ -2302,11 +2758,21 @@ using namespace mlk;
 
 extern "C" {
 
-size_t mlk_mamba3_workspace_bytes(int64_t batch, int64_t length, int64_t nheads, int64_t d_state,
-                                  int64_t num_rope_angles) {
+// What the unfused kernels need; a call with only this much takes the fused scan.
+static size_t scan_workspace_bytes(int64_t batch, int64_t length, int64_t nheads, int64_t d_state, int64_t num_rope_angles) {
     const int64_t blh = batch * length * nheads;
     const int64_t rw = num_rope_angles > 0 ? num_rope_angles : 1;
     return sizeof(float) * static_cast<size_t>(2 * blh * d_state + 3 * blh + blh * rw);
+}
+
+size_t mlk_mamba3_workspace_bytes(int64_t batch, int64_t length, int64_t nheads, int64_t d_state,
+                                  int64_t num_rope_angles) {
+    size_t bytes = scan_workspace_bytes(batch, length, nheads, d_state, num_rope_angles);
+    if (batch * length * nheads > 0 && d_state <= 64 && mlk::split_scan_shape(batch, length, nheads)) {  // (headdim at most 64 there)
+        const size_t split = sizeof(float) * static_cast<size_t>(mlk::split_layout(batch, length, nheads, d_state, 64, num_rope_angles).total);
+        bytes = split > bytes ? split : bytes;
+    }
+    return bytes;
 }
 
 }  // extern "C"
@@ -2512,7 +2978,7 @@ mlk_status mlk_mamba3_siso_forward(const float* projected, int64_t batch, int64_
                   std::to_string(expected));
         return MLK_ERR_INVALID_ARGUMENT;
     }
-    MLK_CHECK(workspace_bytes >= mlk_mamba3_workspace_bytes(batch, length, nheads, d_state, num_rope_angles),
+    MLK_CHECK(workspace_bytes >= scan_workspace_bytes(batch, length, nheads, d_state, num_rope_angles),
               "workspace too small");
     const int64_t blh = batch * length * nheads;
     if (blh == 0) return MLK_OK;
@@ -2554,6 +3020,7 @@ mlk_status mlk_mamba3_siso_forward(const float* projected, int64_t batch, int64_
             s.gate_logits = 0;
         }
         s.out = out;
+        if (launch_scan_split(s, d_state, headdim, workspace, workspace_bytes, stream)) return launch_status("mamba3 split scan");
         if (launch_scan_fused(s, d_state, headdim, stream)) return launch_status("mamba3 fused scan");
     }
     const int64_t rw = num_rope_angles > 0 ? num_rope_angles : 1;

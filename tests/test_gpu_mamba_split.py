@@ -1,0 +1,70 @@
+"""The Mamba-3 scan with its chunks in parallel (few window x head pairs): the unfused prep -> rotate -> chunked
+recurrence bit for bit, at the edges of the rule that chooses it, of a chunk and of the layouts."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from helpers import assert_bitwise, assert_close
+from test_gpu_mamba import _random_layer, _t
+
+pytestmark = pytest.mark.gpu
+
+_KEYS = ("b_bias", "c_bias", "b_norm_w", "c_norm_w", "dt_bias", "skip")
+
+
+def _case(dev, B, L, N, G, H, D, R):
+    proj, p = _random_layer(np.random.default_rng(B + L + N + D), B, L, N, G, H, D, R)
+    return _t(proj, dev), [_t(p[k], dev) for k in _KEYS], (N, G, H, D, R, 1e-5, 1e-5, 1e-4)
+
+
+@pytest.mark.parametrize("B,L,N,G,H,D,R", [(1, 97, 64, 1, 8, 64, 16), (16, 128, 64, 1, 8, 64, 17), (2, 129, 32, 2, 4, 32, 0),
+                                           (3, 480, 16, 1, 4, 32, 4), (1, 500, 64, 1, 1, 64, 32), (7, 161, 16, 3, 6, 64, 8),
+                                           (32, 353, 64, 1, 8, 64, 16), (5, 255, 32, 1, 5, 64, 9), (4, 130, 64, 1, 2, 32, 16)])
+def test_chunk_parallel_scan_equals_unfused(dev, monkeypatch, B, L, N, G, H, D, R):
+    from montlok import _C
+
+    proj, params, geo = _case(dev, B, L, N, G, H, D, R)
+    wide = torch.randn(B, L, proj.shape[-1] + 12, device=dev)
+    wide[..., :proj.shape[-1]] = proj
+    z = proj[..., :H * D].double()
+    gate = (z * torch.sigmoid(z)).float()
+    got = _C.mamba3_siso_forward(proj, None, *params, *geo)
+    strided = _C.mamba3_siso_forward(wide[..., :proj.shape[-1]], None, *params, *geo)
+    gated = _C.mamba3_siso_forward(proj, gate, *params, *geo)
+    monkeypatch.setenv("MLK_MAMBA3_SCAN", "unfused")
+    expect = _C.mamba3_siso_forward(proj, None, *params, *geo).cpu().numpy()
+    assert_bitwise(got, expect, "chunk-parallel vs unfused")
+    assert_bitwise(strided, expect, "strided rows")
+    assert_bitwise(gated, _C.mamba3_siso_forward(proj, gate, *params, *geo).cpu().numpy(), "explicit gate")
+
+
+@pytest.mark.parametrize("B,L,N,G,H,R", [(2, 200, 64, 1, 4, 16), (1, 97, 16, 2, 4, 8)])
+def test_chunk_parallel_scan_headdim16(dev, oracle, monkeypatch, B, L, N, G, H, R):
+    from montlok import _C
+
+    proj, params, geo = _case(dev, B, L, N, G, H, 16, R)
+    got = _C.mamba3_siso_forward(proj, None, *params, *geo)
+    monkeypatch.setenv("MLK_MAMBA3_SCAN", "sequential")
+    assert_close(got, _C.mamba3_siso_forward(proj, None, *params, *geo), tol=1e-6, name="vs sequential")
+
+
+def test_smaller_workspace_takes_the_fused_scan(dev):
+    """A caller that holds only the unfused kernels' slab is served as before, with the same result."""
+    from montlok import _C
+
+    B, L, N, G, H, D, R = 2, 300, 64, 1, 8, 64, 16
+    proj, params, geo = _case(dev, B, L, N, G, H, D, R)
+    expect = _C.mamba3_siso_forward(proj, None, *params, *geo)
+    lib = _C.library()
+    slab = 4 * (2 * B * L * H * N + 3 * B * L * H + B * L * H * R)
+    assert lib.mlk_mamba3_workspace_bytes(B, L, H, N, R) > slab
+    ws = torch.empty(slab, dtype=torch.uint8, device=dev)
+    out = torch.full((B, L, H * D), float("nan"), device=dev)
+    status = lib.mlk_mamba3_siso_forward(proj.data_ptr(), B, L, proj.shape[-1], proj.stride(0), proj.stride(1), None, 0, 0,
+                                         *(t.data_ptr() for t in params), N, G, H, D, R, 1e-5, 1e-5, 1e-4, out.data_ptr(),
+                                         ws.data_ptr(), slab, torch.cuda.current_stream().cuda_stream)
+    assert status == 0
+    assert torch.equal(out, expect)
