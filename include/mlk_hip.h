@@ -148,6 +148,18 @@ mlk_status mlk_rms_norm_linear(const float* x, int64_t rows, int64_t in_features
                                int32_t weight_dtype, const float* bias, int64_t out_features, float* out,
                                int64_t out_stride, mlk_stream_t stream);
 
+/* linear then swiglu (montlok.cpp:967-976 without its second linear): out
+ * [rows, hidden] = silu(g) * u, [g | u] = x W^T + bias, W [2 * hidden, K] and
+ * bias [2 * hidden] or NULL, in one launch without the [rows, 2 * hidden]
+ * intermediate; the linear's values as mlk_linear forms them, silu(g) * u in
+ * double, rounded once. Built for fp32 weights where mlk_linear to 2 * hidden
+ * columns takes its three-plane form (K above 128, 16-byte aligned rows of x
+ * and W, more than a few hundred rows); MLK_ERR_UNSUPPORTED otherwise, and the
+ * caller runs the two operators. */
+mlk_status mlk_linear_swiglu(const float* x, int64_t rows, int64_t in_features, int64_t x_stride, const void* weight,
+                             int32_t weight_dtype, const float* bias, int64_t hidden, float* out, int64_t out_stride,
+                             mlk_stream_t stream);
+
 /* ----------------------------------------------------------------- MLA -- */
 
 /* mla_rope_qk(q, kv, k_rope, cos, sin, nope_dim) -- montlok.cpp:1093-1154,

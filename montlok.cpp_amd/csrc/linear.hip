@@ -1648,3 +1648,25 @@ extern "C" mlk_status mlk_rms_norm_linear(const float* x, int64_t rows, int64_t 
 #undef MLK_NORM_GS
     return launch_status("rms_norm_linear");
 }
+
+extern "C" mlk_status mlk_linear_swiglu(const float* x, int64_t rows, int64_t in_features, int64_t x_stride, const void* weight,
+                                        int32_t weight_dtype, const float* bias, int64_t hidden, float* out, int64_t out_stride,
+                                        mlk_stream_t stream) {
+    MLK_CHECK(rows >= 0 && in_features > 0 && hidden > 0, "invalid linear geometry");
+    MLK_CHECK(x_stride >= in_features, "x row stride must be at least in_features");
+    MLK_CHECK(out_stride >= hidden, "out row stride must be at least hidden");
+    MLK_CHECK(weight_dtype == MLK_DTYPE_F32 || weight_dtype == MLK_DTYPE_BF16, "weight dtype must be f32 or bf16");
+    LinearArgs p{x, rows, in_features, x_stride, weight, bias, hidden, out, out_stride};
+    // The shapes whose linear to 2 hidden columns takes the three-plane form.
+    LinearArgs wide = p;
+    wide.N = 2 * hidden;
+    const bool vec = aligned16(x) && x_stride % 4 == 0 && aligned16(weight) && in_features % 4 == 0;
+    if (weight_dtype != MLK_DTYPE_F32 || !vec || small_split_shape(wide) || !split_shape(wide) || !linear_swiglu_fits(p)) {
+        set_error("linear_swiglu: shape without the fused form (use linear then swiglu)");
+        return MLK_ERR_UNSUPPORTED;
+    }
+    if (rows == 0) return MLK_OK;
+    MLK_CHECK(x && weight && out, "null tensor pointer");
+    launch_linear_swiglu(p, reinterpret_cast<hipStream_t>(stream));
+    return launch_status("linear_swiglu");
+}

@@ -27,9 +27,11 @@ struct LinearArgs {
 
 // The fp32-weight linear on the bf16 matrix cores (linear_split.hip), for 16-byte aligned rows of x and W.
 // _fits: whether its addressing holds the call. _norm: with the grouped RMSNorm of x (group sizes 8, 16, 32, 64;
-// K at most 256).
+// K at most 256). _swiglu: W and bias hold 2 N rows, gate then up; out [rows, N] = silu(gate) * up.
 bool linear_split_fits(const LinearArgs& p);
 void launch_linear_split(const LinearArgs& p, hipStream_t stream);
 void launch_linear_split_norm(const LinearArgs& p, int64_t group_size, hipStream_t stream);
+bool linear_swiglu_fits(const LinearArgs& p);
+void launch_linear_swiglu(const LinearArgs& p, hipStream_t stream);
 
 }  // namespace mlk

@@ -92,7 +92,8 @@ __device__ __forceinline__ void norm_scales(const LinearArgs& p, int64_t row0, i
 // FULL: K a multiple of the step. GS > 0: the grouped RMSNorm of x (groups of GS floats, at most kMaxNormGroups
 // of them) applied to the staged values, bit for bit rms_norm then this kernel. SWIGLU: W holds 2 N rows, gate
 // then up; a wave's W tile is 16 gate rows and the 16 up rows of the same columns, so that a lane holds both
-// of its outputs' factors, and out = silu(gate) * up in fp64, rounded once (p.N = hidden columns of out).
+// of its outputs' factors, and out = silu(gate) * up in fp64, rounded once (p.N = hidden columns of out). The
+// 2 N columns then never reach memory: 7680 x 256 -> 2 x 512 36 us, against 38 for the linear and 13 for swiglu.
 template <bool FULL, int GS, bool SWIGLU>
 __global__ __launch_bounds__(256) void linear_split_kernel(LinearArgs p, unsigned n_blocks) {
     constexpr int kCols = SWIGLU ? kBlock / 2 : kBlock;  // output columns of the block
@@ -274,7 +275,7 @@ void launch(const LinearArgs& p, hipStream_t stream) {
 
 // 32-bit byte offsets from a block's first rows, and the grid.
 bool fits(const LinearArgs& p, int64_t w_rows) {
-    return p.K % 4 == 0 && p.x_stride < (int64_t{1} << 23) && p.K * w_rows < (int64_t{1} << 30) &&
+    return p.K % 4 == 0 && p.x_stride < (int64_t{1} << 23) && p.K * (w_rows + kBlock) < (int64_t{1} << 30) &&
            ceil_div(p.rows, kBlock) * ceil_div(p.N, kBlock / 2) < (int64_t{1} << 31);
 }
 
@@ -292,5 +293,9 @@ void launch_linear_split_norm(const LinearArgs& p, int64_t group_size, hipStream
         default: launch<64, false>(p, stream); break;
     }
 }
+
+bool linear_swiglu_fits(const LinearArgs& p) { return fits(p, 2 * p.N); }
+
+void launch_linear_swiglu(const LinearArgs& p, hipStream_t stream) { launch<0, true>(p, stream); }
 
 }  // namespace mlk

@@ -34,7 +34,7 @@ using OptTensor = std::optional<Tensor>;
 
 #define MLK_FUNCTIONS(X)                                                                                           \
     X(mlk_last_error) X(mlk_rms_norm) X(mlk_add_rms_norm) X(mlk_layer_norm) X(mlk_swiglu) X(mlk_linear)            \
-    X(mlk_linear_residual) X(mlk_rms_norm_linear) X(mlk_mhc_prepare) X(mlk_mhc_combine) X(mlk_mhc_combine_prepare) \
+    X(mlk_linear_residual) X(mlk_rms_norm_linear) X(mlk_linear_swiglu) X(mlk_mhc_prepare) X(mlk_mhc_combine) X(mlk_mhc_combine_prepare) \
     X(mlk_mamba3_workspace_bytes) X(mlk_mamba3_siso_forward) X(mlk_mamba3_siso_step)                               \
     X(mlk_rms_norm_mamba3_forward) X(mlk_mla_rope_qk) X(mlk_attention)
 
@@ -213,6 +213,23 @@ OptTensor rms_norm_linear(const OptTensor& x_, const OptTensor& norm_weight, dou
     const Tensor out = empty(with_last(x, n), x);
     const mlk_status status = lib.mlk_rms_norm_linear(data(r.t), r.count, k, r.stride, data(nw), eps, groups, w.const_data_ptr(),
                                                       dtype_of(w), data(b), n, out_data(out), n, stream());
+    if (status == MLK_ERR_UNSUPPORTED) return std::nullopt;
+    done(status);
+    return out;
+}
+
+// swiglu(linear(input, weight, bias)); None where the shape has no fused form.
+OptTensor linear_swiglu(const OptTensor& input, const OptTensor& weight, const OptTensor& bias) {
+    const Tensor& x = f32_gpu(input, "input");
+    const Tensor w = weight_of(weight);
+    const int64_t n = w.size(0), k = w.size(1);
+    REQUIRE(x.dim() >= 1 && x.size(-1) == k, "input must end in in_features=" + std::to_string(k));
+    const OptTensor b = dense_or_none(bias, n, "bias");
+    REQUIRE(n % 2 == 0, "x must end in an even dimension [gate | up]");
+    const Rows r = rows_of(x, k);
+    const Tensor out = empty(with_last(x, n / 2), x);
+    const mlk_status status = lib.mlk_linear_swiglu(data(r.t), r.count, k, r.stride, w.const_data_ptr(), dtype_of(w), data(b), n / 2,
+                                                    out_data(out), n / 2, stream());
     if (status == MLK_ERR_UNSUPPORTED) return std::nullopt;
     done(status);
     return out;
@@ -523,6 +540,7 @@ PYBIND11_MODULE(_torch_ops, m) {
     m.def("linear", &linear);
     m.def("linear_residual", &linear_residual);
     m.def("rms_norm_linear", &rms_norm_linear);
+    m.def("linear_swiglu", &linear_swiglu);
     m.def("mhc_prepare", &mhc_prepare);
     m.def("mhc_combine", &mhc_combine);
     m.def("mhc_combine_prepare", &mhc_combine_prepare);

@@ -48,6 +48,7 @@ def _load():
         "mlk_linear": [_vp, _i64, _i64, _i64, _vp, C.c_int32, _vp, _i64, _vp, _i64, _vp],
         "mlk_linear_residual": [_vp, _i64, _i64, _i64, _vp, C.c_int32, _vp, _i64, _vp, _i64, _vp, _i64, _vp],
         "mlk_rms_norm_linear": [_vp, _i64, _i64, _i64, _vp, _dbl, _i64, _vp, C.c_int32, _vp, _i64, _vp, _i64, _vp],
+        "mlk_linear_swiglu": [_vp, _i64, _i64, _i64, _vp, C.c_int32, _vp, _i64, _vp, _i64, _vp],
         "mlk_layer_norm_bf16": [_vp, _i64, _i64, _i64, _vp, _vp, _dbl, _vp, _vp],
         "mlk_mla_attend_normed": [_vp, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _vp, _vp, _vp, _vp, _dbl,
                                   _vp, _vp],
@@ -227,8 +228,12 @@ def rms_norm_linear(x: torch.Tensor, norm_weight: torch.Tensor, eps: float, grou
 
 
 def swiglu_mlp(input, in_weight, in_bias=None, out_weight=None, out_bias=None):
-    """montlok.cpp:967-976: linear -> swiglu -> linear."""
-    return linear(swiglu(linear(input, in_weight, in_bias)), out_weight, out_bias)
+    """montlok.cpp:967-976: linear -> swiglu -> linear, the first two in one launch where that is built (fp32
+    weights, more than a few hundred rows)."""
+    hidden = (_native or _ops()).linear_swiglu(input, in_weight, in_bias)
+    if hidden is None:
+        hidden = swiglu(linear(input, in_weight, in_bias))
+    return linear(hidden, out_weight, out_bias)
 
 
 # ------------------------------------------------------------------ mHC
@@ -887,7 +892,7 @@ def exported_symbols() -> list[str]:
             "mlk_layer_norm", "mlk_swiglu", "mlk_mhc_prepare", "mlk_mhc_combine", "mlk_mhc_combine_prepare",
             "mlk_math_check", "mlk_mamba3_workspace_bytes", "mlk_mamba3_siso_recurrent",
             "mlk_mamba3_siso_recurrent_noalloc", "mlk_mamba3_siso_forward", "mlk_rms_norm_mamba3_forward",
-            "mlk_mamba3_siso_step", "mlk_linear", "mlk_linear_residual", "mlk_rms_norm_linear",
+            "mlk_mamba3_siso_step", "mlk_linear", "mlk_linear_residual", "mlk_rms_norm_linear", "mlk_linear_swiglu",
             "mlk_layer_norm_bf16", "mlk_mla_rope_qk", "mlk_attention", "mlk_mla_attend", "mlk_mla_attend_normed",
             "mlk_mla_forward", "mlk_mla_packed_elems", "mlk_mla_pack_weights", "mlk_mla_forward_packed"]
 
