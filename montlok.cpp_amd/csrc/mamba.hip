@@ -1997,12 +1997,12 @@ __global__ __launch_bounds__(64 * DT) void split_out_kernel(SplitScanArgs p) {
 
 // Whether the chunk-parallel form takes the call. With at most 128 pairs (half of the CUs one block each) it wins
 // from four chunks on; at three the launches it adds eat the gain (8 pairs x 96 tokens: 20 against 26 us on the
-// device, and 4 us more on the host). Up to 256 pairs the fused blocks still have a CU each and its extra traffic
-// (73 KB an item at d_state and headdim 64) only pays over many chunks: 192 pairs x 480 tokens 95 against 124 us,
-// 256 pairs x 480 116 against 124, but 256 x 256 70 against 69 and 192 x 96 30 against 27.
+// device, and 4 us more on the host). Up to 192 pairs (the fused blocks then have a CU each, and the workspace's
+// traffic, 73 KB an item at d_state and headdim 64, counts) it wins over many chunks only: 192 pairs x 480 tokens
+// 95 against 124 us, 192 x 96 30 against 27; with 256 pairs x 480 the two are even (131 and 126 us in the model).
 bool split_scan_shape(int64_t B, int64_t L, int64_t H) {
     const int64_t pairs = B * H, chunks = (L + 31) / 32;
-    return (pairs <= 128 && chunks >= 4) || (pairs <= 256 && chunks >= 12);
+    return (pairs <= 128 && chunks >= 4) || (pairs <= 192 && chunks >= 12);
 }
 
 bool launch_scan_split(const ScanArgs& s, int64_t N, int64_t D, void* workspace, size_t bytes, hipStream_t stream) {

@@ -22,7 +22,7 @@ def _case(dev, B, L, N, G, H, D, R):
 
 @pytest.mark.parametrize("B,L,N,G,H,D,R", [(1, 97, 64, 1, 8, 64, 16), (16, 128, 64, 1, 8, 64, 17), (2, 129, 32, 2, 4, 32, 0),
                                            (3, 480, 16, 1, 4, 32, 4), (1, 500, 64, 1, 1, 64, 32), (7, 161, 16, 3, 6, 64, 8),
-                                           (32, 353, 64, 1, 8, 64, 16), (5, 255, 32, 1, 5, 64, 9), (4, 130, 64, 1, 2, 32, 16)])
+                                           (24, 353, 64, 1, 8, 64, 16), (5, 255, 32, 1, 5, 64, 9), (4, 130, 64, 1, 2, 32, 16)])
 def test_chunk_parallel_scan_equals_unfused(dev, monkeypatch, B, L, N, G, H, D, R):
     from montlok import _C
 
