@@ -367,6 +367,188 @@ __global__ __launch_bounds__(256) void attn_kernel(AttnArgs p) {
     }
 }
 
+// fp32 attention with the keys of a query tile split over a block's four waves,
+// no operand in LDS: block = QT tiles of 16 queries of one (window, head); wave w
+// takes the 32-key chunks w, w + 4, ... of the keys the tiles see, with a
+// running max, sum and output of its own, and the four meet in LDS at the end.
+//
+//   S^T = K Q^T   lane (g, l): key l of a 16-key tile, 8 head dims (32 c + 8 g)
+//                 straight from the row, and query l likewise; the products'
+//                 lane holds query l, keys 4 g .. + 3 of a tile.
+//   O^T = V^T P^T row r of output tile t is head dim OT r + t (OT = HD / 16), so
+//                 that a lane's OT operands of one key are OT consecutive floats
+//                 of its row (one 16-byte load at HD 64, 4 whole rows an
+//                 instruction), and the lane ends with 4 OT consecutive outputs.
+//
+// 128-query blocks with K and V^T staged in LDS (attn_kernel) walk up to 15 of those chunks one after another and
+// leave a small batch most of the chip idle: 480 keys, 4 heads of 64: 1 window 50 -> 10.5 us, its last query
+// alone 32 -> 10, 16 windows 58 -> 40, 64 windows 165 -> 113 (the products alone need 51). What bounds it with many windows is the rows' way from L2 to the registers, 16 KB a chunk.
+template <int HD, int QT>
+__global__ __launch_bounds__(256) void attn_split_kernel(AttnArgs p, unsigned q_blocks) {
+    constexpr int HC = HD / 32, OT = HD / 16, KC = 32;
+    typedef float vvec __attribute__((ext_vector_type(OT)));
+    __shared__ float part_s[4][QT][4 * OT + 2][64];
+    const int lane = threadIdx.x & 63, li = lane & 15, g = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    // The blocks of one (window, head) on one XCD, the longest rows first.
+    unsigned lin = blockIdx.x;
+    if (gridDim.x % 8 == 0) lin = (lin % 8) * (gridDim.x / 8) + lin / 8;
+    const unsigned bh = lin / q_blocks, H = static_cast<unsigned>(p.heads);
+    const int64_t b = bh / H, h = bh % H;
+    const int q0 = static_cast<int>(q_blocks - 1 - lin % q_blocks) * (16 * QT);
+    const int Lq = static_cast<int>(p.q_length), Lk = static_cast<int>(p.kv_length);
+    const float* kh = p.k + b * p.kv_length * p.k_ts + h * p.k_hs;
+    const float* vh = p.v + b * p.kv_length * p.v_ts + h * p.v_hs;
+
+    float qf[QT][HC][8];
+    float m_run[QT], l_run[QT];
+    f32x4 acc[QT][OT];
+#pragma unroll
+    for (int i = 0; i < QT; ++i) {
+        const int qi = q0 + 16 * i + li;
+        const float* row = p.q + (b * p.q_length + (qi < Lq ? qi : Lq - 1)) * p.q_ts + h * p.q_hs;
+#pragma unroll
+        for (int c = 0; c < HC; ++c) load_row8(row, 32 * c + 8 * g, HD, true, true, qf[i][c]);
+        m_run[i] = -INFINITY;
+        l_run[i] = 0.0f;
+#pragma unroll
+        for (int t = 0; t < OT; ++t) acc[i][t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+    const int64_t last = q0 + 16 * QT - 1 < Lq ? q0 + 16 * QT - 1 : Lq - 1;
+    const int key_end = static_cast<int>(last + p.offset + 1 < p.kv_length ? last + p.offset + 1 : p.kv_length);
+
+    for (int kbase = KC * wave; kbase < key_end; kbase += 4 * KC) {
+        // Keys past the end read the last one; their weights are zero.
+        float kf[2][HC][8];
+        vvec vf[2][4];
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            const int key = kbase + 16 * t + li;
+            const float* row = kh + static_cast<int64_t>(key < Lk ? key : Lk - 1) * p.k_ts;
+#pragma unroll
+            for (int c = 0; c < HC; ++c) load_row8(row, 32 * c + 8 * g, HD, true, true, kf[t][c]);
+        }
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const int key = kbase + 16 * t + 4 * g + v;
+                vf[t][v] = *reinterpret_cast<const vvec*>(vh + static_cast<int64_t>(key < Lk ? key : Lk - 1) * p.v_ts + OT * li);
+            }
+#pragma unroll
+        for (int i = 0; i < QT; ++i) {
+            if (kbase > q0 + 16 * i + 15 + p.offset) continue;  // chunk fully masked for the tile
+            f32x4 s[2];
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                s[t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                for (int c = 0; c < HC; ++c)
+#pragma unroll
+                    for (int j = 0; j < 8; ++j)
+                        s[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[t][c][j], qf[i][c][j], s[t], 0, 0, 0);
+            }
+            const int64_t see = q0 + 16 * i + li + p.offset;  // the query's last visible key
+            float mx = -INFINITY;
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    const int key = kbase + 16 * t + 4 * g + v;
+                    s[t][v] = key < Lk && key <= see ? s[t][v] * p.scale_log2 : -INFINITY;
+                    mx = fmaxf(mx, s[t][v]);
+                }
+            mx = fmaxf(mx, lane_xor16(mx));
+            mx = fmaxf(mx, lane_xor32(mx));
+            const float m_new = fmaxf(m_run[i], mx);
+            const float m_use = m_new == -INFINITY ? 0.0f : m_new;
+            const float corr = __builtin_amdgcn_exp2f(m_run[i] - m_use);
+            m_run[i] = m_new;
+            float sum = 0.0f;
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    s[t][v] = __builtin_amdgcn_exp2f(s[t][v] - m_use);
+                    sum += s[t][v];
+                }
+            l_run[i] = l_run[i] * corr + sum;
+#pragma unroll
+            for (int t = 0; t < OT; ++t) acc[i][t] *= corr;
+#pragma unroll
+            for (int u = 0; u < 2; ++u)
+#pragma unroll
+                for (int v = 0; v < 4; ++v)
+#pragma unroll
+                    for (int t = 0; t < OT; ++t)
+                        acc[i][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[u][v][t], s[u][v], acc[i][t], 0, 0, 0);
+        }
+    }
+
+#pragma unroll
+    for (int i = 0; i < QT; ++i) {
+        float l = l_run[i] + lane_xor16(l_run[i]);
+        l += lane_xor32(l);
+#pragma unroll
+        for (int t = 0; t < OT; ++t)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) part_s[wave][i][OT * v + t][lane] = acc[i][t][v];
+        part_s[wave][i][4 * OT][lane] = m_run[i];
+        part_s[wave][i][4 * OT + 1][lane] = l;
+    }
+    __syncthreads();
+    // Wave w joins tile w % QT, its share of the lane's 4 OT outputs.
+    constexpr int SH = 4 / QT, PER = 4 * OT / SH;  // waves a tile, outputs a wave
+    const int i = wave % QT, first = wave / QT * PER;
+    const int qi = q0 + 16 * i + li;
+    float m = -INFINITY, f[4], l = 0.0f;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) m = fmaxf(m, part_s[w][i][4 * OT][lane]);
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+        f[w] = __builtin_amdgcn_exp2f(part_s[w][i][4 * OT][lane] - (m == -INFINITY ? 0.0f : m));
+        l += part_s[w][i][4 * OT + 1][lane] * f[w];
+    }
+    const float inv = 1.0f / l;
+    if (qi >= Lq) return;
+    float* orow = p.out + ((b * p.q_length + qi) * p.heads + h) * HD + 4 * OT * g + first;
+    float o[PER];
+#pragma unroll
+    for (int e = 0; e < PER; ++e) {
+        float sum = 0.0f;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) sum += part_s[w][i][first + e][lane] * f[w];
+        o[e] = sum * inv;
+    }
+#pragma unroll
+    for (int e = 0; e < PER; ++e) orow[e] = o[e];
+}
+
+template <int HD>
+void launch_attn_split(const AttnArgs& p, hipStream_t stream) {
+    const int64_t pairs = p.batch * p.heads;
+    // With 32 head dims and several blocks per CU two tiles share the loads (16 windows x 480 x 8 heads: 38 against
+    // 41 us); at 64 the longer products cover them (4 heads: 40 with one tile, 42 with two).
+    const bool two = HD == 32 && pairs * ceil_div(p.q_length, 16) > 1024;
+    const unsigned qb = static_cast<unsigned>(ceil_div(p.q_length, two ? 32 : 16));
+    const dim3 grid(static_cast<unsigned>(pairs) * qb);
+    if (two) {
+        hipLaunchKernelGGL((attn_split_kernel<HD, 2>), grid, dim3(256), 0, stream, p, qb);
+    } else {
+        hipLaunchKernelGGL((attn_split_kernel<HD, 1>), grid, dim3(256), 0, stream, p, qb);
+    }
+}
+
+// Where fp32 takes the split form (operands vec, head_dim 32 or 64): unless the 128-query blocks fill the chip and
+// there are few keys to split (64 windows x 128 x 4 heads: 20 us against 16; 64 x 200 35 against 37). bf16 keeps
+// attn_kernel: its probabilities are rounded relative to the running max of the 64-key chunks in order, which the
+// fused latent attention repeats bit for bit.
+bool attn_split_shape(const AttnArgs& p) {
+    const int64_t blocks = p.batch * p.heads * ceil_div(p.q_length, kQueriesPerBlock);
+    return p.q_length < (1 << 30) && p.kv_length < (1 << 30) &&
+           p.batch * p.heads * ceil_div(p.q_length, 16) < (int64_t{1} << 31) && (p.kv_length > 192 || blocks < 256);
+}
+
 template <int HD, bool BF16>
 void launch_attn(const AttnArgs& p, bool vec, hipStream_t stream) {
     const dim3 grid(static_cast<unsigned>(ceil_div(p.q_length, kQueriesPerBlock)), static_cast<unsigned>(p.heads),
@@ -2095,6 +2277,10 @@ extern "C" mlk_status mlk_attention(const float* q, int64_t q_token_stride, int6
                      q_head_stride % 4 == 0 && k_token_stride % 4 == 0 && k_head_stride % 4 == 0 &&
                      v_token_stride % 4 == 0 && v_head_stride % 4 == 0 && head_dim % 4 == 0;
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+    if (precision == MLK_DTYPE_F32 && vec && (head_dim == 32 || head_dim == 64) && attn_split_shape(p)) {
+        head_dim == 64 ? launch_attn_split<64>(p, s) : launch_attn_split<32>(p, s);
+        return launch_status("attention");
+    }
     if (precision == MLK_DTYPE_BF16) {
         dispatch_attn<true>(p, vec, s);
     } else {
