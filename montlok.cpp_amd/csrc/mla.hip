@@ -1635,7 +1635,7 @@ struct MlaSpanPack {
 };
 
 // mla_forward (montlok.cpp:1159-1211) for every causal query at d_model 256,
-// 4 heads of 64 (rope 32, nope 32), kv rank 64 and L <= 256: one block of 8
+// 4 heads of 64 (rope 32, nope 32), kv rank 64 and L <= 512: one block of 8
 // waves per (window, span of 64 query rows), so that neither the in_proj
 // output nor the attention output goes through HBM. A window's rows do not
 // fit one block's LDS as keys and queries at once (mla_window_kernel's form),
@@ -1657,13 +1657,16 @@ struct MlaSpanPack {
 //            the chunk sequence of mla_attend_kernel (its 64-key chunks are
 //            these tiles, in the same order), the same products and the same
 //            softmax arithmetic, so the result is the four-launch path's bit
-//            for bit. Wave w: head w / 2, query tiles (0, 3) or (1, 2) (the
+//            for bit (that path is built for L <= 256). Wave w: head w / 2, query tiles (0, 3) or (1, 2) (the
 //            diagonal tile's work balanced).
 //   o_proj   the normalised output rounded to bf16 (the o_proj's operand)
 //            in LDS, then wave w's two output column tiles over the 4 row
 //            tiles, the linear's chain again.
 // Blocks of one window run on one XCD (its L2 serves the later spans' reads
-// of the window's x). PACKED: the three weights in MlaSpanPack's order, each
+// of the window's x). Each block forms the latents and keys of the tiles it
+// walks again: at 480 rows 4.5 tiles a block on average, still half the time of
+// the separate operators (64 windows x 480: 172 -> 102 us; 16 x 480: 86 -> 53).
+// PACKED: the three weights in MlaSpanPack's order, each
 // wave's fragment load one contiguous 1 KB.
 template <bool PACKED>
 __global__ __launch_bounds__(512) void mla_span_kernel(MlaWindowArgs p, int spans) {
@@ -2381,7 +2384,7 @@ extern "C" mlk_status mlk_mla_attend_normed(const float* projected, int64_t batc
 namespace {
 
 // The geometries the one-launch kernels are built for (mla_window_kernel: 8 heads of 32, L <= 128;
-// mla_span_kernel: 4 heads of 64, L <= 256), and their operand checks; MLK_OK when a kernel takes the
+// mla_span_kernel: 4 heads of 64, L <= 512), and their operand checks; MLK_OK when a kernel takes the
 // call, MLK_ERR_UNSUPPORTED (with the reason) when the separate operators must run it.
 mlk_status mla_window_supported(const float* x, int64_t length, int64_t d_model, int64_t x_batch_stride,
                                 int64_t x_token_stride, const float* kv_norm_w, const float* kv_norm_b,
@@ -2389,7 +2392,7 @@ mlk_status mla_window_supported(const float* x, int64_t length, int64_t d_model,
                                 int64_t nope_dim, int64_t kv_rank, double scale, const float* out,
                                 std::initializer_list<const void*> weights) {
     const bool window = heads == 8 && head_dim == 32 && nope_dim == 16 && kv_rank == 64 && length <= 128;
-    const bool span = heads == 4 && head_dim == 64 && nope_dim == 32 && kv_rank == 64 && length <= 256;
+    const bool span = heads == 4 && head_dim == 64 && nope_dim == 32 && kv_rank == 64 && length <= 512;
     if (!(window || span) || d_model != heads * head_dim) {
         set_error("mla_forward: geometry without a one-launch kernel (use the separate operators)");
         return MLK_ERR_UNSUPPORTED;

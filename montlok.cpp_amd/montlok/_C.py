@@ -740,7 +740,7 @@ def _mla_window(x, in_proj_weight, kv_norm_weight, kv_norm_bias, kv_norm_eps, kv
                 sine, n_heads, head_dim, nope_dim, kv_lora_rank, scale):
     """The whole forward for every causal query in one launch, on the weights packed in the kernel's fragment
     order (bf16 weights, kv rank 64, a positive scale; 8 heads of 32 with rope 16 and L <= 128: one block per
-    window; 4 heads of 64 with rope 32 and L <= 256: one block per window and 64 query rows); None where no
+    window; 4 heads of 64 with rope 32 and L <= 512: one block per window and 64 query rows); None where no
     such kernel is built for the call."""
     batch, length, d_model = x.shape
     ws = [in_proj_weight, kv_up_weight, out_weight]
@@ -788,7 +788,10 @@ def _mla_forward(x, in_proj_weight, q_weight, kv_norm_weight, kv_norm_bias, kv_n
     _check(n_last == 1 or n_last == length, "native MLA supports the final query or the full sequence")
     precision = torch.bfloat16 if _weight(in_proj_weight, "in_proj_weight").dtype == torch.bfloat16 else torch.float32
     full = n_last == length
-    if allow_fused and allow_window and full and causal and precision == torch.bfloat16:
+    # Beyond 256 rows a block of the one-launch kernel walks up to eight key tiles: 50 us however few windows there
+    # are, against 42 us for one and 56 for four windows of 480 in separate operators.
+    if allow_fused and allow_window and full and causal and precision == torch.bfloat16 and \
+            (length <= 256 or batch >= 4):
         out = _mla_window(x, in_proj_weight, kv_norm_weight, kv_norm_bias, kv_norm_eps, kv_up_weight, out_weight,
                           cosine, sine, n_heads, head_dim, nope_dim, kv_lora_rank, scale)
         if out is not None:

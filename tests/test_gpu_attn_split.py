@@ -1,11 +1,17 @@
-"""fp32 attention with the keys split over four waves (attn_split_kernel) at the edges of its tiles, chunks and rule."""
+"""fp32 attention with the keys split over four waves (attn_split_kernel) at the edges of its tiles, chunks and rule,
+and the one-launch MLA beyond 256 rows."""
 
 from __future__ import annotations
 
 import math
 
+import numpy as np
 import pytest
 import torch
+
+import bf16_emu as emu
+from helpers import BF16_TOL, assert_close, assert_emulated
+from test_gpu_mla import _mla_params, _oracle_mla, _t, rope_tables
 
 pytestmark = pytest.mark.gpu
 
@@ -48,3 +54,29 @@ def test_split_attention_special_values(dev):
     assert torch.isnan(out[:, 150:, 1]).all()
     keep = [j for j in range(200) if j != 70]
     assert torch.allclose(out[0, 199, 0], v[0, keep, 0].mean(0), atol=1e-6)
+
+
+@pytest.mark.parametrize("B,L,bias", [(4, 257, True), (5, 480, False), (8, 512, True), (4, 320, True)])
+def test_one_launch_mla_beyond_256_rows(dev, oracle, B, L, bias):
+    from montlok import _C
+
+    H, hd, nope, kvr = 4, 64, 32, 64
+    d = H * hd
+    rng = np.random.default_rng(B + L)
+    x = rng.standard_normal((B, L, d)).astype(np.float32)
+    p = _mla_params(rng, d, H, hd, nope, kvr, True)
+    if not bias:
+        p["ln_b"] = np.zeros_like(p["ln_b"])
+    cos, sin = rope_tables(L, hd - nope)
+    bw = lambda a: _t(a, dev).to(torch.bfloat16)  # noqa: E731
+    in_w = np.concatenate([p["q"], p["kv_down"], p["k_rope"]])
+    args = (_t(x, dev), bw(in_w), torch.empty(0, device=dev), _t(p["ln_w"], dev), _t(p["ln_b"], dev) if bias else None, 1e-5,
+            bw(p["kv_up"]), bw(p["o"]), _t(cos, dev), _t(sin, dev), H, hd, nope, kvr, L, True, hd ** -0.5)
+    out = _C._mla_forward(*args, allow_fused=True)
+    assert _C.mla_forward_launches() == ["mla_forward"]
+    emulated = emu.mla_forward(x, p["q"], p["kv_down"], p["k_rope"], p["ln_w"], p["ln_b"], 1e-5, p["kv_up"], p["o"],
+                               cos, sin, H, hd, nope, hd ** -0.5)
+    assert_emulated(out, emulated, name=f"one-launch MLA {B}x{L} vs the bf16 emulation")
+    assert_close(out, _oracle_mla(oracle, x, p, H, hd, nope, kvr, L, True, hd ** -0.5, cos, sin), tol=BF16_TOL, name="vs oracle")
+    _C._mla_forward(args[0][:3], *args[1:], allow_fused=True)
+    assert _C.mla_forward_launches() == ["separate"], "few long windows run the separate operators"
