@@ -16,6 +16,8 @@
 // K = 512) where the fp32 forms it replaces have 2.9e-7 (4.1e-7).
 //
 //   block  = 64 rows x 64 columns of y, 4 waves of 32 x 32; K in steps of 32.
+//            Large calls: 128 x 128, 4 waves of 64 x 64 that multiply and 4 that
+//            stage, two LDS buffers.
 //   stage  = 16-row pieces of x and W, whole 128-byte lines per load (the
 //            MFMA operand order straight from memory takes every line in four
 //            separate instructions: 20-25% slower), split in registers and
@@ -23,14 +25,15 @@
 //   D      = transposed products (W as the A operand): lane (g, l) of a wave
 //            holds row l, columns 8 j + 4 g .. + 3 (j = 0..3), 16-byte stores.
 //
-// What bounds it: per step and SIMD the matrix cores take 220 cycles and the
-// splits about 200 issue cycles; both run at 48% of the time with five blocks
-// a CU (27 KiB of LDS, 68 registers) in different phases. One LDS buffer and
-// two barriers: a second buffer, or 64 x 128 and 128 x 128 blocks, which split
-// less often, leave fewer waves to overlap and were not faster below 65,536
-// rows (7680 x 256 -> 1192: 36 us against 38 and 48; 65536 x 512 -> 256: 115
-// against 107 and 101). Measured against the fp32 forms: 7680 x 256 -> 1192
-// 69 -> 36 us, 7680 x 512 -> 256 34 -> 18, 15360 x 256 -> 1192 112 -> 68.
+// What bounds it: the bf16 products. On random data this card's clocks hold a
+// large bf16 matrix product at 1.1 PFLOP/s, 183 TFLOP/s of these sums, and
+// 65536 x 512 -> 256 takes 95 us in the big blocks (180 TFLOP/s). The small
+// blocks keep the matrix cores 43% busy (27 KiB of LDS, 68 registers, five
+// blocks a CU in different phases: a step and SIMD takes 220 cycles of
+// products and about 200 of splitting); a second LDS buffer there, or deeper
+// prefetch in either, was slower. Against the fp32 forms: 7680 x 256 -> 1192
+// 69 -> 35 us, 7680 x 512 -> 256 34 -> 18, 15360 x 256 -> 1192 112 -> 66,
+// 15360 x 512 -> 256 52 -> 26.
 //
 // Parts of an infinity or of a value that rounds to bf16 infinity are
 // inf and -inf (or NaN), so a result that involves one is NaN; such results
@@ -94,188 +97,267 @@ __device__ __forceinline__ void norm_scales(const LinearArgs& p, int64_t row0, i
 // then up; a wave's W tile is 16 gate rows and the 16 up rows of the same columns, so that a lane holds both
 // of its outputs' factors, and out = silu(gate) * up in fp64, rounded once (p.N = hidden columns of out). The
 // 2 N columns then never reach memory: 7680 x 256 -> 2 x 512 36 us, against 38 for the linear and 13 for swiglu.
-template <bool FULL, int GS, bool SWIGLU>
-__global__ __launch_bounds__(256) void linear_split_kernel(LinearArgs p, unsigned n_blocks) {
-    constexpr int kCols = SWIGLU ? kBlock / 2 : kBlock;  // output columns of the block
-    __shared__ uint4 frag[4 * kTileUnits];               // x tiles 0, 1, W tiles 2, 3
+// T: the wave tile is (32 T) x (32 T), the block (64 T) x (64 T). T = 2 has four more waves that stage (PRODUCER
+// below) while the first four multiply, with two LDS buffers and one barrier a step.
+template <bool FULL, int GS, bool SWIGLU, int T>
+__global__ __launch_bounds__(T == 1 ? 256 : 512, T == 1 ? 1 : 2) void linear_split_kernel(LinearArgs p, unsigned n_blocks) {
+    static_assert(T == 1 || GS == 0, "the norm's prologue is the 64 x 64 block's");
+    constexpr int kRows = kBlock * T, kCols = SWIGLU ? kRows / 2 : kRows;  // rows, output columns of the block
+    constexpr int kBuffer = 4 * T * kTileUnits;  // x tiles 0 .. 2 T - 1, then W tiles
+    __shared__ uint4 frag[T * kBuffer];
     __shared__ double scale[GS > 0 ? kBlock * kMaxNormGroups : 1];
     const int lane = threadIdx.x & 63, li = lane & 31, g = lane >> 5;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) & 3;
+    const bool producer = T == 1 || __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) >= 4;
     // XCD x takes the x-th eighth of the blocks, column blocks of one row block side by side: a row block's x
     // is fetched into one L2.
     unsigned lin = blockIdx.x;
     if (gridDim.x % 8 == 0) lin = (lin % 8) * (gridDim.x / 8) + lin / 8;
-    const int64_t row0 = static_cast<int64_t>(lin / n_blocks) * kBlock;
+    const int64_t row0 = static_cast<int64_t>(lin / n_blocks) * kRows;
     const int64_t n0 = static_cast<int64_t>(lin % n_blocks) * kCols;
     const int K = static_cast<int>(p.K);
     const int groups = GS > 0 ? K / GS : 0;
     const float* w = static_cast<const float*>(p.w);
 
-    // Wave w stages rows 16 w .. + 15 of x and of W: lane 8 r + c of a load holds k = 4 c .. + 3 of row r (of
-    // 8), whole lines; byte offsets in 32 bits from the block's first row (strides checked at launch).
+    // Staging wave w takes rows 64 i + 16 w .. + 15 of x and of W: lane 8 r + c of a load holds k = 4 c .. + 3 of
+    // row r (of 8), whole lines; byte offsets in 32 bits from the block's first row (strides checked at launch).
     const int sr = lane >> 3, sc = lane & 7;
     const char* base[2] = {reinterpret_cast<const char*>(p.x + row0 * p.x_stride), reinterpret_cast<const char*>(w + n0 * p.K)};
-    unsigned off[2][2];
-#pragma unroll
-    for (int m = 0; m < 2; ++m) {
-        const int r = 16 * wave + 8 * m + sr;
-        off[0][m] = static_cast<unsigned>((row0 + r < p.rows ? r : p.rows - 1 - row0) * p.x_stride * 4) + 16 * sc;
-        int64_t n = r;
-        if constexpr (SWIGLU) {
-            const int64_t col = 16 * (wave >> 1) + 8 * m + sr;
-            n = (n0 + col < p.N ? col : p.N - 1 - n0) + (wave & 1 ? p.N : 0);
-        } else {
-            n = n0 + n < p.N ? n : p.N - 1 - n0;
-        }
-        off[1][m] = static_cast<unsigned>(n * p.K * 4) + 16 * sc;
-    }
-    float4 v[2][2], nw;
+    unsigned off[2][T][2];
+    float4 v[2][T][2], nw;
     bool live = true;  // of the fetched step (K a multiple of 4: a lane's 4 k are on one side of it)
+    auto rows = [&]() {
+#pragma unroll
+        for (int i = 0; i < T; ++i)
+#pragma unroll
+            for (int m = 0; m < 2; ++m) {
+                const int r = 64 * i + 16 * wave + 8 * m + sr;
+                off[0][i][m] = static_cast<unsigned>((row0 + r < p.rows ? r : p.rows - 1 - row0) * p.x_stride * 4) + 16 * sc;
+                int64_t n = r;
+                if constexpr (SWIGLU) {
+                    const int64_t col = 32 * i + 16 * (wave >> 1) + 8 * m + sr;
+                    n = (n0 + col < p.N ? col : p.N - 1 - n0) + (wave & 1 ? p.N : 0);
+                } else {
+                    n = n0 + n < p.N ? n : p.N - 1 - n0;
+                }
+                off[1][i][m] = static_cast<unsigned>(n * p.K * 4) + 16 * sc;
+            }
+    };
     auto fetch = [&](int k0) {
         live = k0 + 4 * sc < K;
         const unsigned ko = FULL ? (k0 < K ? 4 * k0 : 0u) : (live ? 4 * k0 : 0u - 16 * sc);
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
+        for (int o = 0; o < 2; ++o)
 #pragma unroll
-            for (int m = 0; m < 2; ++m) v[i][m] = *reinterpret_cast<const float4*>(base[i] + static_cast<unsigned>(off[i][m] + ko));
+            for (int i = 0; i < T; ++i)
+#pragma unroll
+                for (int m = 0; m < 2; ++m)
+                    v[o][i][m] = *reinterpret_cast<const float4*>(base[o] + static_cast<unsigned>(off[o][i][m] + ko));
         if constexpr (GS > 0) nw = *reinterpret_cast<const float4*>(p.norm_w + (live ? k0 + 4 * sc : 0));
     };
     // Values past K become zeros here and not at the load, whose wait would then stand in front of the products.
-    auto stage = [&](int k0) {
-        uint2* dst = reinterpret_cast<uint2*>(frag);
+    auto stage = [&](int k0, int buffer) {
+        uint2* dst = reinterpret_cast<uint2*>(frag + buffer * kBuffer);
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
+        for (int o = 0; o < 2; ++o)
 #pragma unroll
-            for (int m = 0; m < 2; ++m) {
-                float4 f = v[i][m];
-                if (GS > 0 && i == 0) {
-                    const int k = live ? k0 + 4 * sc : 0;
-                    const double s = scale[(16 * wave + 8 * m + sr) * groups + k / (GS > 0 ? GS : 1)];
-                    f.x = static_cast<float>((static_cast<double>(f.x) * s) * static_cast<double>(nw.x));
-                    f.y = static_cast<float>((static_cast<double>(f.y) * s) * static_cast<double>(nw.y));
-                    f.z = static_cast<float>((static_cast<double>(f.z) * s) * static_cast<double>(nw.z));
-                    f.w = static_cast<float>((static_cast<double>(f.w) * s) * static_cast<double>(nw.w));
+            for (int i = 0; i < T; ++i)
+#pragma unroll
+                for (int m = 0; m < 2; ++m) {
+                    float4 f = v[o][i][m];
+                    if (GS > 0 && o == 0) {
+                        const int k = live ? k0 + 4 * sc : 0;
+                        const double s = scale[(16 * wave + 8 * m + sr) * groups + k / (GS > 0 ? GS : 1)];
+                        f.x = static_cast<float>((static_cast<double>(f.x) * s) * static_cast<double>(nw.x));
+                        f.y = static_cast<float>((static_cast<double>(f.y) * s) * static_cast<double>(nw.y));
+                        f.z = static_cast<float>((static_cast<double>(f.z) * s) * static_cast<double>(nw.z));
+                        f.w = static_cast<float>((static_cast<double>(f.w) * s) * static_cast<double>(nw.w));
+                    }
+                    if (!FULL && !live) f = float4{0.0f, 0.0f, 0.0f, 0.0f};
+                    f32x2 lo = {f.x, f.y}, hi = {f.z, f.w};
+                    const unsigned slot = unit(2 * (o * T + i) + (wave >> 1), sc >> 2, 0, (sc >> 1) & 1) + 16 * (wave & 1) + 8 * m + sr;
+#pragma unroll
+                    for (int q = 0; q < kPlanes; ++q) dst[2 * (slot + q * 2 * kGroupUnits) + (sc & 1)] = uint2{take_bf16(lo), take_bf16(hi)};
                 }
-                if (!FULL && !live) f = float4{0.0f, 0.0f, 0.0f, 0.0f};
-                f32x2 lo = {f.x, f.y}, hi = {f.z, f.w};
-                const unsigned slot = unit(2 * i + (wave >> 1), sc >> 2, 0, (sc >> 1) & 1) + 16 * (wave & 1) + 8 * m + sr;
-#pragma unroll
-                for (int q = 0; q < kPlanes; ++q) dst[2 * (slot + q * 2 * kGroupUnits) + (sc & 1)] = uint2{take_bf16(lo), take_bf16(hi)};
-            }
     };
 
     const int wm = wave & 1, wn = wave >> 1;
-    f32x16 acc, low;
+    f32x16 acc[T][T], low[T][T];  // [x tile][W tile]
 #pragma unroll
-    for (int c = 0; c < 16; ++c) acc[c] = low[c] = 0.0f;
-
-    fetch(0);
-    if constexpr (GS > 0) {
-        norm_scales<(GS > 0 ? GS : 8)>(p, row0, groups, scale);
-        __syncthreads();
-    }
-    for (int k0 = 0; k0 < K; k0 += kStep) {
-        if (k0 > 0) __syncthreads();
-        stage(k0);
-        __syncthreads();
-        fetch(k0 + kStep);
+    for (int i = 0; i < T; ++i)
+#pragma unroll
+        for (int j = 0; j < T; ++j)
+#pragma unroll
+            for (int c = 0; c < 16; ++c) acc[i][j][c] = low[i][j][c] = 0.0f;
+    auto multiply = [&](int buffer) {
+        const uint4* src = frag + buffer * kBuffer;
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
-            bf16x8 xf[kPlanes], wf[kPlanes];
+            bf16x8 xf[T][kPlanes], wf[T][kPlanes];
 #pragma unroll
-            for (int q = 0; q < kPlanes; ++q) {
-                xf[q] = __builtin_bit_cast(bf16x8, frag[unit(wm, h, q, g) + li]);
-                wf[q] = __builtin_bit_cast(bf16x8, frag[unit(2 + wn, h, q, g) + li]);
-            }
-            acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[0], xf[0], acc, 0, 0, 0);
+            for (int q = 0; q < kPlanes; ++q)
 #pragma unroll
-            for (int order = 1; order < kPlanes; ++order)
+                for (int i = 0; i < T; ++i) {
+                    xf[i][q] = __builtin_bit_cast(bf16x8, src[unit(wm * T + i, h, q, g) + li]);
+                    wf[i][q] = __builtin_bit_cast(bf16x8, src[unit(2 * T + wn * T + i, h, q, g) + li]);
+                }
 #pragma unroll
-                for (int q = 0; q <= order; ++q) low = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[q], xf[order - q], low, 0, 0, 0);
+            for (int order = 0; order < kPlanes; ++order)
+#pragma unroll
+                for (int q = 0; q <= order; ++q)
+#pragma unroll
+                    for (int i = 0; i < T; ++i)
+#pragma unroll
+                        for (int j = 0; j < T; ++j) {
+                            f32x16& c = order == 0 ? acc[i][j] : low[i][j];
+                            c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[j][q], xf[i][order - q], c, 0, 0, 0);
+                        }
         }
-    }
-#pragma unroll
-    for (int c = 0; c < 16; ++c) acc[c] += low[c];
+    };
 
-    const int64_t row = row0 + 32 * wm + li;
-    if (row >= p.rows) return;
-    // W row of accumulator element c (0 .. 15), and its column of out.
-    auto w_row = [&](int c) -> int64_t {
-        const int r = 8 * (c >> 2) + 4 * g + (c & 3);
-        if constexpr (SWIGLU) return n0 + 16 * wn + (r & 15) + (r & 16 ? p.N : 0);
-        return n0 + 32 * wn + r;
-    };
-    auto in_range = [&](int c) {
-        if constexpr (SWIGLU) return w_row(c & 7) < p.N;
-        return w_row(c) < p.N;
-    };
-    bool finite = true;
-#pragma unroll
-    for (int c = 0; c < 16; ++c) finite = finite && acc[c] == acc[c];
-    if (!finite) {
-#pragma unroll 1
-        for (int c = 0; c < 16; ++c) {
-            if (!in_range(c)) continue;
-            const float* xr = p.x + row * p.x_stride;
-            const float* wr = w + w_row(c) * p.K;
-            float sum = 0.0f;
-#pragma unroll 1
-            for (int k = 0; k < K; ++k) {
-                float x = xr[k];
-                if constexpr (GS > 0)
-                    x = static_cast<float>((static_cast<double>(x) * scale[(32 * wm + li) * groups + k / GS]) *
-                                           static_cast<double>(p.norm_w[k]));
-                sum = fmaf(x, wr[k], sum);
-            }
-#pragma unroll
-            for (int e = 0; e < 16; ++e) acc[e] = e == c && acc[e] != acc[e] ? sum : acc[e];
+    if constexpr (T == 1) {
+        rows();
+        fetch(0);
+        if constexpr (GS > 0) {
+            norm_scales<(GS > 0 ? GS : 8)>(p, row0, groups, scale);
+            __syncthreads();
         }
-    }
-    if (p.bias != nullptr) {
-#pragma unroll
-        for (int c = 0; c < 16; ++c) acc[c] += p.bias[in_range(c) ? w_row(c) : 0];
+        for (int k0 = 0; k0 < K; k0 += kStep) {
+            if (k0 > 0) __syncthreads();
+            stage(k0, 0);
+            __syncthreads();
+            fetch(k0 + kStep);
+            multiply(0);
+        }
+    } else if (producer) {
+        rows();
+        fetch(0);
+        stage(0, 0);
+        fetch(kStep);
+        int buffer = 1;
+        for (int k0 = 0; k0 < K; k0 += kStep, buffer ^= 1) {
+            __syncthreads();
+            stage(k0 + kStep, buffer);  // (past K: loads of the first columns, not read)
+            fetch(k0 + 2 * kStep);
+        }
+        return;
+    } else {
+        int buffer = 0;
+        for (int k0 = 0; k0 < K; k0 += kStep, buffer ^= 1) {
+            __syncthreads();
+            multiply(buffer);
+        }
     }
 
     const bool vec_out = (reinterpret_cast<uintptr_t>(p.out) & 15) == 0 && p.out_stride % 4 == 0 &&
                          (p.residual == nullptr ||
                           ((reinterpret_cast<uintptr_t>(p.residual) & 15) == 0 && p.res_stride % 4 == 0));
 #pragma unroll
-    for (int j = 0; j < (SWIGLU ? 2 : 4); ++j) {
-        const int64_t col = w_row(4 * j);
-        if (col >= p.N) continue;
-        f32x4 y = {acc[4 * j], acc[4 * j + 1], acc[4 * j + 2], acc[4 * j + 3]};
-        if constexpr (SWIGLU) {
+    for (int i = 0; i < T; ++i) {
+        const int64_t row = row0 + 32 * (wm * T + i) + li;
+        if (row >= p.rows) continue;
 #pragma unroll
-            for (int c = 0; c < 4; ++c)
-                y[c] = static_cast<float>(silu_d(static_cast<double>(y[c])) * static_cast<double>(acc[8 + 4 * j + c]));
-        }
-        float* dst = p.out + row * p.out_stride + col;
-        const float* res = p.residual != nullptr ? p.residual + row * p.res_stride + col : nullptr;
-        if (vec_out && col + 4 <= p.N) {
-            if (res != nullptr) y = *reinterpret_cast<const f32x4*>(res) + y;
-            *reinterpret_cast<f32x4*>(dst) = y;
-        } else {
+        for (int t = 0; t < T; ++t) {
+            f32x16& y = acc[i][t];
 #pragma unroll
-            for (int c = 0; c < 4; ++c)
-                if (col + c < p.N) dst[c] = res != nullptr ? res[c] + y[c] : y[c];
+            for (int c = 0; c < 16; ++c) y[c] += low[i][t][c];
+            // W row of accumulator element c (0 .. 15), and its column of out.
+            auto w_row = [&](int c) -> int64_t {
+                const int r = 8 * (c >> 2) + 4 * g + (c & 3);
+                if constexpr (SWIGLU) return n0 + 16 * (wn * T + t) + (r & 15) + (r & 16 ? p.N : 0);
+                return n0 + 32 * (wn * T + t) + r;
+            };
+            auto in_range = [&](int c) {
+                if constexpr (SWIGLU) return w_row(c & 7) < p.N;
+                return w_row(c) < p.N;
+            };
+            bool finite = true;
+#pragma unroll
+            for (int c = 0; c < 16; ++c) finite = finite && y[c] == y[c];
+            if (!finite) {
+#pragma unroll 1
+                for (int c = 0; c < 16; ++c) {
+                    if (!in_range(c)) continue;
+                    const float* xr = p.x + row * p.x_stride;
+                    const float* wr = w + w_row(c) * p.K;
+                    float sum = 0.0f;
+#pragma unroll 1
+                    for (int k = 0; k < K; ++k) {
+                        float x = xr[k];
+                        if constexpr (GS > 0)
+                            x = static_cast<float>((static_cast<double>(x) * scale[(32 * wm + li) * groups + k / GS]) *
+                                                   static_cast<double>(p.norm_w[k]));
+                        sum = fmaf(x, wr[k], sum);
+                    }
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) y[e] = e == c && y[e] != y[e] ? sum : y[e];
+                }
+            }
+            if (p.bias != nullptr) {
+#pragma unroll
+                for (int c = 0; c < 16; ++c) y[c] += p.bias[in_range(c) ? w_row(c) : 0];
+            }
+#pragma unroll
+            for (int j = 0; j < (SWIGLU ? 2 : 4); ++j) {
+                const int64_t col = w_row(4 * j);
+                if (col >= p.N) continue;
+                f32x4 o = {y[4 * j], y[4 * j + 1], y[4 * j + 2], y[4 * j + 3]};
+                if constexpr (SWIGLU) {
+#pragma unroll
+                    for (int c = 0; c < 4; ++c)
+                        o[c] = static_cast<float>(silu_d(static_cast<double>(o[c])) * static_cast<double>(y[8 + 4 * j + c]));
+                }
+                float* dst = p.out + row * p.out_stride + col;
+                const float* res = p.residual != nullptr ? p.residual + row * p.res_stride + col : nullptr;
+                if (vec_out && col + 4 <= p.N) {
+                    if (res != nullptr) o = *reinterpret_cast<const f32x4*>(res) + o;
+                    *reinterpret_cast<f32x4*>(dst) = o;
+                } else {
+#pragma unroll
+                    for (int c = 0; c < 4; ++c)
+                        if (col + c < p.N) dst[c] = res != nullptr ? res[c] + o[c] : o[c];
+                }
+            }
         }
     }
+}
+
+template <int GS, bool SWIGLU, int T>
+void launch_blocks(const LinearArgs& p, hipStream_t stream) {
+    const int64_t nb = ceil_div(p.N, (SWIGLU ? kBlock / 2 : kBlock) * T);
+    const dim3 grid(static_cast<unsigned>(ceil_div(p.rows, kBlock * T) * nb)), threads(T == 1 ? 256 : 512);
+    if (p.K % kStep == 0) {
+        hipLaunchKernelGGL((linear_split_kernel<true, GS, SWIGLU, T>), grid, threads, 0, stream, p, static_cast<unsigned>(nb));
+    } else {
+        hipLaunchKernelGGL((linear_split_kernel<false, GS, SWIGLU, T>), grid, threads, 0, stream, p, static_cast<unsigned>(nb));
+    }
+}
+
+// Whether rounds of 256 blocks of 128 x 128 (one a CU) are filled to nine tenths by the call's rows and columns.
+// Then the big blocks, which split every operand half as often and multiply while they split, are the faster ones
+// (15360 x 512 -> 256, 240 blocks: 25.6 us against 30.6; 65536 x 512 -> 256: 95 against 113; 7680 x 256 -> 1024, 480
+// blocks: 28 against 31); otherwise their last round, or the columns past N, cost more than that (7680 x 256 ->
+// 1192, 600 blocks: 41 against 35; 7680 x 512 -> 256, 120 blocks: 20 against 18).
+bool fills_big_blocks(int64_t rows, int64_t w_rows) {
+    const int64_t blocks = ceil_div(rows, 2 * kBlock) * ceil_div(w_rows, 2 * kBlock);
+    const double held = static_cast<double>(ceil_div(blocks, 256) * 256) * (4 * kBlock * kBlock);
+    return static_cast<double>(rows) * static_cast<double>(w_rows) >= 0.9 * held;
 }
 
 template <int GS, bool SWIGLU>
 void launch(const LinearArgs& p, hipStream_t stream) {
-    const int64_t nb = ceil_div(p.N, SWIGLU ? kBlock / 2 : kBlock);
-    const dim3 grid(static_cast<unsigned>(ceil_div(p.rows, kBlock) * nb));
-    if (p.K % kStep == 0) {
-        hipLaunchKernelGGL((linear_split_kernel<true, GS, SWIGLU>), grid, dim3(256), 0, stream, p, static_cast<unsigned>(nb));
-    } else {
-        hipLaunchKernelGGL((linear_split_kernel<false, GS, SWIGLU>), grid, dim3(256), 0, stream, p, static_cast<unsigned>(nb));
+    if constexpr (GS == 0) {
+        if (fills_big_blocks(p.rows, SWIGLU ? 2 * p.N : p.N)) {
+            launch_blocks<0, SWIGLU, 2>(p, stream);
+            return;
+        }
     }
+    launch_blocks<GS, SWIGLU, 1>(p, stream);
 }
 
 // 32-bit byte offsets from a block's first rows, and the grid.
 bool fits(const LinearArgs& p, int64_t w_rows) {
-    return p.K % 4 == 0 && p.x_stride < (int64_t{1} << 23) && p.K * (w_rows + kBlock) < (int64_t{1} << 30) &&
+    return p.K % 4 == 0 && p.x_stride < (int64_t{1} << 23) && p.K * (w_rows + 2 * kBlock) < (int64_t{1} << 30) &&
            ceil_div(p.rows, kBlock) * ceil_div(p.N, kBlock / 2) < (int64_t{1} << 31);
 }
 

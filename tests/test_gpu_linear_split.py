@@ -28,9 +28,11 @@ def _assert_bound(got, x, w, terms, extra=0.0):
 
 
 # (rows, K, N, x row padding): one past a block, K not a multiple of the 32-wide step or of 8, ragged and tiny N, the
-# first shapes past the one-wave rule's 1536 tiles, K just above 128, one row against many columns.
+# first shapes past the one-wave rule's 1536 tiles, K just above 128, one row against many columns; then calls that
+# fill rounds of 128 x 128 blocks, with ragged last rows and columns, K not a multiple of the step, one and two steps.
 SPLIT = [(1921, 256, 352, 0), (2049, 136, 200, 4), (1600, 132, 257, 0), (30000, 256, 1, 8), (64, 2048, 5200, 0),
-         (1, 256, 24592, 0), (12304, 160, 30, 0), (1537, 256, 256, 12)]
+         (1, 256, 24592, 0), (12304, 160, 30, 0), (1537, 256, 256, 12),
+         (15360, 512, 256, 0), (16371, 260, 255, 4), (3840, 136, 1024, 0), (32700, 132, 256, 0), (65536, 544, 120, 0)]
 
 
 @pytest.mark.parametrize("M,K,N,pad", SPLIT)

@@ -10,7 +10,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("M,K,hidden,bias", [(480, 256, 512, False), (1921, 256, 353, True), (2500, 136, 97, True),
-                                             (64, 1032, 5000, False), (30000, 256, 1, True), (129, 256, 3104, True)])
+                                             (64, 1032, 5000, False), (30000, 256, 1, True), (129, 256, 3104, True), (7680, 256, 512, True), (8100, 292, 505, False)])
 def test_linear_swiglu_vs_float64(dev, M, K, hidden, bias):
     from montlok import _C
 
