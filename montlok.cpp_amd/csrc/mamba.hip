@@ -980,6 +980,11 @@ struct ScanArgs {
     int64_t gsb, gst;
     int gate_logits;
     float* out;  // [B, L, H*D] contiguous
+    // TOK: formed by scan_token_kernel, chunks C tokens a window: (alpha, beta, gamma, dt) [B, H, chunks C] and
+    // tanh(angle) * pi [B, chunks C, R].
+    const float4* tok_coef;
+    const float* tok_ang;
+    int64_t chunks;
 };
 
 // The LDS of one (window, head) scan.
@@ -1033,7 +1038,9 @@ struct NoChunkHooks {
 // gates, and rotates those rows in step d; step c skips the angle sums. Steps
 // e and f form token tile 0's G tile, products and outputs in registers (tile
 // 1's are the other waves' after the barrier that ends step d).
-template <int C, int NT, int DT, bool TILE, class Hooks, bool TILE_OUT = TILE, bool PREP = false>
+// TOK: the chunk's coefficients and tanh(angle) * pi come from a.tok_coef and
+// a.tok_ang; step a loads them in place of the columns they are formed from.
+template <int C, int NT, int DT, bool TILE, class Hooks, bool TILE_OUT = TILE, bool PREP = false, bool TOK = false>
 __device__ __forceinline__ void scan_head(const ScanArgs& a, ScanLds<C, NT, DT>& sh, int64_t b, int64_t h,
                                           int tid_base, const Hooks& hooks) {
     static_assert(C == 32, "the BCNorm step takes one lane per (token, B|C) pair of a 64-lane wave");
@@ -1175,9 +1182,15 @@ __device__ __forceinline__ void scan_head(const ScanArgs& a, ScanLds<C, NT, DT>&
                 bx[j] = load_off32(bc, off);
                 cx[j] = load_off32(cc, off);
             }
+            constexpr int kCoefLane = NTH >= 128 ? 64 : 0;  // the coefficient wave's first thread
+            const int tc = static_cast<int>(c0 / C);
+            float4 tok4 = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            if constexpr (TOK) {
+                if (tid >= kCoefLane && tid < kCoefLane + C) tok4 = a.tok_coef[((b * H + h) * a.chunks + tc) * C + tid - kCoefLane];
+            }
 #pragma unroll
             for (int j = 0; j < MU; ++j) {
-                if constexpr (PREP) break;
+                if constexpr (PREP || TOK) break;
                 const int u = tid + NTH * j;
                 const int which = u < 3 * C ? u / C : 0, t = u % C;
                 mx[j] = load_off32(mc, static_cast<unsigned>((t < Lc ? t : Lc - 1) * st32 + which * static_cast<int>(H)));
@@ -1187,6 +1200,10 @@ __device__ __forceinline__ void scan_head(const ScanArgs& a, ScanLds<C, NT, DT>&
                 for (int j = 0; j < AU; ++j) {
                     const unsigned u = static_cast<unsigned>(tid + NTH * j);
                     const unsigned uc = u < static_cast<unsigned>(C * R) ? u : static_cast<unsigned>(C * R - 1);
+                    if constexpr (TOK) {
+                        ax[j] = load_off32(a.tok_ang + (b * a.chunks + tc) * C * R, uc);
+                        continue;
+                    }
                     const int t = static_cast<int>((uc * rmagic) >> 16), r = static_cast<int>(uc) - t * R;
                     ax[j] = load_off32(ac, static_cast<unsigned>((t < Lc ? t : Lc - 1) * st32 + r));
                 }
@@ -1215,9 +1232,15 @@ __device__ __forceinline__ void scan_head(const ScanArgs& a, ScanLds<C, NT, DT>&
             }
 #pragma unroll
             for (int j = 0; j < MU; ++j) {
-                if constexpr (PREP) break;
+                if constexpr (PREP || TOK) break;
                 const int u = tid + NTH * j;
                 if (u < 3 * C) raw_s[u / C][u % C] = mx[j];
+            }
+            if (TOK && tid >= kCoefLane && tid < kCoefLane + C) {
+                coef[0][tid - kCoefLane] = tok4.x;
+                coef[1][tid - kCoefLane] = tok4.y;
+                coef[2][tid - kCoefLane] = tok4.z;
+                coef[3][tid - kCoefLane] = tok4.w;
             }
             if (!PREP && R > 0) {
 #pragma unroll
@@ -1252,7 +1275,7 @@ __device__ __forceinline__ void scan_head(const ScanArgs& a, ScanLds<C, NT, DT>&
         // goes on to the decay weights (decay_walk). tanh runs on the other waves.
         if constexpr (!PREP) {
             const int ct = NTH >= 128 ? tid - 64 : tid;
-            if (ct >= 0 && ct < C) token_coefficients<C>(ct, raw_s[0][ct], raw_s[1][ct], raw_s[2][ct], dt_bias, a.a_floor, Lc, coef);
+            if (!TOK && ct >= 0 && ct < C) token_coefficients<C>(ct, raw_s[0][ct], raw_s[1][ct], raw_s[2][ct], dt_bias, a.a_floor, Lc, coef);
             if (ct >= 0 && ct < 64) {
                 // The coefficients above were written by other lanes of this wave.
                 __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -1261,7 +1284,7 @@ __device__ __forceinline__ void scan_head(const ScanArgs& a, ScanLds<C, NT, DT>&
             }
             decay_walk<C, (DT <= 2)>(ct, first, coef, w_s);
         }
-        if constexpr (!PREP) {
+        if constexpr (!PREP && !TOK) {
             // tanh(angle) * pi on the waves other than the coefficient wave.
             const int tl = NTH >= 128 ? (tid < 64 ? tid : tid - 64) : tid;
             const bool tw = NTH < 128 || tid < 64 || tid >= 128;
@@ -1531,7 +1554,7 @@ __device__ __forceinline__ void scan_head(const ScanArgs& a, ScanLds<C, NT, DT>&
 // tokens, 8 heads); the others as they fall. Blocks are ordered so that the
 // heads of one window run on one XCD and share its L2 copy of the window's
 // B/C rows.
-template <int C, int NT, int DT>
+template <int C, int NT, int DT, bool TOK>
 __global__ __launch_bounds__(64 * DT) __attribute__((amdgpu_waves_per_eu(DT == 4 ? 4 : 1)))
 void scan_fused_kernel(ScanArgs a) {
     __shared__ ScanLds<C, NT, DT> sh;
@@ -1539,7 +1562,7 @@ void scan_fused_kernel(ScanArgs a) {
     const unsigned Hu = static_cast<unsigned>(a.H), nblk = static_cast<unsigned>(a.B * a.H);
     unsigned lin = blockIdx.x;
     if (nblk % 8 == 0) lin = (lin % 8) * (nblk / 8) + lin / 8;
-    scan_head<C, NT, DT, false>(a, sh, lin / Hu, lin % Hu, 0, NoChunkHooks{});
+    scan_head<C, NT, DT, false, NoChunkHooks, false, false, TOK>(a, sh, lin / Hu, lin % Hu, 0, NoChunkHooks{});
 }
 
 bool aligned16(const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15) == 0; }
@@ -1558,13 +1581,79 @@ ScanMode scan_mode() {
     return ScanMode::kFused;
 }
 
-bool launch_scan_fused(const ScanArgs& s, int64_t N, int64_t D, hipStream_t stream) {
+// What the scan reads of a token besides its B and C rows, formed once for all heads and chunks: the step
+// coefficients of every head, tanh(angle) * pi, and (csum not null) each head's fp64 sum of a chunk's angle terms.
+// One block per (window, chunk).
+__global__ __launch_bounds__(256) void scan_token_kernel(ScanArgs a, int64_t N, int64_t D, float4* coef, float* ang, double* csum) {
+    constexpr int C = 32;
+    extern __shared__ float token_s[];  // [C][R] tanh(angle) pi, [H][C] dt
+    const int H = static_cast<int>(a.H), R = static_cast<int>(a.R), L = static_cast<int>(a.L), chunks = static_cast<int>(a.chunks);
+    const int64_t b = blockIdx.x / static_cast<unsigned>(chunks);
+    const int c = static_cast<int>(blockIdx.x % static_cast<unsigned>(chunks)), c0 = C * c, Lc = L - c0 < C ? L - c0 : C;
+    const float* row = a.proj + b * a.sb + static_cast<int64_t>(c0) * a.st + 2 * H * D + 2 * a.G * N;
+    float* ang_s = token_s;
+    float* dt_s = token_s + C * R;
+    for (int i = threadIdx.x; i < C * H; i += 256) {
+        const int t = i % C, h = i / C;
+        const float* m = row + static_cast<int64_t>(t < Lc ? t : Lc - 1) * a.st + h;
+        const float dt = softplus_f(m[0] + a.dt_bias[h]);
+        const float am = -fmaxf(heavy_tail_f(m[H]), a.a_floor);
+        float al, be, ga;
+        step_coefficients(am * dt, dt, m[2 * H], &al, &be, &ga);
+        const bool valid = t < Lc;
+        dt_s[h * C + t] = dt;
+        coef[((b * H + h) * chunks + c) * C + t] = valid ? make_float4(al, be, ga, dt) : make_float4(0.0f, 0.0f, 0.0f, dt);
+    }
+    for (int i = threadIdx.x; i < C * R; i += 256) {
+        const int t = i / R, r = i - t * R;
+        const float v = tanhf_cr(row[static_cast<int64_t>(t < Lc ? t : Lc - 1) * a.st + 3 * H + r]) * kPiF;
+        ang_s[i] = v;
+        ang[(b * chunks + c) * C * R + i] = v;
+    }
+    if (csum == nullptr) return;
+    __syncthreads();
+    for (int i = threadIdx.x; i < H * R; i += 256) {
+        const int h = i / R, r = i - h * R;
+        double running = 0.0;
+#pragma unroll 8
+        for (int t = 0; t < C; ++t) running += static_cast<double>(ang_s[t * R + r] * dt_s[h * C + t]);
+        csum[((b * H + h) * chunks + c) * R + r] = running;
+    }
+}
+
+size_t scan_token_lds(int64_t H, int64_t R) { return sizeof(float) * 32 * static_cast<size_t>(H + R); }
+
+// Whether the fused scan's per-token values are formed by a launch of their own. Every head's block forms the same
+// tanh(angle) of its window, and its coefficient wave runs two exponentials, a log1p and the decay walk one after
+// another while the others wait. Formed before (4 to 7 us), the scan at d_state 64 takes 255 us with that launch
+// against 267 (2048 pairs x 256 tokens), 250 against 260 (1024 x 480), 118 against 124 (256 x 480); below six chunks
+// the launch eats it (256 x 96: 29 against 27), and smaller states gain nothing (16: 73 against 64 at 1024 x 256).
+bool token_scan_shape(const ScanArgs& s, int64_t N) { return N == 64 && s.chunks >= 6 && s.B * s.H >= 192; }
+
+bool launch_scan_fused(ScanArgs s, int64_t N, int64_t D, void* workspace, size_t bytes, hipStream_t stream) {
     const int NT = static_cast<int>(N / 16), DT = static_cast<int>(D / 16);
     const dim3 grid(static_cast<unsigned>(s.B * s.H));
-#define MLK_FUSED(NTV, DTV)                                                                                  \
-    if (NT == NTV && DT == DTV) {                                                                            \
-        hipLaunchKernelGGL((scan_fused_kernel<32, NTV, DTV>), grid, dim3(64 * DTV), 0, stream, s);          \
-        return true;                                                                                         \
+    s.chunks = (s.L + 31) / 32;
+    const int64_t tokens = s.B * s.chunks * 32;
+    const bool tok = token_scan_shape(s, N) && aligned16(workspace) && s.B * s.chunks < (int64_t{1} << 31) &&
+                     bytes >= sizeof(float) * static_cast<size_t>(tokens * (4 * s.H + s.R)) && scan_token_lds(s.H, s.R) <= 64 * 1024;
+    if (tok) {
+        float4* coef = static_cast<float4*>(workspace);
+        float* ang = reinterpret_cast<float*>(coef + tokens * s.H);
+        s.tok_coef = coef;
+        s.tok_ang = ang;
+    }
+#define MLK_FUSED(NTV, DTV)                                                                                            \
+    if (NT == NTV && DT == DTV) {                                                                                      \
+        if (tok) {                                                                                                     \
+            hipLaunchKernelGGL(scan_token_kernel, dim3(static_cast<unsigned>(s.B * s.chunks)), dim3(256),              \
+                               scan_token_lds(s.H, s.R), stream, s, N, D, const_cast<float4*>(s.tok_coef),             \
+                               const_cast<float*>(s.tok_ang), static_cast<double*>(nullptr));                          \
+            hipLaunchKernelGGL((scan_fused_kernel<32, NTV, DTV, true>), grid, dim3(64 * DTV), 0, stream, s);           \
+        } else {                                                                                                       \
+            hipLaunchKernelGGL((scan_fused_kernel<32, NTV, DTV, false>), grid, dim3(64 * DTV), 0, stream, s);          \
+        }                                                                                                              \
+        return true;                                                                                                   \
     }
     MLK_FUSED(1, 1) MLK_FUSED(1, 2) MLK_FUSED(1, 4) MLK_FUSED(2, 1) MLK_FUSED(2, 2) MLK_FUSED(2, 4)
     MLK_FUSED(4, 1) MLK_FUSED(4, 2) MLK_FUSED(4, 4)
@@ -1635,45 +1724,6 @@ struct SplitScanArgs {
     SplitScan s;
     int64_t N, D;
 };
-
-__global__ __launch_bounds__(256) void split_token_kernel(SplitScanArgs p) {
-    constexpr int C = 32;
-    extern __shared__ float token_s[];  // [C][R] tanh(angle) pi, [H][C] dt
-    const int H = static_cast<int>(p.a.H), R = static_cast<int>(p.a.R), L = static_cast<int>(p.a.L);
-    const int chunks = static_cast<int>(p.s.chunks);
-    const int64_t b = blockIdx.x / chunks;
-    const int c = static_cast<int>(blockIdx.x % chunks), c0 = C * c, Lc = L - c0 < C ? L - c0 : C;
-    const float* row = p.a.proj + b * p.a.sb + static_cast<int64_t>(c0) * p.a.st + 2 * H * p.D + 2 * p.a.G * p.N;
-    float* ang_s = token_s;
-    float* dt_s = token_s + C * R;
-    for (int i = threadIdx.x; i < C * H; i += 256) {
-        const int t = i % C, h = i / C;
-        const float* m = row + static_cast<int64_t>(t < Lc ? t : Lc - 1) * p.a.st + h;
-        const float dt = softplus_f(m[0] + p.a.dt_bias[h]);
-        const float am = -fmaxf(heavy_tail_f(m[H]), p.a.a_floor);
-        float al, be, ga;
-        step_coefficients(am * dt, dt, m[2 * H], &al, &be, &ga);
-        const bool valid = t < Lc;
-        dt_s[h * C + t] = dt;
-        float4* coef = reinterpret_cast<float4*>(p.ws + p.s.coef);
-        coef[((b * H + h) * chunks + c) * C + t] = valid ? make_float4(al, be, ga, dt) : make_float4(0.0f, 0.0f, 0.0f, dt);
-    }
-    for (int i = threadIdx.x; i < C * R; i += 256) {
-        const int t = i / R, r = i - t * R;
-        const float v = tanhf_cr(row[static_cast<int64_t>(t < Lc ? t : Lc - 1) * p.a.st + 3 * H + r]) * kPiF;
-        ang_s[i] = v;
-        p.ws[p.s.ang + (b * chunks + c) * C * R + i] = v;
-    }
-    __syncthreads();
-    double* csum = reinterpret_cast<double*>(p.ws + p.s.csum);
-    for (int i = threadIdx.x; i < H * R; i += 256) {
-        const int h = i / R, r = i - h * R;
-        double running = 0.0;
-#pragma unroll 8
-        for (int t = 0; t < C; ++t) running += static_cast<double>(ang_s[t * R + r] * dt_s[h * C + t]);
-        csum[((b * H + h) * chunks + c) * R + r] = running;
-    }
-}
 
 // (window, head, chunk) of a block; as in scan_fused_kernel the heads of one window run on one XCD.
 __device__ __forceinline__ void split_item(const SplitScanArgs& p, int64_t& b, int& h, int& c) {
@@ -2009,14 +2059,19 @@ bool launch_scan_split(const ScanArgs& s, int64_t N, int64_t D, void* workspace,
     const SplitScan layout = split_layout(s.B, s.L, s.H, N, D, s.R);
     if (!split_scan_shape(s.B, s.L, s.H) || bytes < sizeof(float) * static_cast<size_t>(layout.total) || !aligned16(workspace))
         return false;
-    const SplitScanArgs p{s, static_cast<float*>(workspace), layout, N, D};
+    SplitScanArgs p{s, static_cast<float*>(workspace), layout, N, D};
+    p.a.chunks = layout.chunks;
+    p.a.tok_coef = reinterpret_cast<const float4*>(p.ws + layout.coef);
+    p.a.tok_ang = p.ws + layout.ang;
     const unsigned pairs = static_cast<unsigned>(s.B * s.H), items = pairs * static_cast<unsigned>(layout.chunks);
-    const size_t token_lds = sizeof(float) * 32 * static_cast<size_t>(s.H + s.R);
+    const size_t token_lds = scan_token_lds(s.H, s.R);
     if (token_lds > 64 * 1024) return false;
     const int NT = static_cast<int>(N / 16), DT = static_cast<int>(D / 16);
 #define MLK_SPLIT(NTV, DTV)                                                                                                  \
     if (NT == NTV && DT == DTV) {                                                                                            \
-        hipLaunchKernelGGL(split_token_kernel, dim3(static_cast<unsigned>(s.B * layout.chunks)), dim3(256), token_lds, stream, p); \
+        hipLaunchKernelGGL(scan_token_kernel, dim3(static_cast<unsigned>(s.B * layout.chunks)), dim3(256), token_lds, stream, \
+                           p.a, N, D, reinterpret_cast<float4*>(p.ws + layout.coef), p.ws + layout.ang,                      \
+                           reinterpret_cast<double*>(p.ws + layout.csum));                                                   \
         hipLaunchKernelGGL((split_chunk_kernel<NTV>), dim3(items), dim3(256), 0, stream, p);                                 \
         hipLaunchKernelGGL((split_state_kernel<NTV, DTV>), dim3(pairs), dim3(64 * DTV * (NTV > 1 ? 2 : 1)), 0, stream, p);   \
         hipLaunchKernelGGL((split_out_kernel<NTV, DTV>), dim3(items), dim3(64 * DTV), 0, stream, p);                         \
@@ -3021,7 +3076,7 @@ mlk_status mlk_mamba3_siso_forward(const float* projected, int64_t batch, int64_
         }
         s.out = out;
         if (launch_scan_split(s, d_state, headdim, workspace, workspace_bytes, stream)) return launch_status("mamba3 split scan");
-        if (launch_scan_fused(s, d_state, headdim, stream)) return launch_status("mamba3 fused scan");
+        if (launch_scan_fused(s, d_state, headdim, workspace, workspace_bytes, stream)) return launch_status("mamba3 fused scan");
     }
     const int64_t rw = num_rope_angles > 0 ? num_rope_angles : 1;
     float* q = static_cast<float*>(workspace);

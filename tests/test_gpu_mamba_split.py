@@ -41,6 +41,18 @@ def test_chunk_parallel_scan_equals_unfused(dev, monkeypatch, B, L, N, G, H, D, 
     assert_bitwise(gated, _C.mamba3_siso_forward(proj, gate, *params, *geo).cpu().numpy(), "explicit gate")
 
 
+@pytest.mark.parametrize("B,L,G,H,D,R", [(24, 161, 1, 8, 64, 16), (33, 200, 2, 8, 64, 32), (200, 192, 1, 1, 32, 0),
+                                         (65, 225, 1, 3, 64, 9), (48, 170, 1, 4, 32, 17)])
+def test_scan_with_token_launch_equals_unfused(dev, monkeypatch, B, L, G, H, D, R):
+    """d_state 64 over six chunks and more with many pairs: coefficients and tanh(angle) from a launch of their own."""
+    from montlok import _C
+
+    proj, params, geo = _case(dev, B, L, 64, G, H, D, R)
+    got = _C.mamba3_siso_forward(proj, None, *params, *geo)
+    monkeypatch.setenv("MLK_MAMBA3_SCAN", "unfused")
+    assert_bitwise(got, _C.mamba3_siso_forward(proj, None, *params, *geo).cpu().numpy(), "token launch vs unfused")
+
+
 @pytest.mark.parametrize("B,L,N,G,H,R", [(2, 200, 64, 1, 4, 16), (1, 97, 16, 2, 4, 8)])
 def test_chunk_parallel_scan_headdim16(dev, oracle, monkeypatch, B, L, N, G, H, R):
     from montlok import _C
