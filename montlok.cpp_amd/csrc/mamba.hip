@@ -1960,8 +1960,10 @@ __global__ __launch_bounds__(64 * DT * (NT > 1 ? 2 : 1)) void split_state_kernel
 
 template <int NT, int DT>
 __global__ __launch_bounds__(64 * DT) void split_out_kernel(SplitScanArgs p) {
-    constexpr int C = 32, CT = 2, N = 16 * NT, D = 16 * DT;
+    constexpr int C = 32, CT = 2, N = 16 * NT, D = 16 * DT, NP = N + 4;
     __shared__ float ck_s[C];
+    __shared__ __attribute__((aligned(16))) float q_sh[C * NP];
+    __shared__ float kp_s[N];
     int64_t b;
     int h, c;
     split_item(p, b, h, c);
@@ -1985,30 +1987,25 @@ __global__ __launch_bounds__(64 * DT) void split_out_kernel(SplitScanArgs p) {
             zx[st][v] = load_off32(zc, static_cast<unsigned>(tc * gst32));
         }
     const float vp = first ? 0.0f : xc[-a.st];
-    f32x4_t P[3], S[NT], qf[CT][NT];
+    // q once for the block: every wave multiplies all of it, and the carry's dot products walk its rows.
+    for (int i = threadIdx.x; i < C * N / 4; i += 64 * DT)
+        *reinterpret_cast<float4*>(q_sh + 4 * i / N * NP + 4 * i % N) = *reinterpret_cast<const float4*>(item + p.s.q + 4 * i);
+    if (!first) {
+        for (int i = threadIdx.x; i < N; i += 64 * DT) kp_s[i] = (item - p.s.item)[p.s.last + i];
+    }
+    f32x4_t P[3], S[NT];
 #pragma unroll
     for (int i = 0; i < 3; ++i) P[i] = reinterpret_cast<const f32x4_t*>(item + p.s.P)[i * 64 + lane];
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) {
         // (the first chunk has no state before it: its slot is not written, and not read)
         S[nt] = first ? f32x4_t{0.f, 0.f, 0.f, 0.f} : reinterpret_cast<const f32x4_t*>(item + p.s.S)[(wave * NT + nt) * 64 + lane];
-#pragma unroll
-        for (int tt = 0; tt < CT; ++tt)
-            qf[tt][nt] = *reinterpret_cast<const f32x4_t*>(item + p.s.q + (16 * tt + li) * N + 16 * nt + 4 * g);
     }
     float din[CT][4];
 #pragma unroll
     for (int tt = 0; tt < CT; ++tt)
 #pragma unroll
         for (int v = 0; v < 4; ++v) din[tt][v] = item[p.s.w + C + 16 * tt + 4 * g + v];
-    if (!first && wave == DT - 1 && lane < C) {
-        const float* q = item + p.s.q + lane * N;
-        const float* kp = item - p.s.item + p.s.last;
-        float dot = 0.0f;
-#pragma unroll
-        for (int n = 0; n < N; ++n) dot = fmaf(q[n], kp[n], dot);
-        ck_s[lane] = dot * item[p.s.w + 2 * C + lane];
-    }
     double gz[CT][4];
 #pragma unroll
     for (int tt = 0; tt < CT; ++tt)
@@ -2020,6 +2017,19 @@ __global__ __launch_bounds__(64 * DT) void split_out_kernel(SplitScanArgs p) {
         }
     const float skip = a.skip[h];
     __syncthreads();
+    if (!first && wave == DT - 1 && lane < C) {
+        float dot = 0.0f;
+#pragma unroll
+        for (int n = 0; n < N; n += 4) {
+            const float4 q = *reinterpret_cast<const float4*>(q_sh + lane * NP + n);
+            dot = fmaf(q.x, kp_s[n], dot);
+            dot = fmaf(q.y, kp_s[n + 1], dot);
+            dot = fmaf(q.z, kp_s[n + 2], dot);
+            dot = fmaf(q.w, kp_s[n + 3], dot);
+        }
+        ck_s[lane] = dot * item[p.s.w + 2 * C + lane];
+    }
+    __syncthreads();
     float* ochunk = a.out + (b * a.L + c0) * d_inner + h * D + col;
 #pragma unroll
     for (int tt = 0; tt < CT; ++tt) {
@@ -2030,9 +2040,11 @@ __global__ __launch_bounds__(64 * DT) void split_out_kernel(SplitScanArgs p) {
 #pragma unroll
             for (int v = 0; v < 4; ++v) Y = __builtin_amdgcn_mfma_f32_16x16x4f32(P[tt + st][v], vx[st][v], Y, 0, 0, 0);
 #pragma unroll
-        for (int nt = 0; nt < NT; ++nt)
+        for (int nt = 0; nt < NT; ++nt) {
+            const f32x4_t q4 = *reinterpret_cast<const f32x4_t*>(q_sh + (16 * tt + li) * NP + 16 * nt + 4 * g);
 #pragma unroll
-            for (int v = 0; v < 4; ++v) Yi = __builtin_amdgcn_mfma_f32_16x16x4f32(qf[tt][nt][v], S[nt][v], Yi, 0, 0, 0);
+            for (int v = 0; v < 4; ++v) Yi = __builtin_amdgcn_mfma_f32_16x16x4f32(q4[v], S[nt][v], Yi, 0, 0, 0);
+        }
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
             const int t = 16 * tt + 4 * g + v;
