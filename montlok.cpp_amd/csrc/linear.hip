@@ -30,8 +30,9 @@
 // thousand rows) take linear_small_kernel instead: one wave per 16 x 16
 // output tile, operands straight from L2, no LDS; with few tiles and K beyond
 // 256, linear_small_split_kernel, four waves per tile. fp32 weights with K
-// above 128 otherwise take linear_split.hip's three-plane bf16 form; the fp32
-// forms here then serve K up to 128 and operands that are not 16-byte aligned.
+// above 128 (large calls: 64 and more, but 128) otherwise take linear_split.hip's
+// three-plane bf16 form; the fp32 forms here then serve smaller K, K = 128 and
+// operands that are not 16-byte aligned.
 //
 // K is reduced in an order of its own (the 8 k of a lane, then the four lane
 // groups inside the MFMA); for fp32 weights the result differs from a
@@ -1366,10 +1367,13 @@ int64_t tiles16(int64_t rows, int64_t N) { return ceil_div(rows, 16) * ceil_div(
 
 // fp32 weights with K above 128 go to the three-plane form (linear_split.hip) unless so few 16 x 16 tiles are
 // asked for that one wave per tile ends sooner: its blocks walk K alone, 8 us at K = 256 however few they are,
-// and the one-wave form takes 4.0 us for 300 tiles, 7.6 for 1320 and 9.4 for 1920 (12.1 for 2640). Up to K = 128
-// the forms here are kept (the row-layout form has rms_norm_linear's prologue there).
+// and the one-wave form takes 4.0 us for 300 tiles, 7.6 for 1320 and 9.4 for 1920 (12.1 for 2640). So do large calls
+// with K from 64 to 127 (7680 x 64 -> 384: 8.0 us against the row-layout form's 11.8; 65536 x 64 -> 384 35 against
+// 47); K = 128 keeps that form, which has rms_norm_linear's prologue.
 bool split_shape(const LinearArgs& p) {
-    return p.K > 128 && !(small_shape(p.rows, p.K, p.N) && tiles16(p.rows, p.N) <= 1536) && linear_split_fits(p);
+    const bool small = small_shape(p.rows, p.K, p.N);
+    if (p.K <= 128) return p.K >= 64 && p.K < 128 && !small && linear_split_fits(p);
+    return !(small && tiles16(p.rows, p.N) <= 1536) && linear_split_fits(p);
 }
 
 // Four waves a tile for K in (256, 1024] (linear_small_split_kernel): 31 us -> 6.2 at 480 x 512 -> 256 in fp32
