@@ -2681,7 +2681,23 @@ struct StepArgs {
 // Arithmetic per element is that of the sequence kernel.
 constexpr int kStepThreads = 256;
 
-template <int NM, bool VEC>
+//
+// NTL: the state read past the caches too, as it is always written. A step reads it once; without the hint its
+// lines push out the ones the step's other operands need: 16384 streams x 2 layers (4 heads, 64 x 64) 1150 ->
+// 1080 us, 32768 2126 -> 2024, 3000 295 -> 275, and the same below 1000. At 65536 streams, 4.3 GB a layer, it is
+// the slower form (4083 -> 4243 us), so states of 3 GiB and more are read without it.
+template <int NM, bool NTL>
+__device__ __forceinline__ void load_state(const float* st, int64_t N, int64_t D, float (&sv)[NM]) {
+#pragma unroll
+    for (int n = 0; n < NM; ++n) {
+        if (n < N) {
+            const float* src = st + static_cast<int64_t>(n) * D;
+            sv[n] = NTL ? __builtin_nontemporal_load(src) : *src;
+        }
+    }
+}
+
+template <int NM, bool VEC, bool NTL>
 __global__ __launch_bounds__(kStepThreads) void step_kernel(StepArgs p) {
     extern __shared__ float lds[];
     const int64_t H = p.H, N = p.N, D = p.D, G = p.G, R = p.R;
@@ -2710,11 +2726,7 @@ __global__ __launch_bounds__(kStepThreads) void step_kernel(StepArgs p) {
     float sv[NM];
     const int64_t h_first = wave;
     if (h_first < H && lane < D) {
-        const float* st = p.ssm + ((s_idx * H + h_first) * N) * D + lane;
-#pragma unroll
-        for (int n = 0; n < NM; ++n) {
-            if (n < N) sv[n] = st[static_cast<int64_t>(n) * D];
-        }
+        load_state<NM, NTL>(p.ssm + ((s_idx * H + h_first) * N) * D + lane, N, D, sv);
     }
 
     // 2. Per-stream set-up, from the row slice staged in LDS.
@@ -2771,12 +2783,7 @@ __global__ __launch_bounds__(kStepThreads) void step_kernel(StepArgs p) {
         const int d = lane;
         if (d >= D) continue;
         float* st = p.ssm + ((s_idx * H + h) * N) * D + d;
-        if (h != h_first) {
-#pragma unroll
-            for (int n = 0; n < NM; ++n) {
-                if (n < N) sv[n] = st[static_cast<int64_t>(n) * D];
-            }
-        }
+        if (h != h_first) load_state<NM, NTL>(st, N, D, sv);
         const float al = co[4 * h], be = co[4 * h + 1], ga = co[4 * h + 2];
         const float* x = row + d_inner + h * D;
         const float* z = row + h * D;
@@ -3215,19 +3222,23 @@ mlk_status mlk_mamba3_siso_step(const float* projected, int64_t streams, int64_t
     MLK_CHECK(lds_bytes <= 64 * 1024, "too many heads x d_state for the GPU step");
     MLK_CHECK(streams <= 0x7fffffff, "too many streams for one launch");
     const dim3 grid(static_cast<unsigned>(streams));
-#define MLK_STEP(NM)                                                                                         \
-    do {                                                                                                     \
-        if (vec) {                                                                                           \
-            hipLaunchKernelGGL((step_kernel<NM, true>), grid, dim3(kStepThreads), lds_bytes, stream, p);     \
-        } else {                                                                                             \
-            hipLaunchKernelGGL((step_kernel<NM, false>), grid, dim3(kStepThreads), lds_bytes, stream, p);    \
-        }                                                                                                    \
-        return launch_status("mamba3 step");                                                                 \
+    const bool ntl = streams * nheads * d_state * headdim < (int64_t{3} << 28);  // floats: 3 GiB
+#define MLK_STEP_LAUNCH(NM, VEC, NTL)                                                                            \
+    if (vec == VEC && ntl == NTL) {                                                                              \
+        hipLaunchKernelGGL((step_kernel<NM, VEC, NTL>), grid, dim3(kStepThreads), lds_bytes, stream, p);         \
+        return launch_status("mamba3 step");                                                                     \
+    }
+#define MLK_STEP(NM)                                                                                             \
+    do {                                                                                                         \
+        MLK_STEP_LAUNCH(NM, true, true) MLK_STEP_LAUNCH(NM, true, false)                                         \
+        MLK_STEP_LAUNCH(NM, false, true) MLK_STEP_LAUNCH(NM, false, false)                                       \
     } while (0)
     if (d_state <= 16) MLK_STEP(16);
     if (d_state <= 64) MLK_STEP(64);
     MLK_STEP(128);
+    return MLK_OK;  // (not reached)
 #undef MLK_STEP
+#undef MLK_STEP_LAUNCH
 }
 
 mlk_status mlk_rms_norm_mamba3_forward(const float* x, int64_t batch, int64_t length, int64_t d_model,
