@@ -17,7 +17,7 @@
 //
 //   block  = 64 rows x 64 columns of y, 4 waves of 32 x 32; K in steps of 32.
 //            Large calls: 128 x 128, 4 waves of 64 x 64 that multiply and 4 that
-//            stage, two LDS buffers.
+//            stage, two LDS buffers. Up to 256 blocks: 8 waves, two a tile.
 //   stage  = 16-row pieces of x and W, whole 128-byte lines per load (the
 //            MFMA operand order straight from memory takes every line in four
 //            separate instructions: 20-25% slower), split in registers and
@@ -74,7 +74,7 @@ __device__ __forceinline__ uint32_t take_bf16(f32x2& v) {
 // the chunks of a group combined highest index bit first, as tile_rms_norm and rms_norm_vec_kernel do.
 template <int GS>
 __device__ __forceinline__ void norm_scales(const LinearArgs& p, int64_t row0, int groups, double* scale) {
-    for (int u = threadIdx.x; u < kBlock * groups; u += 256) {
+    for (int u = threadIdx.x; u < kBlock * groups; u += blockDim.x) {
         const int64_t row = row0 + u / groups;
         const float* x = p.x + (row < p.rows ? row : p.rows - 1) * p.x_stride + (u % groups) * GS;
         double part[GS / 4];
@@ -99,16 +99,20 @@ __device__ __forceinline__ void norm_scales(const LinearArgs& p, int64_t row0, i
 // 2 N columns then never reach memory: 7680 x 256 -> 2 x 512 36 us, against 38 for the linear and 13 for swiglu.
 // T: the wave tile is (32 T) x (32 T), the block (64 T) x (64 T). T = 2 has four more waves that stage (PRODUCER
 // below) while the first four multiply, with two LDS buffers and one barrier a step.
-template <bool FULL, int GS, bool SWIGLU, int T>
-__global__ __launch_bounds__(T == 1 ? 256 : 512, T == 1 ? 1 : 2) void linear_split_kernel(LinearArgs p, unsigned n_blocks) {
-    static_assert(T == 1 || GS == 0, "the norm's prologue is the 64 x 64 block's");
+// PAIR (T = 1, few blocks): eight waves to the 64 x 64 block, two to a tile, one for each k half of a step; their
+// sums meet in LDS.
+template <bool FULL, int GS, bool SWIGLU, int T, bool PAIR>
+__global__ __launch_bounds__(T == 1 && !PAIR ? 256 : 512, T == 1 ? 1 : 2) void linear_split_kernel(LinearArgs p, unsigned n_blocks) {
+    static_assert(T == 1 || (GS == 0 && !PAIR), "the norm's prologue and the pairs are the 64 x 64 block's");
+    constexpr int MS = PAIR ? 1 : 2;  // 8-row loads a staging wave issues per 64 rows
     constexpr int kRows = kBlock * T, kCols = SWIGLU ? kRows / 2 : kRows;  // rows, output columns of the block
     constexpr int kBuffer = 4 * T * kTileUnits;  // x tiles 0 .. 2 T - 1, then W tiles
     __shared__ uint4 frag[T * kBuffer];
     __shared__ double scale[GS > 0 ? kBlock * kMaxNormGroups : 1];
     const int lane = threadIdx.x & 63, li = lane & 31, g = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) & 3;
-    const bool producer = T == 1 || __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) >= 4;
+    const int upper = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);  // 1: T = 2's staging waves, a pair's second
+    const bool producer = T == 1 || upper == 1;
     // XCD x takes the x-th eighth of the blocks, column blocks of one row block side by side: a row block's x
     // is fetched into one L2.
     unsigned lin = blockIdx.x;
@@ -123,19 +127,19 @@ __global__ __launch_bounds__(T == 1 ? 256 : 512, T == 1 ? 1 : 2) void linear_spl
     // row r (of 8), whole lines; byte offsets in 32 bits from the block's first row (strides checked at launch).
     const int sr = lane >> 3, sc = lane & 7;
     const char* base[2] = {reinterpret_cast<const char*>(p.x + row0 * p.x_stride), reinterpret_cast<const char*>(w + n0 * p.K)};
-    unsigned off[2][T][2];
-    float4 v[2][T][2], nw;
+    unsigned off[2][T][MS];
+    float4 v[2][T][MS], nw;
     bool live = true;  // of the fetched step (K a multiple of 4: a lane's 4 k are on one side of it)
     auto rows = [&]() {
 #pragma unroll
         for (int i = 0; i < T; ++i)
 #pragma unroll
-            for (int m = 0; m < 2; ++m) {
-                const int r = 64 * i + 16 * wave + 8 * m + sr;
+            for (int m = 0; m < MS; ++m) {
+                const int r = 64 * i + 16 * wave + 8 * (PAIR ? upper : m) + sr;
                 off[0][i][m] = static_cast<unsigned>((row0 + r < p.rows ? r : p.rows - 1 - row0) * p.x_stride * 4) + 16 * sc;
                 int64_t n = r;
                 if constexpr (SWIGLU) {
-                    const int64_t col = 32 * i + 16 * (wave >> 1) + 8 * m + sr;
+                    const int64_t col = 32 * i + 16 * (wave >> 1) + 8 * (PAIR ? upper : m) + sr;
                     n = (n0 + col < p.N ? col : p.N - 1 - n0) + (wave & 1 ? p.N : 0);
                 } else {
                     n = n0 + n < p.N ? n : p.N - 1 - n0;
@@ -151,7 +155,7 @@ __global__ __launch_bounds__(T == 1 ? 256 : 512, T == 1 ? 1 : 2) void linear_spl
 #pragma unroll
             for (int i = 0; i < T; ++i)
 #pragma unroll
-                for (int m = 0; m < 2; ++m)
+                for (int m = 0; m < MS; ++m)
                     v[o][i][m] = *reinterpret_cast<const float4*>(base[o] + static_cast<unsigned>(off[o][i][m] + ko));
         if constexpr (GS > 0) nw = *reinterpret_cast<const float4*>(p.norm_w + (live ? k0 + 4 * sc : 0));
     };
@@ -163,11 +167,12 @@ __global__ __launch_bounds__(T == 1 ? 256 : 512, T == 1 ? 1 : 2) void linear_spl
 #pragma unroll
             for (int i = 0; i < T; ++i)
 #pragma unroll
-                for (int m = 0; m < 2; ++m) {
+                for (int m = 0; m < MS; ++m) {
+                    const int r8 = 8 * (PAIR ? upper : m) + sr;  // of the wave's 16 rows
                     float4 f = v[o][i][m];
                     if (GS > 0 && o == 0) {
                         const int k = live ? k0 + 4 * sc : 0;
-                        const double s = scale[(16 * wave + 8 * m + sr) * groups + k / (GS > 0 ? GS : 1)];
+                        const double s = scale[(16 * wave + r8) * groups + k / (GS > 0 ? GS : 1)];
                         f.x = static_cast<float>((static_cast<double>(f.x) * s) * static_cast<double>(nw.x));
                         f.y = static_cast<float>((static_cast<double>(f.y) * s) * static_cast<double>(nw.y));
                         f.z = static_cast<float>((static_cast<double>(f.z) * s) * static_cast<double>(nw.z));
@@ -175,7 +180,7 @@ __global__ __launch_bounds__(T == 1 ? 256 : 512, T == 1 ? 1 : 2) void linear_spl
                     }
                     if (!FULL && !live) f = float4{0.0f, 0.0f, 0.0f, 0.0f};
                     f32x2 lo = {f.x, f.y}, hi = {f.z, f.w};
-                    const unsigned slot = unit(2 * (o * T + i) + (wave >> 1), sc >> 2, 0, (sc >> 1) & 1) + 16 * (wave & 1) + 8 * m + sr;
+                    const unsigned slot = unit(2 * (o * T + i) + (wave >> 1), sc >> 2, 0, (sc >> 1) & 1) + 16 * (wave & 1) + r8;
 #pragma unroll
                     for (int q = 0; q < kPlanes; ++q) dst[2 * (slot + q * 2 * kGroupUnits) + (sc & 1)] = uint2{take_bf16(lo), take_bf16(hi)};
                 }
@@ -192,7 +197,8 @@ __global__ __launch_bounds__(T == 1 ? 256 : 512, T == 1 ? 1 : 2) void linear_spl
     auto multiply = [&](int buffer) {
         const uint4* src = frag + buffer * kBuffer;
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
+        for (int hh = 0; hh < (PAIR ? 1 : 2); ++hh) {
+            const int h = PAIR ? upper : hh;
             bf16x8 xf[T][kPlanes], wf[T][kPlanes];
 #pragma unroll
             for (int q = 0; q < kPlanes; ++q)
@@ -249,6 +255,20 @@ __global__ __launch_bounds__(T == 1 ? 256 : 512, T == 1 ? 1 : 2) void linear_spl
         }
     }
 
+    if constexpr (PAIR) {
+        // (the fragments of the last step are done with: their LDS takes the second waves' sums)
+        float* part = reinterpret_cast<float*>(frag) + wave * 16 * 64 + lane;
+        static_assert(sizeof(frag) >= 4 * 16 * 64 * sizeof(float), "the sums fit the fragments' LDS");
+        __syncthreads();
+        if (upper == 1) {
+#pragma unroll
+            for (int c = 0; c < 16; ++c) part[64 * c] = acc[0][0][c] + low[0][0][c];
+        }
+        __syncthreads();
+        if (upper == 1) return;
+#pragma unroll
+        for (int c = 0; c < 16; ++c) low[0][0][c] += part[64 * c];
+    }
     const bool vec_out = (reinterpret_cast<uintptr_t>(p.out) & 15) == 0 && p.out_stride % 4 == 0 &&
                          (p.residual == nullptr ||
                           ((reinterpret_cast<uintptr_t>(p.residual) & 15) == 0 && p.res_stride % 4 == 0));
@@ -322,14 +342,14 @@ __global__ __launch_bounds__(T == 1 ? 256 : 512, T == 1 ? 1 : 2) void linear_spl
     }
 }
 
-template <int GS, bool SWIGLU, int T>
+template <int GS, bool SWIGLU, int T, bool PAIR = false>
 void launch_blocks(const LinearArgs& p, hipStream_t stream) {
     const int64_t nb = ceil_div(p.N, (SWIGLU ? kBlock / 2 : kBlock) * T);
-    const dim3 grid(static_cast<unsigned>(ceil_div(p.rows, kBlock * T) * nb)), threads(T == 1 ? 256 : 512);
+    const dim3 grid(static_cast<unsigned>(ceil_div(p.rows, kBlock * T) * nb)), threads(T == 1 && !PAIR ? 256 : 512);
     if (p.K % kStep == 0) {
-        hipLaunchKernelGGL((linear_split_kernel<true, GS, SWIGLU, T>), grid, threads, 0, stream, p, static_cast<unsigned>(nb));
+        hipLaunchKernelGGL((linear_split_kernel<true, GS, SWIGLU, T, PAIR>), grid, threads, 0, stream, p, static_cast<unsigned>(nb));
     } else {
-        hipLaunchKernelGGL((linear_split_kernel<false, GS, SWIGLU, T>), grid, threads, 0, stream, p, static_cast<unsigned>(nb));
+        hipLaunchKernelGGL((linear_split_kernel<false, GS, SWIGLU, T, PAIR>), grid, threads, 0, stream, p, static_cast<unsigned>(nb));
     }
 }
 
@@ -344,6 +364,12 @@ bool fills_big_blocks(int64_t rows, int64_t w_rows) {
     return static_cast<double>(rows) * static_cast<double>(w_rows) >= 0.9 * held;
 }
 
+// Up to one 64 x 64 block a CU, a step is a chain of one wave a SIMD (load, split, products); eight waves halve its
+// parts: 480 x 512 -> 256 13.1 -> 11.2 us, 3840 x 256 -> 256 (240 blocks) 8.7 -> 8.0, 3840 x 1024 -> 256 25.8 -> 21.2.
+// Past that the second block of a CU fills the gaps as well: 2880 x 256 -> 352 (270 blocks) 10.0 in both, 5760 x 256 ->
+// 256 (360) 10.4 against 10.7, 2880 x 256 -> 1192 (855) 17.7 against 20.0.
+bool few_blocks(int64_t rows, int64_t w_rows) { return ceil_div(rows, kBlock) * ceil_div(w_rows, kBlock) <= 256; }
+
 template <int GS, bool SWIGLU>
 void launch(const LinearArgs& p, hipStream_t stream) {
     if constexpr (GS == 0) {
@@ -352,7 +378,11 @@ void launch(const LinearArgs& p, hipStream_t stream) {
             return;
         }
     }
-    launch_blocks<GS, SWIGLU, 1>(p, stream);
+    if (few_blocks(p.rows, SWIGLU ? 2 * p.N : p.N)) {
+        launch_blocks<GS, SWIGLU, 1, true>(p, stream);
+    } else {
+        launch_blocks<GS, SWIGLU, 1>(p, stream);
+    }
 }
 
 // 32-bit byte offsets from a block's first rows, and the grid.
