@@ -191,15 +191,54 @@ __device__ __forceinline__ void sincos_d(double x, double* sine, double* cosine)
     *cosine = co;
 }
 
-// Sum over aligned groups of `width` lanes (width a power of two <= 64);
-// every lane of a group receives the group total.
+// v + shfl_xor_d(v, MASK), MASK 16 or 32, in every lane of the wave, by gfx950's
+// row swaps instead of the LDS crossbar: swap(x, x) leaves one partner's value in
+// both lanes of a pair and the other's in the second result (the sum commutes).
+template <int MASK>
+__device__ __forceinline__ double add_cross_row_d(double v) {
+    static_assert(MASK == 16 || MASK == 32, "a partner in another row of 16 lanes");
+    const int lo = __double2loint(v), hi = __double2hiint(v);
+    if constexpr (MASK == 16) {
+        const auto l = __builtin_amdgcn_permlane16_swap(lo, lo, false, false);
+        const auto h = __builtin_amdgcn_permlane16_swap(hi, hi, false, false);
+        return __hiloint2double(h[0], l[0]) + __hiloint2double(h[1], l[1]);
+    } else {
+        const auto l = __builtin_amdgcn_permlane32_swap(lo, lo, false, false);
+        const auto h = __builtin_amdgcn_permlane32_swap(hi, hi, false, false);
+        return __hiloint2double(h[0], l[0]) + __hiloint2double(h[1], l[1]);
+    }
+}
+
+// N sums over aligned groups of `width` lanes (width a power of two <= 64, the
+// same in every lane), the N chains side by side; every lane of a group receives
+// the group's totals. All lanes of the wave are active.
+template <int N>
+__device__ __forceinline__ void group_sums_d(double (&v)[N], int width) {
+    if (width > 32)
+#pragma unroll
+        for (int i = 0; i < N; ++i) v[i] = add_cross_row_d<32>(v[i]);
+    if (width > 16)
+#pragma unroll
+        for (int i = 0; i < N; ++i) v[i] = add_cross_row_d<16>(v[i]);
+    if (width > 8)
+#pragma unroll
+        for (int i = 0; i < N; ++i) v[i] += xor_row_d<8>(v[i]);
+    if (width > 4)
+#pragma unroll
+        for (int i = 0; i < N; ++i) v[i] += xor_row_d<4>(v[i]);
+    if (width > 2)
+#pragma unroll
+        for (int i = 0; i < N; ++i) v[i] += xor_row_d<2>(v[i]);
+    if (width > 1)
+#pragma unroll
+        for (int i = 0; i < N; ++i) v[i] += xor_row_d<1>(v[i]);
+}
+
 template <int width>
 __device__ __forceinline__ double group_sum_d(double v) {
-#pragma unroll
-    for (int mask = width / 2; mask > 0; mask >>= 1) {
-        v += shfl_xor_d(v, mask);
-    }
-    return v;
+    double s[1] = {v};
+    group_sums_d(s, width);
+    return s[0];
 }
 
 }  // namespace mlk

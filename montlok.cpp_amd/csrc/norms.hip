@@ -100,17 +100,21 @@ __global__ __launch_bounds__(kBlock) void rms_norm_vec_kernel(const float* __res
 #pragma unroll
         for (int c = 0; c < CPL; ++c)
             wv[r][c] = *reinterpret_cast<const float4*>(w + g[r] * gs + static_cast<int64_t>(c * LPG + li) * 4);
+    double sumsq[RPW];
 #pragma unroll
     for (int r = 0; r < RPW; ++r) {
-        double sumsq = 0.0;
+        sumsq[r] = 0.0;
 #pragma unroll
         for (int c = 0; c < CPL; ++c) {
             const double a = v[r][c].x, b = v[r][c].y, cc = v[r][c].z, d = v[r][c].w;
-            sumsq += (a * a + b * b) + (cc * cc + d * d);
+            sumsq[r] += (a * a + b * b) + (cc * cc + d * d);
         }
-        sumsq = group_sum_d<LPG>(sumsq);
+    }
+    group_sums_d(sumsq, LPG);
+#pragma unroll
+    for (int r = 0; r < RPW; ++r) {
         if (!active[r]) continue;
-        const double scale = 1.0 / sqrt(sumsq / static_cast<double>(gs) + eps);
+        const double scale = 1.0 / sqrt(sumsq[r] / static_cast<double>(gs) + eps);
         float* og = out + row[r] * dim + g[r] * gs;
 #pragma unroll
         for (int c = 0; c < CPL; ++c) {
@@ -219,7 +223,8 @@ __global__ __launch_bounds__(kBlock) void layer_norm_vec_kernel(const float* __r
                                                                 void* __restrict__ out) {
     // LPG lanes per row: dim = 4 * CPL * LPG with LPG = 64 / rows-per-wave. RPW rows per lane group, all
     // their loads issued first (as rms_norm_vec_kernel): row r of block b's lane group k is
-    // (b RPW + r) (256 / LPG) + k.
+    // (b RPW + r) (256 / LPG) + k. Bound by HBM once a wave's rows no longer sum one after another through the
+    // LDS crossbar: 262144 x 256, RMSNorm and LayerNorm, 195 -> 190 us with the rows' sums side by side in the VALU.
     const int lpg = static_cast<int>(dim / (4 * CPL));
     const int li = threadIdx.x % lpg;
     int64_t row[RPW];
@@ -243,34 +248,41 @@ __global__ __launch_bounds__(kBlock) void layer_norm_vec_kernel(const float* __r
         if (bias == nullptr) bv[c] = make_float4(0.f, 0.f, 0.f, 0.f);
     }
     const double inv_dim = 1.0 / static_cast<double>(dim);
+    double mean[RPW], sumsq[RPW];
 #pragma unroll
     for (int r = 0; r < RPW; ++r) {
-        double sum = 0.0;
+        mean[r] = 0.0;
 #pragma unroll
         for (int c = 0; c < CPL; ++c) {
-            sum += (static_cast<double>(v[r][c].x) + static_cast<double>(v[r][c].y)) +
-                   (static_cast<double>(v[r][c].z) + static_cast<double>(v[r][c].w));
+            mean[r] += (static_cast<double>(v[r][c].x) + static_cast<double>(v[r][c].y)) +
+                       (static_cast<double>(v[r][c].z) + static_cast<double>(v[r][c].w));
         }
-        for (int mask = lpg / 2; mask > 0; mask >>= 1) sum += shfl_xor_d(sum, mask);
-        const double mean = sum * inv_dim;
-        double sumsq = 0.0;
+    }
+    group_sums_d(mean, lpg);
+#pragma unroll
+    for (int r = 0; r < RPW; ++r) {
+        mean[r] *= inv_dim;
+        sumsq[r] = 0.0;
 #pragma unroll
         for (int c = 0; c < CPL; ++c) {
-            const double a = static_cast<double>(v[r][c].x) - mean, b = static_cast<double>(v[r][c].y) - mean;
-            const double cc = static_cast<double>(v[r][c].z) - mean, d = static_cast<double>(v[r][c].w) - mean;
-            sumsq += (a * a + b * b) + (cc * cc + d * d);
+            const double a = static_cast<double>(v[r][c].x) - mean[r], b = static_cast<double>(v[r][c].y) - mean[r];
+            const double cc = static_cast<double>(v[r][c].z) - mean[r], d = static_cast<double>(v[r][c].w) - mean[r];
+            sumsq[r] += (a * a + b * b) + (cc * cc + d * d);
         }
-        for (int mask = lpg / 2; mask > 0; mask >>= 1) sumsq += shfl_xor_d(sumsq, mask);
+    }
+    group_sums_d(sumsq, lpg);
+#pragma unroll
+    for (int r = 0; r < RPW; ++r) {
         if (!active[r]) continue;
-        const double rstd = 1.0 / sqrt(fma(sumsq, inv_dim, eps));
+        const double rstd = 1.0 / sqrt(fma(sumsq[r], inv_dim, eps));
 #pragma unroll
         for (int c = 0; c < CPL; ++c) {
             const int off = (c * lpg + li) * 4;
             float4 o;
-            o.x = static_cast<float>(((static_cast<double>(v[r][c].x) - mean) * rstd) * wv[c].x + static_cast<double>(bv[c].x));
-            o.y = static_cast<float>(((static_cast<double>(v[r][c].y) - mean) * rstd) * wv[c].y + static_cast<double>(bv[c].y));
-            o.z = static_cast<float>(((static_cast<double>(v[r][c].z) - mean) * rstd) * wv[c].z + static_cast<double>(bv[c].z));
-            o.w = static_cast<float>(((static_cast<double>(v[r][c].w) - mean) * rstd) * wv[c].w + static_cast<double>(bv[c].w));
+            o.x = static_cast<float>(((static_cast<double>(v[r][c].x) - mean[r]) * rstd) * wv[c].x + static_cast<double>(bv[c].x));
+            o.y = static_cast<float>(((static_cast<double>(v[r][c].y) - mean[r]) * rstd) * wv[c].y + static_cast<double>(bv[c].y));
+            o.z = static_cast<float>(((static_cast<double>(v[r][c].z) - mean[r]) * rstd) * wv[c].z + static_cast<double>(bv[c].z));
+            o.w = static_cast<float>(((static_cast<double>(v[r][c].w) - mean[r]) * rstd) * wv[c].w + static_cast<double>(bv[c].w));
             if constexpr (BF16OUT) {
                 auto hb = [](float f) { return static_cast<uint32_t>(__builtin_bit_cast(uint16_t, static_cast<__bf16>(f))); };
                 *reinterpret_cast<uint2*>(static_cast<uint16_t*>(out) + row[r] * dim + off) =
