@@ -1369,10 +1369,13 @@ int64_t tiles16(int64_t rows, int64_t N) { return ceil_div(rows, 16) * ceil_div(
 // asked for that one wave per tile ends sooner: its blocks walk K alone, 8 us at K = 256 however few they are,
 // and the one-wave form takes 4.0 us for 300 tiles, 7.6 for 1320 and 9.4 for 1920 (12.1 for 2640). So do large calls
 // with K from 64 to 127 (7680 x 64 -> 384: 8.0 us against the row-layout form's 11.8; 65536 x 64 -> 384 35 against
-// 47); K = 128 keeps that form, which has rms_norm_linear's prologue.
+// 47). At K = 128, where rms_norm_linear (which gives linear's bits) has a row-layout form, up to 3072 of the 64 x 64
+// blocks: 16384 x 128 -> 668 39 -> 27 us, with the norm 41.6 -> 39.8; 6000 rows 23.8 -> 14.2 and 32.6 -> 19.1. Past
+// that every column block's copy of the norm's sums costs more than the products save (65536 rows: 115 -> 133).
 bool split_shape(const LinearArgs& p) {
     const bool small = small_shape(p.rows, p.K, p.N);
-    if (p.K <= 128) return p.K >= 64 && p.K < 128 && !small && linear_split_fits(p);
+    if (p.K < 128) return p.K >= 64 && !small && linear_split_fits(p);
+    if (p.K == 128) return !small && ceil_div(p.rows, 64) * ceil_div(p.N, 64) <= 3072 && linear_split_fits(p);
     return !(small && tiles16(p.rows, p.N) <= 1536) && linear_split_fits(p);
 }
 
@@ -1598,7 +1601,7 @@ extern "C" mlk_status mlk_rms_norm_linear(const float* x, int64_t rows, int64_t 
     const bool vec = aligned16(x) && x_stride % 4 == 0 && aligned16(weight) && (in_features * wsize) % 16 == 0 &&
                      aligned16(norm_weight);
     const bool gs_ok = gs == 8 || gs == 16 || gs == 32 || gs == 64;
-    // Large row counts: the row-layout kernel with the prologue, for fp32 weights and K of one chunk.
+    // Large row counts: fp32 weights and K of one chunk, on the three planes or the row-layout kernel's prologue.
     const bool rows_form = vec && gs_ok && !small_shape(rows, in_features, out_features) &&
                            weight_dtype == MLK_DTYPE_F32 && in_features == WTraits<false>::kKChunk;
     if (!vec || !gs_ok || !(small_shape(rows, in_features, out_features) || rows_form)) {
@@ -1610,7 +1613,7 @@ extern "C" mlk_status mlk_rms_norm_linear(const float* x, int64_t rows, int64_t 
     LinearArgs p{x, rows, in_features, x_stride, weight, bias, out_features, out, out_stride, nullptr, 0,
                  norm_weight, static_cast<double>(static_cast<float>(eps))};
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-    if (rows_form) {
+    if (rows_form && !split_shape(p)) {
         MLK_CHECK(ceil_div(rows, kRowsPerBlock) <= 0x7fffffff, "too many rows");
         const int64_t n_chunks = ceil_div(out_features, kColsPerChunk);
         const int64_t row_blocks = ceil_div(rows, kRowsPerBlock);
@@ -1635,7 +1638,7 @@ extern "C" mlk_status mlk_rms_norm_linear(const float* x, int64_t rows, int64_t 
 #undef MLK_ROWS_GS
         return launch_status("rms_norm_linear");
     }
-    // Where linear takes the three-plane form, so does this (at most 256 of K: a small shape).
+    // Where linear takes the three-plane form, so does this.
     if (weight_dtype == MLK_DTYPE_F32 && split_shape(p)) {
         launch_linear_split_norm(p, gs, s);
         return launch_status("rms_norm_linear");
