@@ -36,9 +36,14 @@
 // 15360 x 512 -> 256 52 -> 26.
 //
 // Parts of an infinity or of a value that rounds to bf16 infinity are
-// inf and -inf (or NaN), so a result that involves one is NaN; such results
-// (and any other NaN) are formed again as a plain fp32 sum, which is infinite
-// or NaN where the fp32 product is.
+// inf and -inf (or NaN), so a result that involves one is NaN. A wave with a
+// NaN among its results that no NaN of the x row explains forms its tile again
+// on the fp32 matrix cores (plain_tile) and takes the NaN ones from there:
+// infinite or NaN where the fp32 products are. Rows with a NaN are ordinary
+// input (bars that are missing), so looking for it has to be cheap, and a
+// serial sum of a lane's 16 results is not: 7680 x 512 -> 256 with one such
+// row 513 us so, 28 with the look and 37 with the tile (22 without the row);
+// all rows 1900 and 31.
 
 #include "linear_args.h"
 #include "mlk_common.h"
@@ -90,6 +95,61 @@ __device__ __forceinline__ void norm_scales(const LinearArgs& p, int64_t row0, i
             for (int c = 0; c < n; ++c) part[c] += part[c + n];
         scale[u] = 1.0 / sqrt(part[0] / static_cast<double>(GS) + p.norm_eps);
     }
+}
+
+// A wave's 32 x 32 tile of sums on the fp32 matrix cores, as linear's fp32 forms take them: lane (g, l) passes the
+// k 8 s + 4 g .. + 3 of its own row of x and of W (for GS > 0 normalised as norm_scales' row scales say), read from
+// memory, and gets row l of x, W rows 8 j + 4 g .. + 3. All lanes of the wave are active.
+template <int GS>
+__device__ __forceinline__ f32x16 plain_tile(const float* x, const float* w, int K, int g, const double* scale, const float* norm_w) {
+    constexpr int kAhead = 4;  // 8-wide steps whose loads are in flight together
+    f32x16 sum;
+#pragma unroll
+    for (int c = 0; c < 16; ++c) sum[c] = 0.0f;
+#pragma unroll 1
+    for (int k0 = 0; k0 < K; k0 += 8 * kAhead) {
+        float4 xv[kAhead], wv[kAhead];
+#pragma unroll
+        for (int s = 0; s < kAhead; ++s) {
+            const int k = k0 + 8 * s + 4 * g, kc = k < K ? k : 0;
+            xv[s] = *reinterpret_cast<const float4*>(x + kc);
+            wv[s] = *reinterpret_cast<const float4*>(w + kc);
+        }
+#pragma unroll
+        for (int s = 0; s < kAhead; ++s) {
+            const int k = k0 + 8 * s + 4 * g;
+            const bool live = k < K;
+            float xs[4] = {xv[s].x, xv[s].y, xv[s].z, xv[s].w}, ws[4] = {wv[s].x, wv[s].y, wv[s].z, wv[s].w};
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                if constexpr (GS > 0) {
+                    const int kc = live ? k : 0;
+                    xs[j] = static_cast<float>((static_cast<double>(xs[j]) * scale[kc / GS]) * static_cast<double>(norm_w[kc + j]));
+                }
+                sum = __builtin_amdgcn_mfma_f32_32x32x2f32(live ? ws[j] : 0.0f, live ? xs[j] : 0.0f, sum, 0, 0, 0);
+            }
+        }
+    }
+    return sum;
+}
+
+// Whether row l of x (lanes l and l + 32, K floats) holds a NaN.
+__device__ __forceinline__ bool row_has_nan(const float* x, int K, int g, int li) {
+    constexpr int kAhead = 8;
+    bool found = false;
+#pragma unroll 1
+    for (int k0 = 0; k0 < K; k0 += 8 * kAhead) {
+        float4 v[kAhead];
+#pragma unroll
+        for (int s = 0; s < kAhead; ++s) {
+            const int k = k0 + 8 * s + 4 * g;
+            v[s] = *reinterpret_cast<const float4*>(x + (k < K ? k : 0));
+        }
+#pragma unroll
+        for (int s = 0; s < kAhead; ++s) found = found || __builtin_isunordered(v[s].x, v[s].y) || __builtin_isunordered(v[s].z, v[s].w);
+    }
+    const uint64_t lanes = __ballot(found);
+    return ((lanes | lanes >> 32) >> li & 1) != 0;
 }
 
 // FULL: K a multiple of the step. GS > 0: the grouped RMSNorm of x (groups of GS floats, at most kMaxNormGroups
@@ -275,7 +335,8 @@ __global__ __launch_bounds__(T == 1 && !PAIR ? 256 : 512, T == 1 ? 1 : 2) void l
 #pragma unroll
     for (int i = 0; i < T; ++i) {
         const int64_t row = row0 + 32 * (wm * T + i) + li;
-        if (row >= p.rows) continue;
+        const float* xr = p.x + (row < p.rows ? row : p.rows - 1) * p.x_stride;
+        bool looked = false, nan_row = false;  // (looked: the same in every lane)
 #pragma unroll
         for (int t = 0; t < T; ++t) {
             f32x16& y = acc[i][t];
@@ -291,28 +352,24 @@ __global__ __launch_bounds__(T == 1 && !PAIR ? 256 : 512, T == 1 ? 1 : 2) void l
                 if constexpr (SWIGLU) return w_row(c & 7) < p.N;
                 return w_row(c) < p.N;
             };
-            bool finite = true;
+            bool whole = true;
 #pragma unroll
-            for (int c = 0; c < 16; ++c) finite = finite && y[c] == y[c];
-            if (!finite) {
-#pragma unroll 1
-                for (int c = 0; c < 16; ++c) {
-                    if (!in_range(c)) continue;
-                    const float* xr = p.x + row * p.x_stride;
-                    const float* wr = w + w_row(c) * p.K;
-                    float sum = 0.0f;
-#pragma unroll 1
-                    for (int k = 0; k < K; ++k) {
-                        float x = xr[k];
-                        if constexpr (GS > 0)
-                            x = static_cast<float>((static_cast<double>(x) * scale[(32 * wm + li) * groups + k / GS]) *
-                                                   static_cast<double>(p.norm_w[k]));
-                        sum = fmaf(x, wr[k], sum);
-                    }
-#pragma unroll
-                    for (int e = 0; e < 16; ++e) y[e] = e == c && y[e] != y[e] ? sum : y[e];
-                }
+            for (int c = 0; c < 16; ++c) whole = whole && y[c] == y[c];
+            bool again = __ballot(!whole) != 0;
+            if (again) {
+                if (!looked) nan_row = row_has_nan(xr, K, g, li);
+                looked = true;
+                again = __ballot(!whole && !nan_row) != 0;
             }
+            if (again) {
+                int64_t wr = n0 + (SWIGLU ? 16 * (wn * T + t) + (li & 15) : 32 * (wn * T + t) + li);
+                wr = (wr < p.N ? wr : p.N - 1) + (SWIGLU && li >= 16 ? p.N : 0);
+                f32x16& plain = low[i][t];
+                plain = plain_tile<GS>(xr, w + wr * p.K, K, g, scale + (GS > 0 ? (32 * wm + li) * groups : 0), p.norm_w);
+#pragma unroll
+                for (int c = 0; c < 16; ++c) y[c] = y[c] == y[c] ? y[c] : plain[c];
+            }
+            if (row >= p.rows) continue;
             if (p.bias != nullptr) {
 #pragma unroll
                 for (int c = 0; c < 16; ++c) y[c] += p.bias[in_range(c) ? w_row(c) : 0];

@@ -95,3 +95,75 @@ def test_split_linear_special_values(dev):
     plain = [i for i in range(2000) if i not in (3, 64, 70, 200, 300)]
     cols = [j for j in range(300) if j != 7]
     _assert_bound(y[plain][:, cols], x[plain], w[cols], 16)
+
+
+# One shape for each form: two waves a tile, 64 x 64 blocks with a ragged step, 128 x 128 blocks.
+FORMS = [(2000, 256, 300), (4000, 260, 350), (16371, 260, 255)]
+
+
+@pytest.mark.parametrize("M,K,N", FORMS)
+def test_split_linear_infinities_in_every_form(dev, M, K, N):
+    """Results that the planes cannot form (infinite operands, operands that round to bf16 infinity) are formed again;
+    the other results of their tiles, and rows with a NaN, stay as they are."""
+    from montlok import _C
+
+    x, w, b, _ = _operands(dev, M, K, N, M)
+    clean = _C.linear(x, w, b)
+    last = M - 1
+    x[3, 5], x[40, 7], x[64, K - 1], x[70], x[last, 0] = float("inf"), float("nan"), float("-inf"), 3.4e38 / K ** 0.5, 3.4e38
+    w[11], w[N - 2] = 0.0, 0.0
+    w[11, 0], w[N - 2, 0] = 0.5, -0.25
+    y, ref = _C.linear(x, w, b), (x.double() @ w.double().t() + b.double()).float()
+    assert torch.equal(torch.isnan(y), torch.isnan(ref))
+    assert torch.equal(y[torch.isinf(ref)], ref[torch.isinf(ref)])
+    assert torch.isnan(y[40]).all() and torch.isinf(y[3]).any()
+    assert abs(y[last, 11].item() / 1.7e38 - 1) < 1e-6 and abs(y[last, N - 2].item() / -0.85e38 - 1) < 1e-6
+    rows = [i for i in range(M) if i not in (3, 40, 64, 70, last)]
+    cols = [j for j in range(N) if j not in (11, N - 2)]
+    assert torch.equal(y[rows][:, cols], clean[rows][:, cols])
+
+
+def test_norm_split_linear_infinities(dev):
+    """The norm's prologue in front of results that are formed again: as the two operators."""
+    from montlok import _C
+
+    x, w, b, _ = _operands(dev, 3300, 256, 300, 5)
+    nw = torch.rand(256, generator=torch.Generator().manual_seed(2)).to(dev) + 0.5
+    w[5, 100], w[6, 30] = float("inf"), 3.4e38
+    x[9, 4], x[100, 7] = float("nan"), float("inf")
+    for groups in (4, 32):
+        normed = _C.rms_norm(x, nw, 1e-5, groups)
+        two, ref = _C.linear(normed, w, b), (normed.double() @ w.double().t() + b.double()).float()
+        one = _C.rms_norm_linear(x, nw, 1e-5, groups, w, b)
+        assert torch.equal(one[~torch.isnan(two)], two[~torch.isnan(two)]) and torch.equal(torch.isnan(one), torch.isnan(two))
+        assert torch.equal(torch.isfinite(two), torch.isfinite(ref)) and torch.isfinite(two[:, 6]).sum() > 2000
+
+
+def _us(fn, calls=20):
+    fn()
+    times = []
+    for _ in range(5):
+        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        a.record()
+        for _ in range(calls):
+            fn()
+        b.record()
+        b.synchronize()
+        times.append(a.elapsed_time(b) * 1e3 / calls)
+    return min(times)
+
+
+@pytest.mark.parametrize("M,K,N", [(7680, 512, 256), (15360, 512, 256), (3840, 1024, 256), (15360, 256, 1192)])
+@pytest.mark.parametrize("value", ["nan", "inf"])
+def test_rows_of_missing_values_do_not_slow_the_call(dev, M, K, N, value):
+    """One row with a NaN or an infinity, and all of them, in the time of a few calls (formed one sum after another in
+    a lane they took 7 to 120 times a call's; 1.0 to 2.0 measured for NaN, up to 3.3 for infinities)."""
+    from montlok import _C
+
+    x, w, _, _ = _operands(dev, M, K, N, 1)
+    plain = _us(lambda: _C.linear(x, w))
+    x[M // 2, 3] = float(value)
+    one = _us(lambda: _C.linear(x, w))
+    x[:, 3] = float(value)
+    every = _us(lambda: _C.linear(x, w))
+    assert one < 5 * plain and every < 8 * plain, (plain, one, every)
