@@ -1,19 +1,23 @@
 // Dense linear y = x W^T (+ bias, + residual) with fp32 weights on the bf16
 // matrix cores, to fp32 accuracy.
 //
-// An fp32 value is the exact sum of three bf16 values (8 + 8 + 8 bits of its
-// 24-bit significand; each part is the rounding of what the ones before it
-// left, so their magnitudes fall by 2^-9 a step), so
+// An fp32 value times 2^24 is the exact sum of three bf16 values (8 + 8 + 8 bits
+// of its 24-bit significand; each part is the rounding of what the ones before
+// it left, so their magnitudes fall by 2^-9 a step; the factor keeps the third
+// part of the smallest subnormal, 2^-149, a normal bf16 value), so with x and w
+// so enlarged
 //
 //   x w = x1 w1 + (x1 w2 + x2 w1) + (x1 w3 + x2 w2 + x3 w1) + O(2^-26 x w)
 //
 // and six v_mfma_f32_32x32x16_bf16 form, with every product exact and fp32
-// accumulation, what the fp32 form needs sixteen v_mfma_f32_32x32x2_f32 for,
-// at a sixth of the matrix-core time (2.2 PFLOP/s bf16 and 155 TFLOP/s fp32
+// accumulation, what the fp32 form needs eight v_mfma_f32_32x32x2_f32 for,
+// at 0.4 of the matrix-core time (2.2 PFLOP/s bf16 and 155 TFLOP/s fp32
 // measured on this chip). The first term and the other five are summed apart
-// and added at the end: the large sum then takes one rounding per 16 k, and
-// the error against float64 is 8.5e-8 (2-norm, N(0, 1) x, K = 256; 1.2e-7 at
-// K = 512) where the fp32 forms it replaces have 2.9e-7 (4.1e-7).
+// and added at the end, then returned to scale by 2^-48: the large sum then
+// takes one rounding per 16 k, and the error against float64 is 8.5e-8 (2-norm,
+// N(0, 1) x, K = 256; 1.2e-7 at K = 512) where the fp32 forms it replaces have
+// 2.9e-7 (4.1e-7). Operands of 2^104 and more and results of 2^80 and more do
+// not fit the enlarged form; they go the way of infinities, below.
 //
 //   block  = 64 rows x 64 columns of y, 4 waves of 32 x 32; K in steps of 32.
 //            Large calls: 128 x 128, 4 waves of 64 x 64 that multiply and 4 that
@@ -27,23 +31,23 @@
 //
 // What bounds it: the bf16 products. On random data this card's clocks hold a
 // large bf16 matrix product at 1.1 PFLOP/s, 183 TFLOP/s of these sums, and
-// 65536 x 512 -> 256 takes 95 us in the big blocks (180 TFLOP/s). The small
-// blocks keep the matrix cores 43% busy (27 KiB of LDS, 68 registers, five
+// 65536 x 512 -> 256 takes 101 us in the big blocks (170 TFLOP/s). The small
+// blocks keep the matrix cores 43% busy (27 KiB of LDS, 84 registers, five
 // blocks a CU in different phases: a step and SIMD takes 220 cycles of
-// products and about 200 of splitting); a second LDS buffer there, or deeper
+// products and about as many of splitting); a second LDS buffer there, or deeper
 // prefetch in either, was slower. Against the fp32 forms: 7680 x 256 -> 1192
-// 69 -> 35 us, 7680 x 512 -> 256 34 -> 18, 15360 x 256 -> 1192 112 -> 66,
-// 15360 x 512 -> 256 52 -> 26.
+// 69 -> 39 us, 7680 x 512 -> 256 33 -> 18, 15360 x 256 -> 1192 112 -> 68,
+// 15360 x 512 -> 256 51 -> 26.5 (the enlargement's multiply: 0 to 3% of these).
 //
-// Parts of an infinity or of a value that rounds to bf16 infinity are
-// inf and -inf (or NaN), so a result that involves one is NaN. A wave with a
-// NaN among its results that no NaN of the x row explains forms its tile again
-// on the fp32 matrix cores (plain_tile) and takes the NaN ones from there:
-// infinite or NaN where the fp32 products are. Rows with a NaN are ordinary
-// input (bars that are missing), so looking for it has to be cheap, and a
-// serial sum of a lane's 16 results is not: 7680 x 512 -> 256 with one such
-// row 513 us so, 28 with the look and 37 with the tile (22 without the row);
-// all rows 1900 and 31.
+// A sum past that range, or with an infinite operand, is infinite or NaN here
+// (the parts of an infinity are inf and NaN). A wave that holds such a result
+// and no NaN in the x row that explains it forms its tile again on the fp32
+// matrix cores (plain_tile) and takes those results from there: the fp32 form's
+// values, infinite or NaN where its are. Rows with a NaN are ordinary input
+// (bars that are missing), so looking for it has to be cheap, and a serial sum
+// of a lane's 16 results is not: 7680 x 512 -> 256 with one such row 513 us so,
+// 28 with the look and 37 with the tile (22 without the row); all rows 1900
+// and 31.
 
 #include "linear_args.h"
 #include "mlk_common.h"
@@ -58,6 +62,7 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 constexpr int kPlanes = 3, kStep = 32, kBlock = 64;
+constexpr float kUp = 0x1p24f, kDown = 0x1p-48f;  // x and W are split 2^24 times as large, the sums returned from 2^48
 constexpr int kMaxNormGroups = 32;  // RMSNorm groups of a row (K = 256 in groups of 8)
 
 // 16-byte units of the LDS image of a 32-row x 32-k tile: [k half][plane][lane group][32 rows]. The groups are
@@ -162,7 +167,7 @@ __device__ __forceinline__ bool row_has_nan(const float* x, int K, int g, int li
 // PAIR (T = 1, few blocks): eight waves to the 64 x 64 block, two to a tile, one for each k half of a step; their
 // sums meet in LDS.
 template <bool FULL, int GS, bool SWIGLU, int T, bool PAIR>
-__global__ __launch_bounds__(T == 1 && !PAIR ? 256 : 512, T == 1 ? 1 : 2) void linear_split_kernel(LinearArgs p, unsigned n_blocks) {
+__global__ __launch_bounds__(T == 1 && !PAIR ? 256 : 512, T == 2 ? 2 : 1) void linear_split_kernel(LinearArgs p, unsigned n_blocks) {
     static_assert(T == 1 || (GS == 0 && !PAIR), "the norm's prologue and the pairs are the 64 x 64 block's");
     constexpr int MS = PAIR ? 1 : 2;  // 8-row loads a staging wave issues per 64 rows
     constexpr int kRows = kBlock * T, kCols = SWIGLU ? kRows / 2 : kRows;  // rows, output columns of the block
@@ -239,7 +244,7 @@ __global__ __launch_bounds__(T == 1 && !PAIR ? 256 : 512, T == 1 ? 1 : 2) void l
                         f.w = static_cast<float>((static_cast<double>(f.w) * s) * static_cast<double>(nw.w));
                     }
                     if (!FULL && !live) f = float4{0.0f, 0.0f, 0.0f, 0.0f};
-                    f32x2 lo = {f.x, f.y}, hi = {f.z, f.w};
+                    f32x2 lo = {f.x * kUp, f.y * kUp}, hi = {f.z * kUp, f.w * kUp};
                     const unsigned slot = unit(2 * (o * T + i) + (wave >> 1), sc >> 2, 0, (sc >> 1) & 1) + 16 * (wave & 1) + r8;
 #pragma unroll
                     for (int q = 0; q < kPlanes; ++q) dst[2 * (slot + q * 2 * kGroupUnits) + (sc & 1)] = uint2{take_bf16(lo), take_bf16(hi)};
@@ -288,7 +293,13 @@ __global__ __launch_bounds__(T == 1 && !PAIR ? 256 : 512, T == 1 ? 1 : 2) void l
             norm_scales<(GS > 0 ? GS : 8)>(p, row0, groups, scale);
             __syncthreads();
         }
-        for (int k0 = 0; k0 < K; k0 += kStep) {
+        if constexpr (FULL) {  // (apart: left in the loop, the compiler keeps a second set of sums, four blocks a CU)
+            stage(0, 0);
+            __syncthreads();
+            fetch(kStep);
+            multiply(0);
+        }
+        for (int k0 = FULL ? kStep : 0; k0 < K; k0 += kStep) {
             if (k0 > 0) __syncthreads();
             stage(k0, 0);
             __syncthreads();
@@ -341,7 +352,7 @@ __global__ __launch_bounds__(T == 1 && !PAIR ? 256 : 512, T == 1 ? 1 : 2) void l
         for (int t = 0; t < T; ++t) {
             f32x16& y = acc[i][t];
 #pragma unroll
-            for (int c = 0; c < 16; ++c) y[c] += low[i][t][c];
+            for (int c = 0; c < 16; ++c) y[c] = (y[c] + low[i][t][c]) * kDown;
             // W row of accumulator element c (0 .. 15), and its column of out.
             auto w_row = [&](int c) -> int64_t {
                 const int r = 8 * (c >> 2) + 4 * g + (c & 3);
@@ -354,7 +365,7 @@ __global__ __launch_bounds__(T == 1 && !PAIR ? 256 : 512, T == 1 ? 1 : 2) void l
             };
             bool whole = true;
 #pragma unroll
-            for (int c = 0; c < 16; ++c) whole = whole && y[c] == y[c];
+            for (int c = 0; c < 16; ++c) whole = whole && fabsf(y[c]) < INFINITY;
             bool again = __ballot(!whole) != 0;
             if (again) {
                 if (!looked) nan_row = row_has_nan(xr, K, g, li);
@@ -367,7 +378,7 @@ __global__ __launch_bounds__(T == 1 && !PAIR ? 256 : 512, T == 1 ? 1 : 2) void l
                 f32x16& plain = low[i][t];
                 plain = plain_tile<GS>(xr, w + wr * p.K, K, g, scale + (GS > 0 ? (32 * wm + li) * groups : 0), p.norm_w);
 #pragma unroll
-                for (int c = 0; c < 16; ++c) y[c] = y[c] == y[c] ? y[c] : plain[c];
+                for (int c = 0; c < 16; ++c) y[c] = fabsf(y[c]) < INFINITY ? y[c] : plain[c];
             }
             if (row >= p.rows) continue;
             if (p.bias != nullptr) {
