@@ -533,20 +533,24 @@ Tensor attention(const OptTensor& q_, const OptTensor& k_, const OptTensor& v_, 
 PYBIND11_MODULE(_torch_ops, m) {
     m.def("bind", &bind);
     m.def("current_stream", [] { return reinterpret_cast<uintptr_t>(stream()); });
-    m.def("rms_norm", &rms_norm);
-    m.def("add_rms_norm", &add_rms_norm);
-    m.def("layer_norm", &layer_norm);
-    m.def("swiglu", &swiglu);
-    m.def("linear", &linear);
-    m.def("linear_residual", &linear_residual);
-    m.def("rms_norm_linear", &rms_norm_linear);
-    m.def("linear_swiglu", &linear_swiglu);
-    m.def("mhc_prepare", &mhc_prepare);
-    m.def("mhc_combine", &mhc_combine);
-    m.def("mhc_combine_prepare", &mhc_combine_prepare);
-    m.def("mamba3_siso_forward", &mamba3_siso_forward);
-    m.def("mamba3_siso_step", &mamba3_siso_step);
-    m.def("rms_norm_mamba3_forward", &rms_norm_mamba3_forward);
-    m.def("mla_rope_qk", &mla_rope_qk);
-    m.def("attention", &attention);
+    // The operators run without the interpreter's lock: the allocator and a full queue can make a call wait, and
+    // other threads have streams of their own to serve.
+#define OPERATOR(name) m.def(#name, &name, py::call_guard<py::gil_scoped_release>())
+    OPERATOR(rms_norm);
+    OPERATOR(add_rms_norm);
+    OPERATOR(layer_norm);
+    OPERATOR(swiglu);
+    OPERATOR(linear);
+    OPERATOR(linear_residual);
+    OPERATOR(rms_norm_linear);
+    OPERATOR(linear_swiglu);
+    OPERATOR(mhc_prepare);
+    OPERATOR(mhc_combine);
+    OPERATOR(mhc_combine_prepare);
+    OPERATOR(mamba3_siso_forward);
+    OPERATOR(mamba3_siso_step);
+    OPERATOR(rms_norm_mamba3_forward);
+    OPERATOR(mla_rope_qk);
+    OPERATOR(attention);
+#undef OPERATOR
 }

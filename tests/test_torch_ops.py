@@ -2,6 +2,9 @@
 
 from __future__ import annotations
 
+import sys
+import threading
+
 import pytest
 import torch
 
@@ -35,3 +38,59 @@ def test_missing_library_is_refused(tmp_path):
 
     with pytest.raises(RuntimeError):
         _C._ops().bind(str(tmp_path / "absent.so"))
+
+
+_N = (None,)
+_OPERATORS = [
+    lambda c, x: c.rms_norm(x, x, 1e-5, 1),
+    lambda c, x: c.add_rms_norm(x, x, x, 1e-5, 1),
+    lambda c, x: c.layer_norm(x, x, None, 1e-5),
+    lambda c, x: c.swiglu(x),
+    lambda c, x: c.linear(x, x),
+    lambda c, x: c.linear_residual(x, x, None, x),
+    lambda c, x: c.rms_norm_linear(x, x, 1e-5, 1, x),
+    lambda c, x: c.swiglu_mlp(x, x, None, x),
+    lambda c, x: c.mhc_prepare(x, x, 1e-5, *_N * 7, 20),
+    lambda c, x: c.mhc_combine(x, x, x, x),
+    lambda c, x: c.mhc_combine_collapse(x, x, x, x),
+    lambda c, x: c.mhc_combine_prepare(x, x, x, x, x, 1e-5, *_N * 7, 20),
+    lambda c, x: c.mamba3_siso_forward(x, None, *_N * 6, 16, 1, 2, 32, 4, 1e-5, 1e-5, 1e-4),
+    lambda c, x: c.mamba3_siso_step(x, dict(ssm=x, k=x, v=x, angle=x), *_N * 6, 16, 1, 2, 32, 4, 1e-5, 1e-5, 1e-4),
+    lambda c, x: c.rms_norm_mamba3_forward(x, x, 1e-5, 1, x, *_N * 6, 16, 1, 2, 32, 4, 1e-5, 1e-5, 1e-4),
+    lambda c, x: c.mla_rope_qk(x, x, x, x, x, 2),
+    lambda c, x: c.attention(x, x, x, 0, 1.0),
+]
+
+
+@pytest.mark.parametrize("call", _OPERATORS)
+def test_operators_let_other_threads_run(call):
+    """The checks, the allocation and the launch run without the interpreter's lock. With the switch interval out of
+    reach, a thread that waits for the lock gets it only where a call gives it up."""
+    from montlok import _C
+
+    _C._ops()
+    x, ran, gate = torch.ones(4, 4), threading.Event(), threading.Lock()
+
+    def other():
+        with gate:
+            ran.set()
+
+    before = sys.getswitchinterval()
+    sys.setswitchinterval(1000.0)
+    try:
+        gate.acquire()
+        thread = threading.Thread(target=other, daemon=True)
+        thread.start()
+        gate.release()
+        for _ in range(20000):
+            try:
+                call(_C, x)
+            except RuntimeError:
+                pass
+            if ran.is_set():
+                break
+        passed = ran.is_set()
+    finally:
+        sys.setswitchinterval(before)
+    thread.join(10.0)
+    assert passed
