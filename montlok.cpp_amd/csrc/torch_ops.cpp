@@ -22,6 +22,46 @@
 #include "../../include/mlk_hip.h"
 
 namespace {
+// Arguments taken as Python's int() and float() take them: a count may be any whole number (4.0, a numpy or torch
+// scalar), a real anything with a value (the text "1e-5", as YAML reads it, among them).
+struct Count {
+    int64_t value = 0;
+    operator int64_t() const { return value; }
+};
+struct Real {
+    double value = 0.0;
+    operator double() const { return value; }
+};
+bool no_error() {
+    const bool failed = PyErr_Occurred() != nullptr;
+    if (failed) PyErr_Clear();
+    return !failed;
+}
+}  // namespace
+
+namespace pybind11::detail {
+template <>
+struct type_caster<Count> {
+    PYBIND11_TYPE_CASTER(Count, const_name("int"));
+    bool load(handle source, bool) {
+        const object whole = reinterpret_steal<object>(PyNumber_Long(source.ptr()));
+        const bool same = whole && PyObject_RichCompareBool(source.ptr(), whole.ptr(), Py_EQ) == 1;
+        if (same) value.value = PyLong_AsLongLong(whole.ptr());
+        return no_error() && same;
+    }
+};
+template <>
+struct type_caster<Real> {
+    PYBIND11_TYPE_CASTER(Real, const_name("float"));
+    bool load(handle source, bool) {
+        const object number = reinterpret_steal<object>(PyNumber_Float(source.ptr()));
+        if (number) value.value = PyFloat_AsDouble(number.ptr());
+        return no_error();
+    }
+};
+}  // namespace pybind11::detail
+
+namespace {
 
 using at::Tensor;
 using OptTensor = std::optional<Tensor>;
@@ -118,7 +158,7 @@ std::vector<int64_t> with_last(const Tensor& x, int64_t n) {
 
 // ------------------------------------------------------------------ norms
 
-Tensor rms_norm(const OptTensor& x_, const OptTensor& weight, double eps, int64_t groups) {
+Tensor rms_norm(const OptTensor& x_, const OptTensor& weight, Real eps, Count groups) {
     const Tensor& x = f32_gpu(x_, "x");
     REQUIRE(x.dim() >= 1, "x must have at least one dimension");
     const int64_t dim = x.size(-1);
@@ -130,8 +170,8 @@ Tensor rms_norm(const OptTensor& x_, const OptTensor& weight, double eps, int64_
     return out;
 }
 
-std::tuple<Tensor, Tensor> add_rms_norm(const OptTensor& left, const OptTensor& right, const OptTensor& weight, double eps,
-                                        int64_t groups) {
+std::tuple<Tensor, Tensor> add_rms_norm(const OptTensor& left, const OptTensor& right, const OptTensor& weight, Real eps,
+                                        Count groups) {
     f32_gpu(left, "left");
     f32_gpu(right, "right");
     REQUIRE(left->sizes() == right->sizes() && left->dim() >= 1, "residual operands must have the same shape");
@@ -144,7 +184,7 @@ std::tuple<Tensor, Tensor> add_rms_norm(const OptTensor& left, const OptTensor& 
     return {residual, normalized};
 }
 
-Tensor layer_norm(const OptTensor& x_, const OptTensor& weight, const OptTensor& bias, double eps) {
+Tensor layer_norm(const OptTensor& x_, const OptTensor& weight, const OptTensor& bias, Real eps) {
     const Tensor& x = f32_gpu(x_, "x");
     REQUIRE(x.dim() >= 1, "x must have at least one dimension");
     const int64_t dim = x.size(-1);
@@ -198,7 +238,7 @@ Tensor linear_residual(const OptTensor& input, const OptTensor& weight, const Op
 }
 
 // None where the shape has no fused form.
-OptTensor rms_norm_linear(const OptTensor& x_, const OptTensor& norm_weight, double eps, int64_t groups, const OptTensor& weight,
+OptTensor rms_norm_linear(const OptTensor& x_, const OptTensor& norm_weight, Real eps, Count groups, const OptTensor& weight,
                           const OptTensor& bias) {
     const Tensor& x = f32_gpu(x_, "x");
     REQUIRE(x.dim() >= 1, "x must have at least one dimension");
@@ -295,12 +335,12 @@ Prepare prepare_of(int64_t n, int64_t d, const OptTensor& norm_w, const OptTenso
     return p;
 }
 
-std::tuple<Tensor, Tensor, Tensor, Tensor> mhc_prepare(const OptTensor& streams, const OptTensor& norm_w, double eps,
+std::tuple<Tensor, Tensor, Tensor, Tensor> mhc_prepare(const OptTensor& streams, const OptTensor& norm_w, Real eps,
                                                        const OptTensor& proj_w, const OptTensor& pre_bias,
                                                        const OptTensor& post_bias, const OptTensor& res_bias,
                                                        const OptTensor& pre_alpha, const OptTensor& post_alpha,
-                                                       const OptTensor& res_alpha, int64_t iters, int64_t n_streams,
-                                                       const OptTensor& agg_norm_w, double agg_norm_eps) {
+                                                       const OptTensor& res_alpha, Count iters, Count n_streams,
+                                                       const OptTensor& agg_norm_w, Real agg_norm_eps) {
     const Streams v = streams_of(streams, n_streams);
     const Prepare p = prepare_of(v.n, v.d, norm_w, proj_w, pre_bias, post_bias, res_bias, pre_alpha, post_alpha, res_alpha, iters, agg_norm_w);
     const Tensor agg = empty({v.B, v.L, v.d}, *streams), pre = empty({v.B, v.L, v.n}, *streams);
@@ -332,10 +372,10 @@ Tensor mhc_combine(const OptTensor& streams, const OptTensor& res, const OptTens
 }
 
 std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor> mhc_combine_prepare(
-    const OptTensor& streams, const OptTensor& res, const OptTensor& post, const OptTensor& out, const OptTensor& norm_w, double eps,
+    const OptTensor& streams, const OptTensor& res, const OptTensor& post, const OptTensor& out, const OptTensor& norm_w, Real eps,
     const OptTensor& proj_w, const OptTensor& pre_bias, const OptTensor& post_bias, const OptTensor& res_bias,
-    const OptTensor& pre_alpha, const OptTensor& post_alpha, const OptTensor& res_alpha, int64_t iters, const OptTensor& agg_norm_w,
-    double agg_norm_eps, bool reuse_streams, const std::optional<std::tuple<Tensor, Tensor, Tensor, Tensor>>& into) {
+    const OptTensor& pre_alpha, const OptTensor& post_alpha, const OptTensor& res_alpha, Count iters, const OptTensor& agg_norm_w,
+    Real agg_norm_eps, bool reuse_streams, const std::optional<std::tuple<Tensor, Tensor, Tensor, Tensor>>& into) {
     const Streams v = combine_inputs(streams, res, post, out);
     const Prepare p = prepare_of(v.n, v.d, norm_w, proj_w, pre_bias, post_bias, res_bias, pre_alpha, post_alpha, res_alpha, iters, agg_norm_w);
     Tensor fresh, agg, pre_o, post_o, res_o;
@@ -389,8 +429,8 @@ void inner_dense(const Tensor& t, const char* name) {
 
 Tensor mamba3_siso_forward(const OptTensor& projected_, const OptTensor& gate, const OptTensor& b_bias, const OptTensor& c_bias,
                            const OptTensor& b_norm_w, const OptTensor& c_norm_w, const OptTensor& dt_bias, const OptTensor& skip,
-                           int64_t d_state, int64_t ngroups, int64_t nheads, int64_t headdim, int64_t angles, double b_eps,
-                           double c_eps, double a_floor) {
+                           int64_t d_state, int64_t ngroups, int64_t nheads, int64_t headdim, int64_t angles, Real b_eps,
+                           Real c_eps, Real a_floor) {
     const Tensor& projected = f32_gpu(projected_, "projected");
     const bool logits = !gate.has_value() || gate->numel() == 0;
     if (!logits) f32_gpu(gate, "gate");
@@ -421,8 +461,8 @@ Tensor mamba3_siso_forward(const OptTensor& projected_, const OptTensor& gate, c
 Tensor mamba3_siso_step(const OptTensor& projected_, const OptTensor& ssm, const OptTensor& k, const OptTensor& v,
                         const OptTensor& angle, bool started, const OptTensor& b_bias, const OptTensor& c_bias,
                         const OptTensor& b_norm_w, const OptTensor& c_norm_w, const OptTensor& dt_bias, const OptTensor& skip,
-                        int64_t d_state, int64_t ngroups, int64_t nheads, int64_t headdim, int64_t angles, double b_eps,
-                        double c_eps, double a_floor) {
+                        int64_t d_state, int64_t ngroups, int64_t nheads, int64_t headdim, int64_t angles, Real b_eps,
+                        Real c_eps, Real a_floor) {
     const Tensor& projected = f32_gpu(projected_, "projected");
     REQUIRE(projected.dim() == 2, "projected must be [S,W]");
     inner_dense(projected, "projected");
@@ -450,11 +490,11 @@ Tensor mamba3_siso_step(const OptTensor& projected_, const OptTensor& ssm, const
 }
 
 // None where the geometry has no one-launch kernel.
-OptTensor rms_norm_mamba3_forward(const OptTensor& inputs, const OptTensor& norm_weight, double norm_eps, int64_t norm_groups,
+OptTensor rms_norm_mamba3_forward(const OptTensor& inputs, const OptTensor& norm_weight, Real norm_eps, Count norm_groups,
                                   const OptTensor& in_weight, const OptTensor& b_bias, const OptTensor& c_bias,
                                   const OptTensor& b_norm_w, const OptTensor& c_norm_w, const OptTensor& dt_bias,
                                   const OptTensor& skip, int64_t d_state, int64_t ngroups, int64_t nheads, int64_t headdim,
-                                  int64_t angles, double b_eps, double c_eps, double a_floor) {
+                                  int64_t angles, Real b_eps, Real c_eps, Real a_floor) {
     const Tensor& x = f32_gpu(inputs, "inputs");
     REQUIRE(x.dim() == 3, "inputs must be [B,L,d_model]");
     const int64_t B = x.size(0), L = x.size(1), dm = x.size(2);
@@ -512,7 +552,7 @@ std::pair<int64_t, int64_t> token_strides(const Tensor& t, const char* name) {
     return {ts, H > 1 ? t.stride(2) : hd};
 }
 
-Tensor attention(const OptTensor& q_, const OptTensor& k_, const OptTensor& v_, int64_t mask, double scale, bool bf16) {
+Tensor attention(const OptTensor& q_, const OptTensor& k_, const OptTensor& v_, Count mask, Real scale, bool bf16) {
     const Tensor& q = f32_gpu(q_, "q");
     REQUIRE(q.dim() == 4, "q must be [B,L,H,head_dim]");
     const Tensor& k = f32_gpu(k_, "k");

@@ -5,6 +5,7 @@ from __future__ import annotations
 import sys
 import threading
 
+import numpy as np
 import pytest
 import torch
 
@@ -38,6 +39,34 @@ def test_missing_library_is_refused(tmp_path):
 
     with pytest.raises(RuntimeError):
         _C._ops().bind(str(tmp_path / "absent.so"))
+
+
+@pytest.mark.parametrize("one", [1, 1.0, torch.tensor(1), np.float32(1), np.int64(1)])
+@pytest.mark.parametrize("eps", [1e-5, "1e-5", torch.tensor(1e-5), np.float32(1e-5)])
+def test_numbers_as_int_and_float_take_them(one, eps):
+    """Whole numbers of any type for groups, iterations, streams and mask; anything float() takes for eps and scale."""
+    from montlok import _C
+
+    x, n = torch.ones(4, 4), (None,)
+    for call in (lambda: _C.rms_norm(x, x, eps, one), lambda: _C.add_rms_norm(x, x, x, eps, one),
+                 lambda: _C.rms_norm_linear(x, x, eps, one, x), lambda: _C.layer_norm(x, x, None, eps),
+                 lambda: _C.mhc_prepare(x, x, eps, *n * 7, one, one, None, eps),
+                 lambda: _C.mhc_combine_prepare(x, x, x, x, x, eps, *n * 7, one, None, eps),
+                 lambda: _C.mamba3_siso_forward(x, None, *n * 6, 16, 1, 2, 32, 4, eps, eps, eps),
+                 lambda: _C.rms_norm_mamba3_forward(x, x, eps, one, x, *n * 6, 16, 1, 2, 32, 4, eps, eps, eps),
+                 lambda: _C.attention(x, x, x, one, eps)):
+        with pytest.raises(RuntimeError, match="must be on the GPU"):
+            call()
+
+
+@pytest.mark.parametrize("groups,eps", [(1.5, 1e-5), ("1", 1e-5), (None, 1e-5), (2.0 ** 70, 1e-5), (float("nan"), 1e-5),
+                                        (1, None), (1, "small"), (1, 1j)])
+def test_what_is_no_number_is_refused(groups, eps):
+    from montlok import _C
+
+    x = torch.ones(4, 4)
+    with pytest.raises(TypeError):
+        _C.rms_norm(x, x, eps, groups)
 
 
 _N = (None,)
