@@ -317,8 +317,9 @@ mlk_status mlk_mhc_combine_prepare(const float* streams, int64_t tokens, int64_t
 /* Bytes of device workspace for mamba3_siso_forward: q, k [B,L,H,N], (alpha,
  * beta, gamma) [3,B,L,H] and the rotary angle terms [B,L,H,max(R,1)] (the slab
  * of montlok.cpp:396-420), or, for few (window, head) pairs over several
- * 32-token chunks, the chunks' items of the chunk-parallel scan. A call with
- * the slab alone is accepted and takes another form of the scan there. */
+ * 32-token chunks with d_state 16, 32 or 64, the chunks' items of the
+ * chunk-parallel scan where those are at most 4 GiB more. A call with the slab
+ * alone is accepted and takes another form of the scan there. */
 size_t mlk_mamba3_workspace_bytes(int64_t batch, int64_t length, int64_t nheads, int64_t d_state,
                                   int64_t num_rope_angles);
 

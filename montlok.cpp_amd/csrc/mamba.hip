@@ -1735,6 +1735,31 @@ __device__ __forceinline__ void split_item(const SplitScanArgs& p, int64_t& b, i
     b = lin / chunks / H;
 }
 
+// Beyond this many chunks the sums of the chunks before each one are formed in a launch of their own: added by every
+// chunk's block they grow with the square of the window (64 pairs x 32000 tokens at d_state 16, headdim 32: 2.03 ms, 1.25 so;
+// at 64 chunks they cost what the launch does, 2 to 6 us).
+constexpr int kPrefixChunks = 64;
+
+// Each chunk's angle sum becomes the sum of the chunks before it, added in split_chunk_kernel's order. One thread per
+// (window, head, angle); a chain of fp64 additions, so the loads run ahead of it.
+__global__ __launch_bounds__(64) void split_prefix_kernel(double* csum, int64_t rows, int64_t chunks, int R) {
+    const int64_t row = static_cast<int64_t>(blockIdx.x) * 64 + threadIdx.x;
+    if (row >= rows) return;
+    double* p = csum + row / R * chunks * R + row % R;
+    double running = 0.0;
+    constexpr int kAhead = 16;
+    for (int64_t i = 0; i < chunks; i += kAhead) {
+        double v[kAhead];
+#pragma unroll
+        for (int j = 0; j < kAhead; ++j) v[j] = p[(i + j < chunks ? i + j : chunks - 1) * R];
+#pragma unroll
+        for (int j = 0; j < kAhead; ++j) {
+            if (i + j < chunks) p[(i + j) * R] = running;
+            running += v[j];
+        }
+    }
+}
+
 template <int NT>
 __global__ __launch_bounds__(256) void split_chunk_kernel(SplitScanArgs p) {
     constexpr int C = 32, CT = 2, N = 16 * NT, NTH = 256, NP = N + 4, WP = C + 4, RM = N / 2;
@@ -1792,8 +1817,12 @@ __global__ __launch_bounds__(256) void split_chunk_kernel(SplitScanArgs p) {
         const int r = tid - 128;
         const double* csum = reinterpret_cast<const double*>(p.ws + p.s.csum) + bh * p.s.chunks * R + r;
         double running = 0.0;
+        if (p.s.chunks > kPrefixChunks) {
+            running = csum[static_cast<int64_t>(c) * R];  // split_prefix_kernel's
+        } else {
 #pragma unroll 4
-        for (int i = 0; i < c; ++i) running += csum[i * R];
+            for (int i = 0; i < c; ++i) running += csum[i * R];
+        }
 #pragma unroll
         for (int t0 = 0; t0 < C; t0 += 16) {
             float term[16];
@@ -2057,19 +2086,29 @@ __global__ __launch_bounds__(64 * DT) void split_out_kernel(SplitScanArgs p) {
     }
 }
 
+// What the unfused kernels need; a call with only this much takes the fused scan.
+size_t scan_workspace_bytes(int64_t B, int64_t L, int64_t H, int64_t N, int64_t R) {
+    const int64_t blh = B * L * H;
+    return sizeof(float) * static_cast<size_t>(2 * blh * N + 3 * blh + blh * (R > 0 ? R : 1));
+}
+
 // Whether the chunk-parallel form takes the call. With at most 128 pairs (half of the CUs one block each) it wins
 // from four chunks on; at three the launches it adds eat the gain (8 pairs x 96 tokens: 20 against 26 us on the
 // device, and 4 us more on the host). Up to 192 pairs (the fused blocks then have a CU each, and the workspace's
 // traffic, 73 KB an item at d_state and headdim 64, counts) it wins over many chunks only: 192 pairs x 480 tokens
 // 95 against 124 us, 192 x 96 30 against 27; with 256 pairs x 480 the two are even (131 and 126 us in the model).
-bool split_scan_shape(int64_t B, int64_t L, int64_t H) {
+// Smaller d_state and headdim gain as much or more (16 and 32: 128 pairs x 100 tokens 19 against 22, 192 x 384 39
+// against 60). Its workspace is about twice the unfused kernels', so it stops where that would be 4 GiB more.
+bool split_scan_shape(int64_t B, int64_t L, int64_t H, int64_t N, int64_t R) {
     const int64_t pairs = B * H, chunks = (L + 31) / 32;
-    return (pairs <= 128 && chunks >= 4) || (pairs <= 192 && chunks >= 12);
+    if (!((pairs <= 128 && chunks >= 4) || (pairs <= 192 && chunks >= 12)) || (N != 16 && N != 32 && N != 64)) return false;
+    const size_t bytes = sizeof(float) * static_cast<size_t>(split_layout(B, L, H, N, 64, R).total);  // (headdim at most 64)
+    return bytes <= scan_workspace_bytes(B, L, H, N, R) + (size_t{4} << 30);
 }
 
 bool launch_scan_split(const ScanArgs& s, int64_t N, int64_t D, void* workspace, size_t bytes, hipStream_t stream) {
     const SplitScan layout = split_layout(s.B, s.L, s.H, N, D, s.R);
-    if (!split_scan_shape(s.B, s.L, s.H) || bytes < sizeof(float) * static_cast<size_t>(layout.total) || !aligned16(workspace))
+    if (!split_scan_shape(s.B, s.L, s.H, N, s.R) || bytes < sizeof(float) * static_cast<size_t>(layout.total) || !aligned16(workspace))
         return false;
     SplitScanArgs p{s, static_cast<float*>(workspace), layout, N, D};
     p.a.chunks = layout.chunks;
@@ -2078,12 +2117,16 @@ bool launch_scan_split(const ScanArgs& s, int64_t N, int64_t D, void* workspace,
     const unsigned pairs = static_cast<unsigned>(s.B * s.H), items = pairs * static_cast<unsigned>(layout.chunks);
     const size_t token_lds = scan_token_lds(s.H, s.R);
     if (token_lds > 64 * 1024) return false;
+    double* csum = reinterpret_cast<double*>(p.ws + layout.csum);
     const int NT = static_cast<int>(N / 16), DT = static_cast<int>(D / 16);
 #define MLK_SPLIT(NTV, DTV)                                                                                                  \
     if (NT == NTV && DT == DTV) {                                                                                            \
         hipLaunchKernelGGL(scan_token_kernel, dim3(static_cast<unsigned>(s.B * layout.chunks)), dim3(256), token_lds, stream, \
                            p.a, N, D, reinterpret_cast<float4*>(p.ws + layout.coef), p.ws + layout.ang,                      \
-                           reinterpret_cast<double*>(p.ws + layout.csum));                                                   \
+                           csum);                                                                                            \
+        if (layout.chunks > kPrefixChunks && s.R > 0)                                                                        \
+            hipLaunchKernelGGL(split_prefix_kernel, dim3(static_cast<unsigned>(ceil_div(pairs * s.R, 64))), dim3(64), 0, stream, \
+                               csum, pairs * s.R, layout.chunks, static_cast<int>(s.R));                                     \
         hipLaunchKernelGGL((split_chunk_kernel<NTV>), dim3(items), dim3(256), 0, stream, p);                                 \
         hipLaunchKernelGGL((split_state_kernel<NTV, DTV>), dim3(pairs), dim3(64 * DTV * (NTV > 1 ? 2 : 1)), 0, stream, p);   \
         hipLaunchKernelGGL((split_out_kernel<NTV, DTV>), dim3(items), dim3(64 * DTV), 0, stream, p);                         \
@@ -2832,18 +2875,11 @@ using namespace mlk;
 
 extern "C" {
 
-// What the unfused kernels need; a call with only this much takes the fused scan.
-static size_t scan_workspace_bytes(int64_t batch, int64_t length, int64_t nheads, int64_t d_state, int64_t num_rope_angles) {
-    const int64_t blh = batch * length * nheads;
-    const int64_t rw = num_rope_angles > 0 ? num_rope_angles : 1;
-    return sizeof(float) * static_cast<size_t>(2 * blh * d_state + 3 * blh + blh * rw);
-}
-
 size_t mlk_mamba3_workspace_bytes(int64_t batch, int64_t length, int64_t nheads, int64_t d_state,
                                   int64_t num_rope_angles) {
     size_t bytes = scan_workspace_bytes(batch, length, nheads, d_state, num_rope_angles);
-    if (batch * length * nheads > 0 && d_state <= 64 && mlk::split_scan_shape(batch, length, nheads)) {  // (headdim at most 64 there)
-        const size_t split = sizeof(float) * static_cast<size_t>(mlk::split_layout(batch, length, nheads, d_state, 64, num_rope_angles).total);
+    if (batch * length * nheads > 0 && split_scan_shape(batch, length, nheads, d_state, num_rope_angles)) {
+        const size_t split = sizeof(float) * static_cast<size_t>(split_layout(batch, length, nheads, d_state, 64, num_rope_angles).total);
         bytes = split > bytes ? split : bytes;
     }
     return bytes;

@@ -65,3 +65,18 @@ def test_invalid_arguments_are_rejected_before_launch(lib):
     assert g(None, 8, 4, 16, 16, 64, None, 1e-5, None, None, None, None, None, None, None, -1, None, 0.0, None, None,
              None, None, None) == 1
     assert b"sinkhorn_iters must be non-negative" in lib.mlk_last_error()
+
+
+@pytest.mark.parametrize("B,L,H,N,R", [(1, 480, 8, 64, 16), (16, 14000, 8, 64, 16), (16, 400000, 8, 64, 16), (1, 20000000, 1, 16, 4),
+                                       (24, 32000, 8, 16, 4), (3, 500, 4, 48, 8), (1, 200000, 1, 24, 3), (40, 480, 8, 64, 16)])
+def test_mamba3_workspace_is_bounded(lib, B, L, H, N, R):
+    """At most 4 GiB above the slab of the unfused kernels, and the slab itself where d_state has no chunk-parallel scan."""
+    f = lib.mlk_mamba3_workspace_bytes
+    f.argtypes, f.restype = [C.c_int64] * 5, C.c_size_t
+    slab = 4 * (2 * B * L * H * N + 3 * B * L * H + B * L * H * max(R, 1))
+    got = f(B, L, H, N, R)
+    assert slab <= got <= slab + 2 ** 32
+    if N not in (16, 32, 64) or B * H > 192:
+        assert got == slab
+    if (B, L) == (1, 480):
+        assert got > slab

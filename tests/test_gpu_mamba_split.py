@@ -63,6 +63,42 @@ def test_chunk_parallel_scan_headdim16(dev, oracle, monkeypatch, B, L, N, G, H, 
     assert_close(got, _C.mamba3_siso_forward(proj, None, *params, *geo), tol=1e-6, name="vs sequential")
 
 
+@pytest.mark.parametrize("B,L,N,G,H,D,R", [(1, 2048, 16, 1, 3, 32, 8), (1, 2049, 16, 1, 3, 32, 8), (2, 2600, 64, 1, 2, 64, 32),
+                                           (3, 2100, 32, 2, 4, 16, 5), (1, 2200, 16, 1, 1, 64, 0)])
+def test_long_windows_equal_unfused(dev, monkeypatch, B, L, N, G, H, D, R):
+    """On both sides of 64 chunks, past which the angle sums before each chunk come from a launch of their own."""
+    from montlok import _C
+
+    proj, params, geo = _case(dev, B, L, N, G, H, D, R)
+    got = _C.mamba3_siso_forward(proj, None, *params, *geo)
+    if D == 16:
+        monkeypatch.setenv("MLK_MAMBA3_SCAN", "sequential")
+        assert_close(got, _C.mamba3_siso_forward(proj, None, *params, *geo), tol=1e-6, name="vs sequential")
+        return
+    monkeypatch.setenv("MLK_MAMBA3_SCAN", "unfused")
+    assert_bitwise(got, _C.mamba3_siso_forward(proj, None, *params, *geo).cpu().numpy(), "chunk-parallel vs unfused")
+
+
+def test_time_grows_with_the_window_not_its_square(dev):
+    """64 pairs at four times the length: 4.1 times the time (5.9 where each chunk adds up all before it)."""
+    from montlok import _C
+
+    us = []
+    _, params, geo = _case(dev, 8, 8, 16, 1, 8, 32, 4)
+    for L in (8000, 32000):
+        proj = torch.randn(8, L, 2 * 8 * 32 + 2 * 16 + 3 * 8 + 4, device=dev)
+        times = []
+        for _ in range(6):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            _C.mamba3_siso_forward(proj, None, *params, *geo)
+            b.record()
+            b.synchronize()
+            times.append(a.elapsed_time(b) * 1e3)
+        us.append(min(times))
+    assert us[1] < 5.0 * us[0], us
+
+
 def test_smaller_workspace_takes_the_fused_scan(dev):
     """A caller that holds only the unfused kernels' slab is served as before, with the same result."""
     from montlok import _C
