@@ -11,6 +11,7 @@ from __future__ import annotations
 import os
 import shutil
 import subprocess
+import sys
 import time
 from pathlib import Path
 
@@ -54,3 +55,45 @@ def test_build_entry_raises_on_make_failure(monkeypatch):
     monkeypatch.setattr(ge.subprocess, "run", fake_run)
     with pytest.raises(RuntimeError, match="failed"):
         ge._make("-C", str(PKG))
+
+
+def _dry_run(*args):
+    return subprocess.run(["make", "-n", "-C", str(PKG), *args], capture_output=True, text=True, timeout=120)
+
+
+def test_the_library_builds_without_torch():
+    """Without torch (here: without a Python at all) make builds the C ABI and says what it left out; with torch, both."""
+    bare = _dry_run("-B", "PYTHON=/nonexistent/python3")
+    assert bare.returncode == 0, bare.stderr
+    assert "libmlk_hip.so" in bare.stdout and "torch_ops.cpp" not in bare.stdout and "is not built" in bare.stdout
+    assert "torch_ops.cpp" not in _dry_run("-B", "lib").stdout
+    full = _dry_run("-B", f"PYTHON={sys.executable}")
+    assert full.returncode == 0 and "torch_ops.cpp" in full.stdout and "compiled_with_cxx11_abi" in full.stdout
+
+
+def test_the_extension_follows_torch(tmp_path):
+    """Built already, it is built again when the torch or the Python it was built against changes, and only then."""
+    pkg = tmp_path / "pkg"
+    (pkg / "_build").mkdir(parents=True)
+    shutil.copy(PKG / "Makefile", pkg / "Makefile")
+    shutil.copytree(PKG / "csrc", pkg / "csrc")
+    shutil.copytree(ROOT / "include", tmp_path / "include")
+    ops = pkg / "montlok" / "rdt" / "lib" / "_torch_ops.so"
+    ops.parent.mkdir(parents=True)
+    env = pkg / "_build" / "torch_ops.env"
+    cxx = tmp_path / "cxx"  # writes its output and compiles nothing
+    cxx.write_text('#!/bin/sh\nwhile [ $# -gt 0 ]; do [ "$1" = -o ] && echo built > "$2"; shift; done\n')
+    cxx.chmod(0o755)
+
+    def make(*args):
+        out = subprocess.run(["make", "-C", str(pkg), f"PYTHON={sys.executable}", f"CXX={cxx}", *args], capture_output=True,
+                             text=True, timeout=300)
+        assert out.returncode == 0, out.stderr
+        return out.stdout
+
+    assert "torch_ops.cpp" in make("ops") and ops.read_text() == "built\n"
+    assert len(env.read_text().split()) == 4
+    assert "torch_ops.cpp" not in make("ops")
+    env.write_text("/another/torch /another/python 2.0 3.9\n")
+    assert "torch_ops.cpp" in make("ops")
+    assert "torch_ops.cpp" not in make("ops")
