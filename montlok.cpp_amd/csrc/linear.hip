@@ -1347,17 +1347,17 @@ void linear_stream_io_kernel(LinearArgs p, int col_groups, int row_parts) {
     }
 }
 
-// Shapes too small to give the 128-row blocks one per CU (256 CUs), with K
-// held in at most eight 32-wide steps.
-// linear_tiles_kernel's BUF form: K a multiple of the 16-byte unit (kper elements), N % 4 = 0, 16-byte
-// aligned output (and residual) rows, the output within 2 GiB.
-bool tiles_buf_fits(const LinearArgs& p, int64_t rows, int kper) {
+// linear_tiles_kernel's BUF form, for VEC: N % 4 = 0, 16-byte aligned output (and residual) rows, the output
+// within 2 GiB.
+bool tiles_buf_fits(const LinearArgs& p, int64_t rows) {
     auto a16 = [](const void* q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; };
-    return p.K % kper == 0 && p.N % 4 == 0 && a16(p.out) && p.out_stride % 4 == 0 &&
+    return p.N % 4 == 0 && a16(p.out) && p.out_stride % 4 == 0 &&
            (p.residual == nullptr || (a16(p.residual) && p.res_stride % 4 == 0)) &&
            (rows + 1) * p.out_stride * 4 < (int64_t{1} << 31);
 }
 
+// Shapes too small to give the 128-row blocks one per CU (256 CUs), with K
+// held in at most eight 32-wide steps.
 bool small_shape(int64_t rows, int64_t K, int64_t N) {
     return K % 8 == 0 && K <= 256 && ceil_div(rows, kRowsPerBlock) * ceil_div(N, kColsPerChunk) < 256 &&
            ceil_div(rows, 16) * ceil_div(N, 16) <= 0x7fffffff;
@@ -1510,25 +1510,29 @@ void launch(const LinearArgs& p, int64_t rows, int64_t n_chunks, hipStream_t str
     // faster there: 7.2 vs 8.6 us at 2048 x 64 -> 304, 71 vs 79 us at
     // 65536 x 128 -> 257); bf16 weights take the tiled kernel (27.6 vs 29.3 us
     // at 32768 x 256 -> 336).
-    if (p.K <= KC && !BF16W) {
-        hipLaunchKernelGGL((linear_kernel<BF16W, VEC, false>), grid, dim3(kThreads), 0, stream, p);
-    } else if (p.K <= KC) {
-        // (KS = 1 keeps four waves per SIMD: the residual's registers would spill, so it takes BUF = 1 only)
-        if (VEC && p.residual == nullptr && tiles_buf_fits(p, rows, 16 / static_cast<int>(sizeof(typename WTraits<BF16W>::T)))) {
+    if (p.K <= KC) {
+        if constexpr (!BF16W) {
+            hipLaunchKernelGGL((linear_kernel<BF16W, VEC, false>), grid, dim3(kThreads), 0, stream, p);
+        } else if (VEC && p.residual == nullptr && tiles_buf_fits(p, rows)) {
+            // (KS = 1 keeps four waves per SIMD: the residual's registers would spill, so it takes BUF = 1 only)
             hipLaunchKernelGGL((linear_tiles_kernel<BF16W, VEC, 1, 1, VEC ? 1 : 0>), grid, dim3(kThreads), 0, stream, p);
         } else {
             hipLaunchKernelGGL((linear_tiles_kernel<BF16W, VEC, 1, 1>), grid, dim3(kThreads), 0, stream, p);
         }
-    } else if (p.K <= 2 * KC) {
-        if (VEC && p.residual == nullptr && tiles_buf_fits(p, rows, 16 / static_cast<int>(sizeof(typename WTraits<BF16W>::T)))) {
-            hipLaunchKernelGGL((linear_tiles_kernel<BF16W, VEC, 1, 2, VEC ? 1 : 0>), grid, dim3(kThreads), 0, stream, p);
-        } else if (VEC && tiles_buf_fits(p, rows, 16 / static_cast<int>(sizeof(typename WTraits<BF16W>::T)))) {
-            hipLaunchKernelGGL((linear_tiles_kernel<BF16W, VEC, 1, 2, VEC ? 2 : 0>), grid, dim3(kThreads), 0, stream, p);
-        } else {
-            hipLaunchKernelGGL((linear_tiles_kernel<BF16W, VEC, 1, 2>), grid, dim3(kThreads), 0, stream, p);
-        }
     } else {
-        hipLaunchKernelGGL((linear_kernel<BF16W, VEC, true>), grid, dim3(kThreads), 0, stream, p);
+        // fp32 weights come here unaligned, or with strides past the three-plane form's 32-bit offsets: one form serves both.
+        constexpr bool vec = BF16W && VEC;
+        if (p.K > 2 * KC) {
+            hipLaunchKernelGGL((linear_kernel<BF16W, vec, true>), grid, dim3(kThreads), 0, stream, p);
+        } else if (vec && tiles_buf_fits(p, rows)) {
+            if (p.residual == nullptr) {
+                hipLaunchKernelGGL((linear_tiles_kernel<BF16W, vec, 1, 2, vec ? 1 : 0>), grid, dim3(kThreads), 0, stream, p);
+            } else {
+                hipLaunchKernelGGL((linear_tiles_kernel<BF16W, vec, 1, 2, vec ? 2 : 0>), grid, dim3(kThreads), 0, stream, p);
+            }
+        } else {
+            hipLaunchKernelGGL((linear_tiles_kernel<BF16W, vec, 1, 2>), grid, dim3(kThreads), 0, stream, p);
+        }
     }
 }
 

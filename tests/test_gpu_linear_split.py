@@ -192,3 +192,16 @@ def test_rows_of_missing_values_do_not_slow_the_call(dev, M, K, N, value):
     x[:, 3] = float(value)
     every = _us(lambda: _C.linear(x, w))
     assert one < 5 * plain and every < 8 * plain, (plain, one, every)
+
+
+@pytest.mark.parametrize("K", [100, 128, 196, 260, 1028])
+def test_rows_too_far_apart_for_the_planes(dev, K):
+    """A row stride of 2^23 floats and more (the last position of very long windows) takes the fp32 forms."""
+    from montlok import _C
+
+    x, w, b, r = _operands(dev, 3, K, 300, K)
+    far = torch.empty(3 * 2 ** 23, device=dev).view(3, 2 ** 23)[:, :K]
+    far.copy_(x)
+    y = _C.linear(far, w)
+    _assert_bound(y, x, w, 2)
+    assert torch.equal(_C.linear(far, w, b), y + b) and torch.equal(_C.linear_residual(far, w, b, r), r + (y + b))
