@@ -41,7 +41,8 @@ def test_split_attention_vs_float64(dev, B, Lq, Lk, H, hd, mask, scale):
 
 
 def test_split_attention_special_values(dev):
-    """A score of +-inf and a NaN key: as softmax has them, in the rows that see the key and in no others."""
+    """A score of -inf (no weight), of +inf (inf - inf: NaN) and a NaN key: as softmax has them, in the rows that see
+    the key and in no others."""
     from montlok import _C
 
     q = torch.ones(1, 200, 2, 64, device=dev)
@@ -54,6 +55,9 @@ def test_split_attention_special_values(dev):
     assert torch.isnan(out[:, 150:, 1]).all()
     keep = [j for j in range(200) if j != 70]
     assert torch.allclose(out[0, 199, 0], v[0, keep, 0].mean(0), atol=1e-6)
+    k[0, 90, 0, 5] = float("inf")
+    out = _C.attention(q, k, v, _C.MASK_CAUSAL_TOP_LEFT, 0.125)
+    assert torch.isfinite(out[:, :90, 0]).all() and torch.isnan(out[:, 90:, 0]).all()
 
 
 @pytest.mark.parametrize("B,L,bias", [(4, 257, True), (5, 480, False), (8, 512, True), (4, 320, True)])

@@ -31,11 +31,11 @@ def _assert_bound(got, x, w, terms, extra=0.0):
 # first shapes past the one-wave rule's 1536 tiles, K just above 128, one row against many columns; then calls that
 # fill rounds of 128 x 128 blocks, with ragged last rows and columns, K not a multiple of the step, one and two steps;
 # then 256 blocks of 64 x 64, the last of two waves a tile, and one row more; K = 128 on both
-# sides of its 3072 blocks.
+# sides of its 3072 blocks; K from 64 to 127 that is no multiple of 8, which has no one-wave form, on few rows.
 SPLIT = [(1921, 256, 352, 0), (2049, 136, 200, 4), (1600, 132, 257, 0), (30000, 256, 1, 8), (64, 2048, 5200, 0),
          (1, 256, 24592, 0), (12304, 160, 30, 0), (1537, 256, 256, 12),
          (15360, 512, 256, 0), (16371, 260, 255, 4), (3840, 136, 1024, 0), (32700, 132, 256, 0), (65536, 544, 120, 0),
-         (4096, 148, 256, 0), (4097, 148, 256, 0), (6001, 128, 667, 4), (65537, 128, 130, 0)]
+         (4096, 148, 256, 0), (4097, 148, 256, 0), (6001, 128, 667, 4), (65537, 128, 130, 0), (1, 68, 30, 0), (16, 100, 257, 0), (130, 124, 64, 8)]
 
 
 @pytest.mark.parametrize("M,K,N,pad", SPLIT)
@@ -63,9 +63,11 @@ def test_four_waves_per_tile_vs_float64(dev, M, K, N, wdt):
 
 @pytest.mark.parametrize("M,K,N,groups", [(1921, 256, 352, 32), (1921, 256, 352, 16), (2500, 256, 300, 8),
                                           (3001, 256, 270, 4), (2100, 160, 260, 20), (1930, 192, 350, 3), (3300, 256, 300, 16),
-                                          (7000, 128, 300, 16), (33000, 128, 24, 8), (65536, 128, 200, 4)])
+                                          (7000, 128, 300, 16), (33000, 128, 24, 8), (65536, 128, 200, 4),
+                                          (16384, 128, 256, 16), (16371, 128, 255, 8)])
 def test_rms_norm_split_linear_equals_the_two_operators(dev, M, K, N, groups):
-    """Still one launch where the one-wave form used to serve these shapes, and the two operators bit for bit."""
+    """One launch, and the two operators bit for bit, also where linear takes 128 x 128 blocks (the last two shapes) and
+    the norm's form 64 x 64 ones."""
     from montlok import _C
     from montlok._C import _load
 
@@ -80,7 +82,7 @@ def test_rms_norm_split_linear_equals_the_two_operators(dev, M, K, N, groups):
 
 
 def test_split_linear_special_values(dev):
-    """Infinities, NaN, values whose bf16 rounding is infinite, subnormals: as the fp32 sum has them."""
+    """Infinities, NaN, values whose bf16 rounding is infinite: as the fp32 sum has them; subnormals to its bound."""
     from montlok import _C
 
     x, w, _, _ = _operands(dev, 2000, 256, 300, 7)
