@@ -1616,6 +1616,13 @@ extern "C" mlk_status mlk_rms_norm_linear(const float* x, int64_t rows, int64_t 
     MLK_CHECK(x && norm_weight && weight && out, "null tensor pointer");
     LinearArgs p{x, rows, in_features, x_stride, weight, bias, out_features, out, out_stride, nullptr, 0,
                  norm_weight, static_cast<double>(static_cast<float>(eps))};
+    // linear's bits: its form is that of the norm's dense rows, which x's stride must allow too.
+    LinearArgs dense = p;
+    dense.x_stride = in_features;
+    if (weight_dtype == MLK_DTYPE_F32 && split_shape(dense) && !split_shape(p)) {
+        set_error("rms_norm_linear: rows too far apart for the fused form (use rms_norm then linear)");
+        return MLK_ERR_UNSUPPORTED;
+    }
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     if (rows_form && !split_shape(p)) {
         MLK_CHECK(ceil_div(rows, kRowsPerBlock) <= 0x7fffffff, "too many rows");

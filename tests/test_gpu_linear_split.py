@@ -207,3 +207,15 @@ def test_rows_too_far_apart_for_the_planes(dev, K):
     y = _C.linear(far, w)
     _assert_bound(y, x, w, 2)
     assert torch.equal(_C.linear(far, w, b), y + b) and torch.equal(_C.linear_residual(far, w, b, r), r + (y + b))
+
+
+@pytest.mark.parametrize("M,K,N", [(100, 256, 4000), (3, 64, 40)])
+def test_norm_linear_of_rows_far_apart_equals_the_two_operators(dev, M, K, N):
+    """The norm leaves dense rows, so linear's form may differ from the one that x's stride would ask for."""
+    from montlok import _C
+
+    x, w, b, _ = _operands(dev, M, K, N, K)
+    nw = torch.rand(K, generator=torch.Generator().manual_seed(1)).to(dev) + 0.5
+    far = torch.empty(M * 2 ** 23, device=dev).view(M, 2 ** 23)[:, :K]
+    far.copy_(x)
+    assert torch.equal(_C.rms_norm_linear(far, nw, 1e-5, 4, w, b), _C.linear(_C.rms_norm(far, nw, 1e-5, 4), w, b))
