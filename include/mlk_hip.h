@@ -137,9 +137,10 @@ mlk_status mlk_linear_residual(const float* x, int64_t rows, int64_t in_features
  * or 64 floats and 16-byte aligned x rows, norm weight and weight rows, on
  * the shapes that take the one-wave-per-tile linear (fewer 128-row blocks x
  * 64-column chunks than CUs, in_features <= 256 and a multiple of 8) and, for
- * fp32 weights with in_features 128, on any row count (the row-layout linear
- * with the norm applied to its loaded fragments); other shapes return
- * MLK_ERR_UNSUPPORTED and the caller runs the two operators.
+ * fp32 weights with in_features 128, on any row count (each in mlk_linear's
+ * form for the shape); other shapes, and x rows too far apart for that form
+ * (2^23 floats), return MLK_ERR_UNSUPPORTED and the caller runs the two
+ * operators.
  * No single counterpart in the reference's op table: it fuses rms_norm
  * (montlok.cpp:1481) with the in_proj linear that follows it (stage1_forward,
  * montlok.cpp:1030-1034). */
@@ -153,9 +154,10 @@ mlk_status mlk_rms_norm_linear(const float* x, int64_t rows, int64_t in_features
  * bias [2 * hidden] or NULL, in one launch without the [rows, 2 * hidden]
  * intermediate; the linear's values as mlk_linear forms them, silu(g) * u in
  * double, rounded once. Built for fp32 weights where mlk_linear to 2 * hidden
- * columns takes its three-plane form (K above 128, 16-byte aligned rows of x
- * and W, more than a few hundred rows); MLK_ERR_UNSUPPORTED otherwise, and the
- * caller runs the two operators. */
+ * columns takes its three-plane form (in_features from 64 on and a multiple of
+ * 4, 16-byte aligned rows of x and W, and more 16 x 16 tiles than the
+ * one-wave-per-tile forms take); MLK_ERR_UNSUPPORTED otherwise, and the caller
+ * runs the two operators. */
 mlk_status mlk_linear_swiglu(const float* x, int64_t rows, int64_t in_features, int64_t x_stride, const void* weight,
                              int32_t weight_dtype, const float* bias, int64_t hidden, float* out, int64_t out_stride,
                              mlk_stream_t stream);

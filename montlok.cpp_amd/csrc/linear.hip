@@ -29,10 +29,11 @@
 // Shapes with fewer 128-row blocks x 64-column chunks than CUs (a few
 // thousand rows) take linear_small_kernel instead: one wave per 16 x 16
 // output tile, operands straight from L2, no LDS; with few tiles and K beyond
-// 256, linear_small_split_kernel, four waves per tile. fp32 weights with K
-// above 128 (large calls: 64 and more, but 128) otherwise take linear_split.hip's
-// three-plane bf16 form; the fp32 forms here then serve smaller K, K = 128 and
-// operands that are not 16-byte aligned.
+// 256, linear_small_split_kernel, four waves per tile. fp32 weights with K from
+// 64 on otherwise take linear_split.hip's three-plane bf16 form (split_shape
+// below says where); the fp32 forms here then serve K below 64, the largest
+// calls with K = 128, rows that are not 16-byte aligned and row strides past
+// that form's 32-bit offsets.
 //
 // K is reduced in an order of its own (the 8 k of a lane, then the four lane
 // groups inside the MFMA); for fp32 weights the result differs from a
@@ -345,7 +346,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(BUF ? 
 // the accumulator of lane (g, l) holds row l, columns 4g .. 4g + 3 of a tile
 // and leaves as one 16-byte store (scalar stores at a ragged N edge or an
 // unaligned output).
-// BUF > 0 (VEC, K a multiple of the 16-byte unit, N % 4 = 0, 16-byte aligned output and residual within
+// BUF > 0 (VEC, N % 4 = 0, 16-byte aligned output and residual within
 // 2 GiB): W fetched without per-unit branches (also past the last chunk, clamped) and the results stored
 // through a buffer resource (a store past its range dropped), so no memory operation sits behind a branch
 // and no wait covers the stores or the next W chunk. BUF = 1: no residual; BUF = 2: the residual fetched
@@ -1367,9 +1368,10 @@ int64_t tiles16(int64_t rows, int64_t N) { return ceil_div(rows, 16) * ceil_div(
 
 // fp32 weights with K above 128 go to the three-plane form (linear_split.hip) unless so few 16 x 16 tiles are
 // asked for that one wave per tile ends sooner: its blocks walk K alone, 8 us at K = 256 however few they are,
-// and the one-wave form takes 4.0 us for 300 tiles, 7.6 for 1320 and 9.4 for 1920 (12.1 for 2640). So do large calls
-// with K from 64 to 127 (7680 x 64 -> 384: 8.0 us against the row-layout form's 11.8; 65536 x 64 -> 384 35 against
-// 47). At K = 128, where rms_norm_linear (which gives linear's bits) has a row-layout form, up to 3072 of the 64 x 64
+// and the one-wave form takes 4.0 us for 300 tiles, 7.6 for 1320 and 9.4 for 1920 (12.1 for 2640). So do calls with K
+// from 64 to 127 that the one-wave form does not take: large ones (7680 x 64 -> 384: 8.0 us against the row-layout
+// form's 11.8; 65536 x 64 -> 384 35 against 47), and all whose K is no multiple of 8 (K = 68 and 100, 1 to 30000 rows,
+// N 16 to 1192: even or up to 1.9 times as fast, 1 x 68 -> 304 8.6 -> 7.5 us, 1000 x 100 -> 304 11.1 -> 6.6). At K = 128, where rms_norm_linear (which gives linear's bits) has a row-layout form, up to 3072 of the 64 x 64
 // blocks: 16384 x 128 -> 668 39 -> 27 us, with the norm 41.6 -> 39.8; 6000 rows 23.8 -> 14.2 and 32.6 -> 19.1. Past
 // that every column block's copy of the norm's sums costs more than the products save (65536 rows: 115 -> 133).
 bool split_shape(const LinearArgs& p) {

@@ -1708,7 +1708,7 @@ struct MlaSpanPack {
 // Blocks of one window run on one XCD (its L2 serves the later spans' reads
 // of the window's x). Each block forms the latents and keys of the tiles it
 // walks again: at 480 rows 4.5 tiles a block on average, still half the time of
-// the separate operators (64 windows x 480: 172 -> 102 us; 16 x 480: 86 -> 53).
+// the separate operators (64 windows x 480: 172 -> 96 us; 16 x 480: 86 -> 51).
 // PACKED: the three weights in MlaSpanPack's order, each
 // wave's fragment load one contiguous 1 KB.
 template <bool PACKED>

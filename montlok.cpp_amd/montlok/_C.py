@@ -220,7 +220,7 @@ def linear_residual(input: torch.Tensor, weight: torch.Tensor, bias: torch.Tenso
 def rms_norm_linear(x: torch.Tensor, norm_weight: torch.Tensor, eps: float, groups: int, weight: torch.Tensor,
                     bias: torch.Tensor | None = None) -> torch.Tensor:
     """linear(rms_norm(x, norm_weight, eps, groups), weight, bias), one launch where the fused form is
-    built (small row counts), else the two operators; the results are identical either way."""
+    built (few rows, or K = 128 with fp32 weights), else the two operators; the results are identical either way."""
     out = (_native or _ops()).rms_norm_linear(x, norm_weight, eps, groups, weight, bias)
     if out is None:  # no fused form for this shape
         return linear(rms_norm(x, norm_weight, eps, groups), weight, bias)
@@ -229,7 +229,7 @@ def rms_norm_linear(x: torch.Tensor, norm_weight: torch.Tensor, eps: float, grou
 
 def swiglu_mlp(input, in_weight, in_bias=None, out_weight=None, out_bias=None):
     """montlok.cpp:967-976: linear -> swiglu -> linear, the first two in one launch where that is built (fp32
-    weights, more than a few hundred rows)."""
+    weights with K from 64 on, more than a few hundred rows)."""
     hidden = (_native or _ops()).linear_swiglu(input, in_weight, in_bias)
     if hidden is None:
         hidden = swiglu(linear(input, in_weight, in_bias))
@@ -788,8 +788,9 @@ def _mla_forward(x, in_proj_weight, q_weight, kv_norm_weight, kv_norm_bias, kv_n
     _check(n_last == 1 or n_last == length, "native MLA supports the final query or the full sequence")
     precision = torch.bfloat16 if _weight(in_proj_weight, "in_proj_weight").dtype == torch.bfloat16 else torch.float32
     full = n_last == length
-    # Beyond 256 rows a block of the one-launch kernel walks up to eight key tiles: 50 us however few windows there
-    # are, against 42 us for one and 56 for four windows of 480 in separate operators.
+    # Beyond 256 rows a block of the one-launch kernel walks up to eight key tiles: 35 us at 257 rows and 53 at 512
+    # however few windows there are, against 33 and 48 us for one window, 39 and 59 for three, 41 and 65 for four in
+    # separate operators (ten lengths from 257 to 512, from four windows on 1.17 to 2.1 times as fast at each).
     if allow_fused and allow_window and full and causal and precision == torch.bfloat16 and \
             (length <= 256 or batch >= 4):
         out = _mla_window(x, in_proj_weight, kv_norm_weight, kv_norm_bias, kv_norm_eps, kv_up_weight, out_weight,

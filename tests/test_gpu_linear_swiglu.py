@@ -28,15 +28,19 @@ def test_linear_swiglu_vs_float64(dev, M, K, hidden, bias):
     assert bool(((out.double() - ref).abs() <= 2.0 ** -24 * (1 + 1e-6) * ref.abs() + 1e-45).all())
 
 
-def test_linear_swiglu_infinities(dev):
+@pytest.mark.parametrize("M,hidden", [(2000, 700), (600, 350), (7680, 512)])
+def test_linear_swiglu_infinities(dev, M, hidden):
+    """In 64 x 64 blocks, with two waves a tile, and in 128 x 128 blocks."""
     from montlok import _C
 
-    x = torch.randn(2000, 256, generator=torch.Generator().manual_seed(3)).to(dev)
-    w = torch.randn(700, 256, generator=torch.Generator().manual_seed(4)).to(dev)
-    x[70, 3], x[900, 7] = float("inf"), float("nan")
+    x = torch.randn(M, 256, generator=torch.Generator().manual_seed(3)).to(dev)
+    w = torch.randn(2 * hidden, 256, generator=torch.Generator().manual_seed(4)).to(dev)
+    x[70, 3], x[M // 2 - 100, 7], x[M - 1] = float("inf"), float("nan"), 1e-37
+    w[hidden + 3] *= 2.0 ** 30
     out = _C._ops().linear_swiglu(x, w, None)
     expect = _C.swiglu(_C.linear(x, w))
     assert torch.equal(torch.isnan(out), torch.isnan(expect)) and torch.equal(torch.isinf(out), torch.isinf(expect))
+    assert torch.equal(out[~torch.isnan(out)], expect[~torch.isnan(expect)])
 
 
 def test_other_shapes_run_the_two_operators(dev):
