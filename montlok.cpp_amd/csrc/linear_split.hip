@@ -423,9 +423,9 @@ void launch_blocks(const LinearArgs& p, hipStream_t stream) {
 
 // Whether rounds of 256 blocks of 128 x 128 (one a CU) are filled to nine tenths by the call's rows and columns.
 // Then the big blocks, which split every operand half as often and multiply while they split, are the faster ones
-// (15360 x 512 -> 256, 240 blocks: 25.6 us against 30.6; 65536 x 512 -> 256: 95 against 113; 7680 x 256 -> 1024, 480
-// blocks: 28 against 31); otherwise their last round, or the columns past N, cost more than that (7680 x 256 ->
-// 1192, 600 blocks: 41 against 35; 7680 x 512 -> 256, 120 blocks: 20 against 18).
+// (15360 x 512 -> 256, 240 blocks: 28 us against 33; 65536 x 512 -> 256: 102 against 114; 7680 x 256 -> 1024, 480
+// blocks: 30 against 32); otherwise their last round, or the columns past N, cost more than that (7680 x 256 ->
+// 1192, 600 blocks: 41 against 36; 7680 x 512 -> 256, 120 blocks: 21 against 18).
 bool fills_big_blocks(int64_t rows, int64_t w_rows) {
     const int64_t blocks = ceil_div(rows, 2 * kBlock) * ceil_div(w_rows, 2 * kBlock);
     const double held = static_cast<double>(ceil_div(blocks, 256) * 256) * (4 * kBlock * kBlock);
